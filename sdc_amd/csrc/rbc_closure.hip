@@ -36,7 +36,8 @@ constexpr int OFF_B2 = OFF_W2 + NH * NH;    // [NH]
 constexpr int OFF_W3 = OFF_B2 + NH;         // [NOUT][NH]
 constexpr int OFF_B3 = OFF_W3 + NOUT * NH;  // [NOUT]
 constexpr int NW = OFF_B3 + NOUT;           // 4931 parameters
-constexpr int kTrainWaves = 512;
+constexpr int kTrainBlocks = 256;  // partial gradients of a batch, at most
+constexpr int kTrainWaves = 8;     // waves per block
 
 struct Norm {
     float in_mean[NIN], in_inv[NIN];  // x_n = (x - mean) * inv
@@ -557,132 +558,336 @@ int infer_blocks(int npts) {
     return std::max(1, std::min(2048, (groups + 3) / 4));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
+// Training: gradient of the mean squared error (normalised targets, mean over points and outputs)
+// over `batch` points, on the matrix cores.  A wave takes 32 points at a time (columns of the
+// 32x32 tiles) and runs the three 64 x 64 products of the two hidden layers with
+// v_mfma_f32_32x32x2_f32: H2 = W2 H1, D1 = W2^T D2, G2 += D2 H1^T -- FP32 operands and sums, as a
+// scalar loop would have.  In the accumulator layout a lane holds one point and 32 hidden units
+// (rows 8 (r / 4) + 4 h + r % 4 of tile t, h = lane / 32); used in register order as a B operand that
+// is the K order the W2 fragments are stored in (w2f, w2t), so activations go from layer to layer
+// without leaving the registers.  The sums over points (G2, and G1, G3, the biases on the VALU)
+// need units across lanes: each factor is transposed once through the wave's LDS tile.
+//
+// Bound: 200 MFMAs of 64 cycles per 32 points, 12 us for 65,536 points on 1,024 SIMDs at two waves
+// each (LDS: 33 KiB of weight fragments and 9 KiB per wave).  One block of 8 waves per CU: the
+// gradients of its waves are added in LDS in a fixed order, so 256 partials leave the chip
+// instead of one per wave.  Groups go to blocks first, then to waves, so that small batches still
+// spread over the CUs.  65,536 points: 35 us (a scalar form, one point per wave at a time and 512
+// one-wave blocks, took 307 us).
+constexpr int kTP = 36;                      // row stride of the transposing tile (32 points + pad)
+constexpr int kTrainThreads = 64 * kTrainWaves;
+constexpr int NGV = 64 + 2 * NIN + 4 + 2 * NOUT + NOUT;  // gradient values per lane in the block's reduction
+// fragments (2 x 16 KiB) and the waves' tiles; the reduction reuses the same memory
+constexpr size_t kTrainLds =
+    std::max<size_t>((size_t)2 * NH * NH + (size_t)kTrainWaves * NH * kTP, (size_t)(kTrainWaves / 2) * NGV * 64) *
+    sizeof(float);
 
-// Training: gradient of the mean squared error (normalised targets, mean over points and
-// outputs) over `batch` points.  One wave per block; lane j is hidden unit j of both layers.
-// Wave w takes batch points [w per, (w+1) per); the point index is drawn uniformly from the
-// dataset (random != 0) or is the batch position itself.  Partial gradients per wave go to
-// gpart[w][NW], partial losses to lpart[w].
-__global__ void __launch_bounds__(64) k_mlp_train(int count, int batch, int per, int random, uint64_t seed,
-                                                  uint64_t step, const uint16_t* __restrict__ wbf, Norm nm,
-                                                  const float* __restrict__ X, const float* __restrict__ Y,
-                                                  float* __restrict__ gpart, double* __restrict__ lpart) {
-    __shared__ float sW2[NH * NH];
-    __shared__ float sh1[NH], sd2[NH];
-    const int j = threadIdx.x, wv = blockIdx.x;
-    for (int i = j; i < NH * NH; i += 64) sW2[i] = bf16_bits_to_f32(wbf[OFF_W2 + i]);
-    float w1[NIN], w2[NH], w3[NOUT], b3[NOUT];
-#pragma unroll
-    for (int i = 0; i < NIN; ++i) w1[i] = bf16_bits_to_f32(wbf[OFF_W1 + j * NIN + i]);
-    const float b1 = bf16_bits_to_f32(wbf[OFF_B1 + j]), b2 = bf16_bits_to_f32(wbf[OFF_B2 + j]);
-#pragma unroll
-    for (int o = 0; o < NOUT; ++o) {
-        w3[o] = bf16_bits_to_f32(wbf[OFF_W3 + o * NH + j]);
-        b3[o] = bf16_bits_to_f32(wbf[OFF_B3 + o]);
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__global__ void __launch_bounds__(kTrainThreads) k_mlp_train(int count, int batch, int random, uint64_t seed,
+                                                             uint64_t step, const uint16_t* __restrict__ wbf, Norm nm,
+                                                             const float* __restrict__ X, const float* __restrict__ Y,
+                                                             float* __restrict__ gpart, double* __restrict__ lpart) {
+    extern __shared__ float smem[];
+    __shared__ float b1s[NH], b2s[NH], w3s[NOUT * NH], b3s[NOUT];
+    __shared__ float w1s[NH * NIN];
+    __shared__ float xs[kTrainWaves][32][NIN + 4];  // a group's inputs and dy[0..2]
+    __shared__ double lsum[kTrainWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 31, h = lane >> 5;
+    float* w2f = smem;                // [tile row][tile col][r / 4][lane][r % 4]: W2[32 t2 + c][unit(t, r, h)]
+    float* w2t = smem + NH * NH;      // same with W2 transposed
+    float* tile = smem + 2 * NH * NH + wave * NH * kTP;  // [unit][point]
+    for (int i = tid; i < NH * NH; i += kTrainThreads) {
+        const int r4 = i & 3, l = (i >> 2) & 63, rq = (i >> 8) & 3, t = (i >> 10) & 1, t2 = i >> 11;
+        const int row = 32 * t2 + (l & 31), unit = 32 * t + 8 * rq + 4 * (l >> 5) + r4;
+        w2f[i] = bf16_bits_to_f32(wbf[OFF_W2 + row * NH + unit]);
+        w2t[i] = bf16_bits_to_f32(wbf[OFF_W2 + unit * NH + row]);
     }
+    for (int i = tid; i < NH * NIN; i += kTrainThreads) w1s[i] = bf16_bits_to_f32(wbf[OFF_W1 + i]);
+    for (int i = tid; i < NOUT * NH; i += kTrainThreads) w3s[i] = bf16_bits_to_f32(wbf[OFF_W3 + i]);
+    if (tid < NH) {
+        b1s[tid] = bf16_bits_to_f32(wbf[OFF_B1 + tid]);
+        b2s[tid] = bf16_bits_to_f32(wbf[OFF_B2 + tid]);
+    }
+    if (tid < NOUT) b3s[tid] = bf16_bits_to_f32(wbf[OFF_B3 + tid]);
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NH; ++i) w2[i] = sW2[j * NH + i];
-    float g1[NIN] = {}, g2[NH] = {}, g3[NOUT] = {}, gb3[NOUT] = {};
-    float gb1 = 0.f, gb2 = 0.f;
-    double loss = 0.0;
     const float inv_outs = 1.0f / ((float)batch * NOUT);
-    const int b0 = wv * per, b1e = min(batch, b0 + per);
-    for (int bi = b0; bi < b1e; ++bi) {
-        size_t idx = (size_t)bi;
-        if (random) idx = (size_t)(mix64(seed * 0x100000001B3ull + step * 0x9E3779B1ull + (uint64_t)bi) % (uint64_t)count);
-        float x[NIN];
-#pragma unroll
-        for (int i = 0; i < NIN; ++i) x[i] = (X[idx * NIN + i] - nm.in_mean[i]) * nm.in_inv[i];
-        float a1 = b1;
-#pragma unroll
-        for (int i = 0; i < NIN; ++i) a1 += w1[i] * x[i];
-        const float h1 = tanh_fast(a1);
-        sh1[j] = h1;
+    const int ngroups = (batch + 31) / 32;
+    f32x16 g2[2][2] = {};
+    float g1[2][NIN] = {}, gb1[2] = {}, gb2[2] = {}, g3[2][NOUT] = {}, gb3[NOUT] = {};
+    double loss = 0.0;
+    // rows of the accumulator layout into the [unit][point] tile; points 16 h + 4 q .. + 3 of unit
+    // 32 t + c from it
+    auto put = [&](const f32x16 (&d)[2]) {
         wave_sync();
-        float a2 = b2;
 #pragma unroll
-        for (int i = 0; i < NH; ++i) a2 += w2[i] * sh1[i];
-        const float h2 = tanh_fast(a2);
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tile[(32 * t + 8 * (r >> 2) + 4 * h + (r & 3)) * kTP + c] = d[t][r];
+        wave_sync();
+    };
+    auto points = [&](int t, int q) { return *(const f32x4*)(tile + (32 * t + c) * kTP + 16 * h + 4 * q); };
+    for (int gi = wave * gridDim.x + blockIdx.x; gi < ngroups; gi += kTrainWaves * gridDim.x) {  // wave-uniform
+        const int bi = gi * 32 + c;
+        const bool valid = bi < batch;
+        size_t idx = valid ? (size_t)bi : 0;
+        if (random)
+            idx = (size_t)(mix64(seed * 0x100000001B3ull + step * 0x9E3779B1ull + (uint64_t)bi) % (uint64_t)count);
+        // every lane loads (row 0 or a drawn row where the batch has ended) and drops it if not valid
+        const f32x4 xr = *(const f32x4*)(X + idx * NIN + 4 * h);
+        float yr[NOUT];
+#pragma unroll
+        for (int o = 0; o < NOUT; ++o) yr[o] = Y[idx * NOUT + o];
+        float xv[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float z = (xr[e] - nm.in_mean[4 * h + e]) * nm.in_inv[4 * h + e];
+            xv[e] = valid ? z : 0.f;
+            xs[wave][c][4 * h + e] = xv[e];
+        }
+        f32x16 h1[2], h2[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            f32x16 a = {};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                a = __builtin_amdgcn_mfma_f32_32x32x2f32(w1s[(32 * t + c) * NIN + 4 * h + e], xv[e], a, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) h1[t][r] = tanh_fast(a[r] + b1s[32 * t + 8 * (r >> 2) + 4 * h + (r & 3)]);
+        }
+        // 64 x 64 times 64 x 32: fragments from LDS, four K steps a read
+        auto product = [&](const float* frag, const f32x16 (&b)[2], f32x16 (&out)[2]) {
+            out[0] = out[1] = f32x16{};
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f32x4 a0 = *(const f32x4*)(frag + ((t * 4 + q) * 64 + lane) * 4);
+                    const f32x4 a1 = *(const f32x4*)(frag + ((8 + t * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        out[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], b[t][4 * q + e], out[0], 0, 0, 0);
+                        out[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], b[t][4 * q + e], out[1], 0, 0, 0);
+                    }
+                }
+        };
+        asm volatile("" ::: "memory");  // the tables are read where they are used, not held in registers
+        product(w2f, h1, h2);
+        asm volatile("" ::: "memory");
+        float y[NOUT] = {};
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int unit = 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+                h2[t][r] = tanh_fast(h2[t][r] + b2s[unit]);
+#pragma unroll
+                for (int o = 0; o < NOUT; ++o) y[o] += w3s[o * NH + unit] * h2[t][r];
+            }
         float dy[NOUT];
-        float d2s = 0.f;
 #pragma unroll
         for (int o = 0; o < NOUT; ++o) {
-            const float y = wave_sum(w3[o] * h2) + b3[o];
-            const float t = Y[idx * NOUT + o] / nm.out_scale[o];
-            const float e = y - t;
-            loss += (double)e * e;
+            y[o] += __shfl_xor(y[o], 32);
+            const float err = y[o] + b3s[o] - yr[o] / nm.out_scale[o], e = valid ? err : 0.f;
             dy[o] = 2.f * e * inv_outs;
-            g3[o] += dy[o] * h2;
+            loss += (double)e * e;  // both lane halves: halved where it is written
             gb3[o] += dy[o];
-            d2s += w3[o] * dy[o];
+            xs[wave][c][NIN + o] = dy[o];
         }
-        const float d2 = d2s * (1.f - h2 * h2);
-        gb2 += d2;
+        asm volatile("" ::: "memory");
+        f32x16 d[2];
 #pragma unroll
-        for (int i = 0; i < NH; ++i) g2[i] += d2 * sh1[i];
-        sd2[j] = d2;
-        wave_sync();
-        float d1s = 0.f;
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int k = 0; k < NH; ++k) d1s += sW2[k * NH + j] * sd2[k];
-        const float d1 = d1s * (1.f - h1 * h1);
-        gb1 += d1;
+            for (int r = 0; r < 16; ++r) {
+                const int unit = 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+                float s = 0.f;
 #pragma unroll
-        for (int i = 0; i < NIN; ++i) g1[i] += d1 * x[i];
-        wave_sync();  // sh1 / sd2 are rewritten by the next point
+                for (int o = 0; o < NOUT; ++o) s += w3s[o * NH + unit] * dy[o];
+                d[t][r] = s * (1.f - h2[t][r] * h2[t][r]);
+            }
+        put(h2);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 u0 = points(0, q), u1 = points(1, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int o = 0; o < NOUT; ++o) {
+                    const float v = xs[wave][16 * h + 4 * q + e][NIN + o];
+                    g3[0][o] += v * u0[e];
+                    g3[1][o] += v * u1[e];
+                }
+        }
+        put(d);
+        f32x4 dt[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) dt[t][q] = points(t, q);
+        put(h1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 u0 = points(0, q), u1 = points(1, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t2 = 0; t2 < 2; ++t2) {
+                    g2[t2][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(dt[t2][q][e], u0[e], g2[t2][0], 0, 0, 0);
+                    g2[t2][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(dt[t2][q][e], u1[e], g2[t2][1], 0, 0, 0);
+                    gb2[t2] += dt[t2][q][e];
+                }
+        }
+        asm volatile("" ::: "memory");
+        product(w2t, d, h2);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) d[t][r] = h2[t][r] * (1.f - h1[t][r] * h1[t][r]);
+        put(d);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 u0 = points(0, q), u1 = points(1, q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                gb1[0] += u0[e];
+                gb1[1] += u1[e];
+#pragma unroll
+                for (int i = 0; i < NIN; ++i) {
+                    const float v = xs[wave][16 * h + 4 * q + e][i];
+                    g1[0][i] += v * u0[e];
+                    g1[1][i] += v * u1[e];
+                }
+            }
+        }
+        wave_sync();  // xs is rewritten by the next group
     }
-    float* gp = gpart + (size_t)wv * NW;
+    // the waves' gradients, added pairwise in a fixed order (upper half to lower half)
+    float v[NGV];
+    {
+        int n = 0;
 #pragma unroll
-    for (int i = 0; i < NIN; ++i) gp[OFF_W1 + j * NIN + i] = g1[i];
-    gp[OFF_B1 + j] = gb1;
+        for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
-    for (int i = 0; i < NH; ++i) gp[OFF_W2 + j * NH + i] = g2[i];
-    gp[OFF_B2 + j] = gb2;
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int o = 0; o < NOUT; ++o) gp[OFF_W3 + o * NH + j] = g3[o];
-    if (j == 0) {
+                for (int r = 0; r < 16; ++r) v[n++] = g2[t2][t][r];
 #pragma unroll
-        for (int o = 0; o < NOUT; ++o) gp[OFF_B3 + o] = gb3[o];
-        lpart[wv] = loss / ((double)batch * NOUT);
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int i = 0; i < NIN; ++i) v[n++] = g1[t][i];
+            v[n++] = gb1[t];
+            v[n++] = gb2[t];
+#pragma unroll
+            for (int o = 0; o < NOUT; ++o) v[n++] = g3[t][o];
+        }
+#pragma unroll
+        for (int o = 0; o < NOUT; ++o) v[n++] = gb3[o];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+    if (lane == 0) lsum[wave] = loss;
+#pragma unroll
+    for (int half = kTrainWaves / 2; half > 0; half >>= 1) {
+        __syncthreads();
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int n = 0; n < NGV; ++n) smem[((wave - half) * NGV + n) * 64 + lane] = v[n];
+        }
+        __syncthreads();
+        if (wave < half) {
+#pragma unroll
+            for (int n = 0; n < NGV; ++n) v[n] += smem[(wave * NGV + n) * 64 + lane];
+        }
+    }
+    if (wave != 0) return;
+    float* gp = gpart + (size_t)blockIdx.x * NW;
+    int n = 0;
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                gp[OFF_W2 + (32 * t2 + 8 * (r >> 2) + 4 * h + (r & 3)) * NH + 32 * t + c] = v[n++];
+    // per-unit values: the two lane halves hold sums over different points
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int i = 0; i < NIN + 2 + NOUT; ++i, ++n) {
+            const float s = v[n] + __shfl_xor(v[n], 32);
+            const int unit = 32 * t + c;
+            const int at = i < NIN ? OFF_W1 + unit * NIN + i
+                                   : (i == NIN ? OFF_B1 + unit
+                                               : (i == NIN + 1 ? OFF_B2 + unit : OFF_W3 + (i - NIN - 2) * NH + unit));
+            if (h == 0) gp[at] = s;
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < NOUT; ++o, ++n) {
+        float s = v[n];
+        for (int k = 16; k > 0; k >>= 1) s += __shfl_xor(s, k);
+        if (lane == 0) gp[OFF_B3 + o] = s;
+    }
+    if (lane == 0) {
+        double s = 0.0;
+        for (int w = 0; w < kTrainWaves; ++w) s += lsum[w];
+        lpart[blockIdx.x] = 0.5 * s / ((double)batch * NOUT);
     }
 }
 
-// sum of the per-wave partials (fixed order) and the batch loss into lossbuf[slot]
-__global__ void k_grad_reduce(int nw, const float* __restrict__ gpart, const double* __restrict__ lpart,
-                              float* __restrict__ grad, double* __restrict__ lossbuf, int slot) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// The batch gradient: FP64 sum of the blocks' partials in a fixed order (32 parameters a block, 8
+// threads each take every 8th partial), the batch loss into lossbuf[slot], and, with ADAM, the Adam
+// update (Kingma & Ba 2015) of the FP32 master weights and their BF16 copies in the same launch.
+// Bound: 5 MB of partials; 155 blocks with 8 partial rows in flight each (5.5 us; one thread per
+// parameter over 512 partials, 20 blocks, took 137 us and Adam a launch of 5 us more).
+struct AdamStep {
+    float lr, beta1, beta2, eps, c1, c2;
+};
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_grad_finish(int nblk, const float* __restrict__ gpart,
+                                                     const double* __restrict__ lpart, float* __restrict__ grad,
+                                                     double* __restrict__ lossbuf, int slot, AdamStep ad,
+                                                     float* __restrict__ wm, float* __restrict__ m1,
+                                                     float* __restrict__ m2, uint16_t* __restrict__ wbf) {
+    __shared__ double part[8][32];
+    const int c = threadIdx.x & 31, row = threadIdx.x >> 5, i = blockIdx.x * 32 + c;
+    double s = 0.0;
     if (i < NW) {
-        double s = 0.0;
-        for (int w = 0; w < nw; ++w) s += gpart[(size_t)w * NW + i];
-        grad[i] = (float)s;
+#pragma unroll 8
+        for (int b = row; b < nblk; b += 8) s += gpart[(size_t)b * NW + i];
     }
-    if (i == 0) {
-        double s = 0.0;
-        for (int w = 0; w < nw; ++w) s += lpart[w];
-        lossbuf[slot] = s;
+    part[row][c] = s;
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x >= 192) {  // the last wave: the loss
+        double l = 0.0;
+        for (int b = threadIdx.x - 192; b < nblk; b += 64) l += lpart[b];
+        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+        if (threadIdx.x == 192) lossbuf[slot] = l;
+    }
+    if (row != 0 || i >= NW) return;
+    for (int r = 1; r < 8; ++r) s += part[r][c];
+    const float gr = (float)s;
+    grad[i] = gr;
+    if (ADAM) {
+        const float a = ad.beta1 * m1[i] + (1.f - ad.beta1) * gr;
+        const float b = ad.beta2 * m2[i] + (1.f - ad.beta2) * gr * gr;
+        m1[i] = a;
+        m2[i] = b;
+        const float w = wm[i] - ad.lr * (a / ad.c1) / (sqrtf(b / ad.c2) + ad.eps);
+        wm[i] = w;
+        wbf[i] = f32_to_bf16_bits(w);
     }
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master weights; writes the BF16 copies
-__global__ void k_adam(const float* __restrict__ grad, float* __restrict__ wm, float* __restrict__ m1,
-                       float* __restrict__ m2, uint16_t* __restrict__ wbf, float lr, float beta1, float beta2,
-                       float eps, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= NW) return;
-    const float gr = grad[i];
-    const float a = beta1 * m1[i] + (1.f - beta1) * gr;
-    const float b = beta2 * m2[i] + (1.f - beta2) * gr * gr;
-    m1[i] = a;
-    m2[i] = b;
-    const float w = wm[i] - lr * (a / c1) / (sqrtf(b / c2) + eps);
-    wm[i] = w;
-    wbf[i] = f32_to_bf16_bits(w);
+// gradient partials of `batch` points of (X, Y); returns the number of partials
+int launch_train(hipStream_t s, int count, int batch, int random, uint64_t seed, uint64_t step, const uint16_t* wbf,
+                 const Norm& nm, const float* X, const float* Y, float* gpart, double* lpart) {
+    const int nblk = std::min(kTrainBlocks, (batch + 31) / 32);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(kTrainThreads), kTrainLds, s, count, batch, random, seed, step,
+                       wbf, nm, X, Y, gpart, lpart);
+    return nblk;
 }
 
 // per-column sums and sums of squares (FP64) of a row-major [n][nc] array, per block
@@ -754,8 +959,8 @@ struct rbc_closure {
     float* grad = nullptr;
     float* m1 = nullptr;
     float* m2 = nullptr;
-    float* gpart = nullptr;           // [kTrainWaves][NW]
-    double* lpart = nullptr;          // [kTrainWaves]
+    float* gpart = nullptr;           // [kTrainBlocks][NW]
+    double* lpart = nullptr;          // [kTrainBlocks]
     double* lossbuf = nullptr;        // [lossbuf_n]
     int lossbuf_n = 0;
     int adam_t = 0;
@@ -1107,8 +1312,8 @@ int rbc_closure_create(rbc_ctx* c, int nz, int capacity_points, rbc_closure** ou
         cl->grad = (float*)cl->al(NW * sizeof(float));
         cl->m1 = (float*)cl->al(NW * sizeof(float));
         cl->m2 = (float*)cl->al(NW * sizeof(float));
-        cl->gpart = (float*)cl->al((size_t)kTrainWaves * NW * sizeof(float));
-        cl->lpart = (double*)cl->al(kTrainWaves * sizeof(double));
+        cl->gpart = (float*)cl->al((size_t)kTrainBlocks * NW * sizeof(float));
+        cl->lpart = (double*)cl->al(kTrainBlocks * sizeof(double));
         for (int i = 0; i < 11; ++i) cl->snap.push_back(cl->al(snap_bytes(c, i)));
         // Glorot-uniform initial weights from SplitMix64, zero biases
         std::vector<float> w0(NW, 0.f);
@@ -1338,12 +1543,10 @@ int rbc_closure_gradient(rbc_closure* cl, int n, const float* X, const float* Y,
         HIPCHK(hipMalloc(&lb, sizeof(double)));
         HIPCHK(hipMemcpy(dx, X, (size_t)n * NIN * sizeof(float), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(dy, Y, (size_t)n * NOUT * sizeof(float), hipMemcpyHostToDevice));
-        const int per = (n + kTrainWaves - 1) / kTrainWaves;
-        const int nwv = (n + per - 1) / per;
-        hipLaunchKernelGGL(k_mlp_train, dim3(nwv), dim3(64), 0, c->stream, n, n, per, 0, (uint64_t)0, (uint64_t)0,
-                           (const uint16_t*)cl->wbf, cl->nm, (const float*)dx, (const float*)dy, cl->gpart, cl->lpart);
-        hipLaunchKernelGGL(k_grad_reduce, dim3((NW + 255) / 256), dim3(256), 0, c->stream, nwv,
-                           (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, lb, 0);
+        const int nblk = launch_train(c->stream, n, n, 0, 0, 0, cl->wbf, cl->nm, dx, dy, cl->gpart, cl->lpart);
+        hipLaunchKernelGGL(k_grad_finish<false>, dim3((NW + 31) / 32), dim3(256), 0, c->stream, nblk,
+                           (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, lb, 0, AdamStep{}, nullptr,
+                           nullptr, nullptr, nullptr);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(grad, cl->grad, NW * sizeof(float), hipMemcpyDeviceToHost, c->stream));
         double l = 0;
@@ -1371,21 +1574,17 @@ int rbc_closure_train(rbc_closure* cl, int steps, int batch, double lr, unsigned
             cl->lossbuf = (double*)cl->al((size_t)std::max(1, steps) * sizeof(double));
             cl->lossbuf_n = steps;
         }
-        const int per = (batch + kTrainWaves - 1) / kTrainWaves;
-        const int nwv = (batch + per - 1) / per;
         const float* X = cl->DX + (size_t)first * NIN;
         const float* Y = cl->DY + (size_t)first * NOUT;
         for (int s = 0; s < steps; ++s) {
-            hipLaunchKernelGGL(k_mlp_train, dim3(nwv), dim3(64), 0, c->stream, n, batch, per, 1, (uint64_t)seed,
-                               (uint64_t)(cl->adam_t + 1), (const uint16_t*)cl->wbf, cl->nm, X, Y, cl->gpart,
-                               cl->lpart);
-            hipLaunchKernelGGL(k_grad_reduce, dim3((NW + 255) / 256), dim3(256), 0, c->stream, nwv,
-                               (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, cl->lossbuf, s);
+            const int nblk = launch_train(c->stream, n, batch, 1, seed, (uint64_t)(cl->adam_t + 1), cl->wbf, cl->nm, X,
+                                          Y, cl->gpart, cl->lpart);
             cl->adam_t++;
             const float b1 = 0.9f, b2 = 0.999f;
             const float c1 = 1.f - std::pow(b1, (float)cl->adam_t), c2 = 1.f - std::pow(b2, (float)cl->adam_t);
-            hipLaunchKernelGGL(k_adam, dim3((NW + 255) / 256), dim3(256), 0, c->stream, (const float*)cl->grad, cl->wm,
-                               cl->m1, cl->m2, cl->wbf, (float)lr, b1, b2, 1e-8f, c1, c2);
+            hipLaunchKernelGGL(k_grad_finish<true>, dim3((NW + 31) / 32), dim3(256), 0, c->stream, nblk,
+                               (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, cl->lossbuf, s,
+                               AdamStep{(float)lr, b1, b2, 1e-8f, c1, c2}, cl->wm, cl->m1, cl->m2, cl->wbf);
         }
         HIPCHK(hipGetLastError());
         if (loss && steps > 0)
