@@ -1021,7 +1021,7 @@ int y_tile(int N) {
 void synth_points(rbc_closure* cl, int F, int os, int zcol, float* out) {
     rbc_ctx* c = cl->c;
     const DevGeom& g = cl->gz;
-    if (!launch_y_inv_group(g, F, cl->spec, cl->twN, cl->hyb, c->stream)) {
+    if (!launch_y_inv_group<float>(g, F, cl->spec, cl->twN, cl->hyb, c->stream)) {
         const int TX = y_tile(g.N);
         hipLaunchKernelGGL(k_fft_y_inv<float>, dim3((g.KX + TX - 1) / TX, cl->nz, F), dim3(256),
                            (size_t)2 * TX * g.N * sizeof(cpx<float>), c->stream, g, TX, (const cpx<float>*)cl->spec,
@@ -1095,7 +1095,7 @@ void apply_closure(rbc_ctx* c, void* user) {
         hipLaunchKernelGGL(k_anal_rows, dim3(g.N, cl->nz), dim3(256), (size_t)2 * NOUT * g.M * sizeof(cpx<float>),
                            c->stream, g, (const float*)cl->pred, (const cpx<float>*)cl->twM, cl->hyb);
     }
-    if (!launch_y_fwd_group(g, 3, cl->hyb, cl->twN, cl->spec, c->stream)) {
+    if (!launch_y_fwd_group<float>(g, 3, cl->hyb, cl->twN, cl->spec, c->stream)) {
         const int TX = y_tile(g.N);
         hipLaunchKernelGGL(k_fft_y_fwd<float>, dim3((g.KX + TX - 1) / TX, cl->nz, 3), dim3(256),
                            (size_t)2 * TX * g.N * sizeof(cpx<float>), c->stream, g, TX, (const cpx<float>*)cl->hyb,

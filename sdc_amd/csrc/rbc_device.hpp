@@ -126,7 +126,7 @@ __device__ __forceinline__ void dft8(cpx<T> v[8]) {
     v[7] = c7;
 }
 
-// max over aligned groups of W lanes (W = 8, 16, 32 or 64), the result in every lane of the
+// max over aligned groups of W lanes (W = 2, 4, .., 64), the result in every lane of the
 // group: DPP lane permutations inside 16-lane rows (quad_perm [1,0,3,2], quad_perm [2,3,0,1],
 // row_half_mirror, row_mirror; after the earlier steps each is a max with the partner half),
 // then a shuffle across rows (W = 32) or lane reads of the four rows (W = 64).  All lanes active.
@@ -147,8 +147,8 @@ template <int W>
 __device__ __forceinline__ float group_max(float v) {
     unsigned x = __float_as_uint(v);
     x = dpp_max_step(x, 0);
-    x = dpp_max_step(x, 1);
-    x = dpp_max_step(x, 2);
+    if (W >= 4) x = dpp_max_step(x, 1);
+    if (W >= 8) x = dpp_max_step(x, 2);
     if (W >= 16) x = dpp_max_step(x, 3);
     if (W == 32) x = max(x, (unsigned)__shfl_xor((int)x, 16));
     if (W == 64) {
@@ -177,35 +177,68 @@ __device__ __forceinline__ float inv_pow2(float s) {
 }
 
 // radix-4 butterfly in place (natural order outputs): X_p = sum_q a_q (-+i)^{pq}
-template <bool INV>
-__device__ __forceinline__ void dft4(cpx<float>& a0, cpx<float>& a1, cpx<float>& a2, cpx<float>& a3) {
-    const cpx<float> t0 = a0 + a2, t1 = a0 - a2, t2 = a1 + a3, t3 = a1 - a3;
-    const cpx<float> it3 = INV ? mk(-t3.y, t3.x) : mk(t3.y, -t3.x);  // -+ i t3
+template <bool INV, typename T>
+__device__ __forceinline__ void dft4(cpx<T>& a0, cpx<T>& a1, cpx<T>& a2, cpx<T>& a3) {
+    const cpx<T> t0 = a0 + a2, t1 = a0 - a2, t2 = a1 + a3, t3 = a1 - a3;
+    const cpx<T> it3 = INV ? mk(-t3.y, t3.x) : mk(t3.y, -t3.x);  // -+ i t3
     a0 = t0 + t2;
     a1 = t1 + it3;
     a2 = t0 - t2;
     a3 = t1 - it3;
 }
 
-// n-point FFT (n = 2^LOGN, 64 <= n <= 1024) of NF sequences on a group of W = n / 8 lanes in
+// 16-point DFT in registers (natural order in and out): 4 x 4
+template <typename T, bool INV>
+__device__ __forceinline__ void dft16(cpx<T> v[16]) {
+    constexpr T c1 = T(0.92387953251128675613), s1 = T(0.38268343236508977173), h = T(0.70710678118654752440);
+#pragma unroll
+    for (int n2 = 0; n2 < 4; ++n2) dft4<INV>(v[n2], v[4 + n2], v[8 + n2], v[12 + n2]);
+    // v[4 k1 + n2] times w16^(n2 k1)
+    const T sg = INV ? T(1) : T(-1);
+    v[5] = cmul(v[5], mk(c1, sg * s1));
+    v[6] = cmul(v[6], mk(h, sg * h));
+    v[7] = cmul(v[7], mk(s1, sg * c1));
+    v[9] = cmul(v[9], mk(h, sg * h));
+    v[10] = INV ? mk(-v[10].y, v[10].x) : mk(v[10].y, -v[10].x);
+    v[11] = cmul(v[11], mk(-h, sg * h));
+    v[13] = cmul(v[13], mk(s1, sg * c1));
+    v[14] = cmul(v[14], mk(-h, sg * h));
+    v[15] = cmul(v[15], mk(-c1, -sg * s1));
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) dft4<INV>(v[4 * k1], v[4 * k1 + 1], v[4 * k1 + 2], v[4 * k1 + 3]);
+    // X[k1 + 4 k2] sits in v[4 k1 + k2]: transpose
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1)
+#pragma unroll
+        for (int k2 = k1 + 1; k2 < 4; ++k2) {
+            const cpx<T> t = v[4 * k1 + k2];
+            v[4 * k1 + k2] = v[4 * k2 + k1];
+            v[4 * k2 + k1] = t;
+        }
+}
+
+// Elements per lane of the group transforms: a group of W = n / E lanes stays inside one wavefront.
+constexpr int group_elems(int logn) { return logn <= 9 ? 8 : 16; }
+
+// n-point FFT (n = 2^LOGN, 16 <= n <= 1024) of NF sequences on a group of W = n / E lanes in
 // natural layout: element i of a sequence sits in register i / W of lane i % W of the group,
-// on entry and on exit.  Stockham passes: radix 8 while three or more radix-2 stages remain,
-// then one radix-2^(LOGN mod 3) pass.  Lane j runs the butterflies j + W b (b < 8 / R) of a
-// radix-R pass, whose inputs x[j + W b + q n / R] are registers b + q 8 / R on the first pass
-// and whose outputs y[j + W b + p n / R] are registers b + p 8 / R on the last; passes between
+// on entry and on exit.  Stockham passes: radix E, then radix 8 while three or more radix-2
+// stages remain, then one radix-2^(rest) pass.  Lane j runs the butterflies j + W b (b < E / R) of
+// a radix-R pass, whose inputs x[j + W b + q n / R] are registers b + q E / R on the first pass
+// and whose outputs y[j + W b + p n / R] are registers b + p E / R on the last; passes between
 // exchange through the group's LDS scratch (element i at sb[pad8(i) S], so a column of an LDS
 // tile of row stride S can serve).  The NF sequences go through the scratch one after the
 // other.  tw[t] = exp(-2 pi i t / n); the inverse uses conjugate twiddles; unnormalised.
-template <int LOGN, bool INV, int NF, int S = 1>
-__device__ __forceinline__ void fft_group(cpx<float> (&v)[NF][8], cpx<float>* sb, const cpx<float>* tw, int j) {
-    constexpr int n = 1 << LOGN, W = n / 8;
-    constexpr int NP8 = LOGN / 3, REM = LOGN % 3, NPASS = NP8 + (REM ? 1 : 0);
+template <int LOGN, bool INV, int NF, int S = 1, typename T = float, int E = 8>
+__device__ __forceinline__ void fft_group(cpx<T> (&v)[NF][E], cpx<T>* sb, const cpx<T>* tw, int j) {
+    constexpr int n = 1 << LOGN, W = n / E, LE = E == 16 ? 4 : 3;
+    constexpr int NP8 = (LOGN - LE) / 3, REM = (LOGN - LE) % 3, NPASS = 1 + NP8 + (REM ? 1 : 0);
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
         int logLs = 0;
 #pragma unroll
         for (int ps = 0; ps < NPASS; ++ps) {
-            const int LR = ps < NP8 ? 3 : REM, R = 1 << LR, NB = 8 / R, Ls = 1 << logLs;
+            const int LR = ps == 0 ? LE : (ps <= NP8 ? 3 : REM), R = 1 << LR, NB = E / R, Ls = 1 << logLs;
             if (ps > 0) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
@@ -219,18 +252,29 @@ __device__ __forceinline__ void fft_group(cpx<float> (&v)[NF][8], cpx<float>* sb
                 if (ps > 0)
 #pragma unroll
                     for (int q = 1; q < R; ++q) {
-                        cpx<float> w = tw[(q * k) << (LOGN - LR - logLs)];
+                        cpx<T> w = tw[(q * k) << (LOGN - LR - logLs)];
                         if (INV) w.y = -w.y;
                         v[f][b + q * NB] = cmul(v[f][b + q * NB], w);
                     }
-                if (R == 8) {
-                    dft8<float, INV>(v[f]);
+                if constexpr (E == 16) {
+                    if (R == 16) {
+                        dft16<T, INV>(v[f]);
+                    } else if (R == 8) {
+                        cpx<T> t[8];
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) t[q] = v[f][(b + q * NB) & (E - 1)];
+                        dft8<T, INV>(t);
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) v[f][(b + q * NB) & (E - 1)] = t[q];
+                    }
+                } else if (R == 8) {
+                    dft8<T, INV>(v[f]);
                 } else if (R == 4) {
-                    dft4<INV>(v[f][b], v[f][b + 2], v[f][b + 4], v[f][b + 6]);
+                    dft4<INV>(v[f][b & 7], v[f][(b + 2) & 7], v[f][(b + 4) & 7], v[f][(b + 6) & 7]);
                 } else {
-                    const cpx<float> a0 = v[f][b], a1 = v[f][b + 4];
-                    v[f][b] = a0 + a1;
-                    v[f][b + 4] = a0 - a1;
+                    const cpx<T> a0 = v[f][b & 7], a1 = v[f][(b + 4) & 7];
+                    v[f][b & 7] = a0 + a1;
+                    v[f][(b + 4) & 7] = a0 - a1;
                 }
             }
             if (ps + 1 < NPASS) {
@@ -381,50 +425,58 @@ __global__ void __launch_bounds__(256) k_fft_y_fwd(DevGeom g, int TX, const cpx<
     }
 }
 
-// y-FFTs at N = 64, 128, 256 (FP32): a block of WPB waves handles CB = WPB (64 / W) kx columns
-// of one (field, level), one group of W = N / 8 lanes per column (fft_group in natural layout);
+// y-FFTs at N = 16 .. 1024 on the group transforms: a block of WPB waves handles CB = WPB (64 / W)
+// kx columns of one (field, level), one group of W lanes per column (fft_group in natural layout);
 // the LDS tile [pad8(y)][CB + 1] is each column's FFT scratch and the transpose to the
-// row-major hybrid layout (rows of CB contiguous values).
-template <int LOGN, int WPB>
-__device__ __forceinline__ void k_fft_y_inv_w_body(int bz, DevGeom g, const cpx<float>* __restrict__ lev,
-                                                   const cpx<float>* __restrict__ twN, cpx<float>* __restrict__ hin) {
-    constexpr int N = 1 << LOGN, W = N / 8, G = 64 / W, CB = WPB * G, S = CB + 1;
-    __shared__ cpx<float> tw[N];
-    __shared__ cpx<float> tile[(N + N / 8) * S];
+// row-major hybrid layout (rows of CB contiguous values).  256^2 x 24 FP64: inverse 53 us, forward with
+// the level combinations 99 us (the LDS radix-4 kernels and the separate combination pass: 118 and
+// 148 + 37 us).
+template <typename T, int LOGN, int WPB>
+struct YShape {
+    static constexpr int N = 1 << LOGN, E = group_elems(LOGN), W = N / E, G = 64 / W, CB = WPB * G, S = CB + 1;
+    static constexpr int NYc = kept_rows(N), a = (NYc - 1) / 2, shift = N - NYc;  // kept rows [0, a] U [N - a, N)
+    static constexpr size_t lds = ((size_t)N + (size_t)(N + N / 8) * S) * sizeof(cpx<T>);
+};
+template <typename T, int LOGN, int WPB>
+__device__ __forceinline__ void k_fft_y_inv_w_body(int bz, DevGeom g, const cpx<T>* __restrict__ lev,
+                                                   const cpx<T>* __restrict__ twN, cpx<T>* __restrict__ hin) {
+    using Y = YShape<T, LOGN, WPB>;
+    constexpr int N = Y::N, W = Y::W, G = Y::G, CB = Y::CB, S = Y::S, E = Y::E, NYc = Y::NYc, a = Y::a;
+    __shared__ cpx<T> tw[N];
+    __shared__ cpx<T> tile[(N + N / 8) * S];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
-    constexpr int NYc = kept_rows(N), a = (NYc - 1) / 2, shift = N - NYc;  // kept rows [0, a] U [N - a, N)
     const int P = g.P, nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y, field = bz;
     const int c = wave * G + grp, kx = kx0 + c;
     for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
     __syncthreads();
-    const cpx<float>* src = lev + ((size_t)field * nq + l) * P + (size_t)kx * NYc;
-    cpx<float> v[1][8];
+    const cpx<T>* src = lev + ((size_t)field * nq + l) * P + (size_t)kx * NYc;
+    cpx<T> v[1][E];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
+    for (int r = 0; r < E; ++r) {
         const int n = j + W * r;
-        v[0][r] = mk(0.f, 0.f);
+        v[0][r] = mk(T(0), T(0));
         if (kx < KX) {
             if (n <= a) v[0][r] = src[n];
-            else if (n >= N - a) v[0][r] = src[n - shift];
+            else if (n >= N - a) v[0][r] = src[n - Y::shift];
         }
     }
     fft_group<LOGN, true, 1, S>(v, tile + c, tw, j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) tile[pad8(j + W * r) * S + c] = v[0][r];
+    for (int r = 0; r < E; ++r) tile[pad8(j + W * r) * S + c] = v[0][r];
     __syncthreads();
     const int ncol = min(CB, KX - kx0);
-    cpx<float>* dst = hin + ((size_t)field * nq + l) * (size_t)N * g.KXp + kx0;
+    cpx<T>* dst = hin + ((size_t)field * nq + l) * (size_t)N * g.KXp + kx0;
     for (int e = threadIdx.x; e < N * CB; e += blockDim.x) {
         const int yy = e / CB, cc = e - yy * CB;
         if (cc < ncol) dst[(size_t)yy * g.KXp + cc] = tile[pad8(yy) * S + cc];
     }
 }
 
-template <int LOGN, int WPB>
-__global__ void __launch_bounds__(64 * WPB) k_fft_y_inv_w(DevGeom g, const cpx<float>* __restrict__ lev,
-                                                     const cpx<float>* __restrict__ twN, cpx<float>* __restrict__ hin) {
-    k_fft_y_inv_w_body<LOGN, WPB>(blockIdx.z, g, lev, twN, hin);
+template <typename T, int LOGN, int WPB>
+__global__ void __launch_bounds__(64 * WPB) k_fft_y_inv_w(DevGeom g, const cpx<T>* __restrict__ lev,
+                                                     const cpx<T>* __restrict__ twN, cpx<T>* __restrict__ hin) {
+    k_fft_y_inv_w_body<T, LOGN, WPB>(blockIdx.z, g, lev, twN, hin);
 }
 // one member's arguments of k_fft_y_inv_w_batch, which runs the k_fft_y_inv_w body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
@@ -438,79 +490,115 @@ template <int LOGN, int WPB>
 __global__ void __launch_bounds__(64 * WPB) k_fft_y_inv_w_batch(const k_fft_y_inv_w_args* __restrict__ tab, int zdim) {
     const int mb = blockIdx.z / zdim;
     const k_fft_y_inv_w_args& a = tab[mb];
-    k_fft_y_inv_w_body<LOGN, WPB>(blockIdx.z - mb * zdim, a.g, a.lev, a.twN, a.hin);
+    k_fft_y_inv_w_body<float, LOGN, WPB>(blockIdx.z - mb * zdim, a.g, a.lev, a.twN, a.hin);
 }
 
 
-template <int LOGN, int WPB>
-__global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_w(DevGeom g, const cpx<float>* __restrict__ hout,
-                                                     const cpx<float>* __restrict__ twN, cpx<float>* __restrict__ prod) {
-    constexpr int N = 1 << LOGN, W = N / 8, G = 64 / W, CB = WPB * G, S = CB + 1;
-    __shared__ cpx<float> tw[N];
-    __shared__ cpx<float> tile[(N + N / 8) * S];
+template <typename T, int LOGN, int WPB>
+__global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_w(DevGeom g, const cpx<T>* __restrict__ hout,
+                                                     const cpx<T>* __restrict__ twN, cpx<T>* __restrict__ prod) {
+    using Y = YShape<T, LOGN, WPB>;
+    constexpr int N = Y::N, W = Y::W, G = Y::G, CB = Y::CB, S = Y::S, E = Y::E, NYc = Y::NYc, a = Y::a;
+    __shared__ cpx<T> tw[N];
+    __shared__ cpx<T> tile[(N + N / 8) * S];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
-    constexpr int NYc = kept_rows(N), a = (NYc - 1) / 2, shift = N - NYc;
     const int P = g.P, nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y, q = blockIdx.z;
     const int c = wave * G + grp, kx = kx0 + c;
     const int ncol = min(CB, KX - kx0);
     for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
-    const cpx<float>* src = hout + ((size_t)q * nq + l) * (size_t)N * g.KXp + kx0;
+    const cpx<T>* src = hout + ((size_t)q * nq + l) * (size_t)N * g.KXp + kx0;
     for (int e = threadIdx.x; e < N * CB; e += blockDim.x) {
         const int yy = e / CB, cc = e - yy * CB;
-        tile[pad8(yy) * S + cc] = (cc < ncol) ? src[(size_t)yy * g.KXp + cc] : mk(0.f, 0.f);
+        tile[pad8(yy) * S + cc] = (cc < ncol) ? src[(size_t)yy * g.KXp + cc] : mk(T(0), T(0));
     }
     __syncthreads();
-    cpx<float> v[1][8];
+    cpx<T> v[1][E];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[0][r] = tile[pad8(j + W * r) * S + c];
+    for (int r = 0; r < E; ++r) v[0][r] = tile[pad8(j + W * r) * S + c];
     wave_sync();  // the column is read before it becomes the scratch
     fft_group<LOGN, false, 1, S>(v, tile + c, tw, j);
     if (kx < KX) {
-        cpx<float>* dst = prod + ((size_t)q * nq + l) * P + (size_t)kx * NYc;
+        cpx<T>* dst = prod + ((size_t)q * nq + l) * P + (size_t)kx * NYc;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < E; ++r) {
             const int n = j + W * r;
             if (n <= a) dst[n] = v[0][r];
-            else if (n >= N - a) dst[n - shift] = v[0][r];
+            else if (n >= N - a) dst[n - Y::shift] = v[0][r];
         }
     }
 }
 
+// Waves per block of the group y-FFTs: cb (kx columns per block asked for, 0: none) in waves of 2, 4 or 8
+// where that was tuned (FP32, N = 64 .. 256); else 4, or as many as the columns fill at the sizes
+// where one wave takes 8 columns or more, and no more than keep the tile within 64 KiB.
+template <typename T, int LOGN>
+constexpr int y_group_max_waves() {
+    return YShape<T, LOGN, 4>::lds <= 65536 ? 4 : (YShape<T, LOGN, 2>::lds <= 65536 ? 2 : 1);
+}
+template <typename T>
+inline int y_group_waves(const DevGeom& g, int most) {
+    const int G = 64 / (g.N / group_elems(g.logN));  // columns per wave
+    int w = 1;
+    while (w < most && w * G < g.KX) w *= 2;
+    return w;
+}
+
 // Launchers of the group y-FFTs for nf fields of g.nq levels each ([field][l][p] spectra,
 // [field][l][y][kx] hybrid rows); cb = kx columns per block (WPB = cb / (512 / N) waves of 2, 4
-// or 8; 0: 4 waves).  false (nothing launched) unless N is 64, 128 or 256.
-template <int LOGN, int WPB>
-inline void launch_y_group_t(bool inv, const DevGeom& g, int nf, const cpx<float>* in, const cpx<float>* twN,
-                             cpx<float>* out, hipStream_t s) {
-    constexpr int CB = WPB * 512 / (1 << LOGN);
-    const dim3 gr((g.KX + CB - 1) / CB, g.nq, nf);
-    if (inv) hipLaunchKernelGGL((k_fft_y_inv_w<LOGN, WPB>), gr, dim3(64 * WPB), 0, s, g, in, twN, out);
-    else hipLaunchKernelGGL((k_fft_y_fwd_w<LOGN, WPB>), gr, dim3(64 * WPB), 0, s, g, in, twN, out);
+// or 8; 0: built-in choice).  false (nothing launched) unless N is 16 .. 1024
+// (FP64: 512).
+template <typename T, int LOGN, int WPB>
+inline void launch_y_group_t(bool inv, const DevGeom& g, int nf, const cpx<T>* in, const cpx<T>* twN,
+                             cpx<T>* out, hipStream_t s) {
+    if constexpr (YShape<T, LOGN, WPB>::lds <= 65536) {
+        constexpr int CB = YShape<T, LOGN, WPB>::CB;
+        const dim3 gr((g.KX + CB - 1) / CB, g.nq, nf);
+        if (inv) hipLaunchKernelGGL((k_fft_y_inv_w<T, LOGN, WPB>), gr, dim3(64 * WPB), 0, s, g, in, twN, out);
+        else hipLaunchKernelGGL((k_fft_y_fwd_w<T, LOGN, WPB>), gr, dim3(64 * WPB), 0, s, g, in, twN, out);
+    }
 }
-template <int LOGN>
-inline void launch_y_group_w(bool inv, int wpb, const DevGeom& g, int nf, const cpx<float>* in,
-                             const cpx<float>* twN, cpx<float>* out, hipStream_t s) {
-    if (wpb == 2) launch_y_group_t<LOGN, 2>(inv, g, nf, in, twN, out, s);
-    else if (wpb == 8) launch_y_group_t<LOGN, 8>(inv, g, nf, in, twN, out, s);
-    else launch_y_group_t<LOGN, 4>(inv, g, nf, in, twN, out, s);
+template <typename T, int LOGN>
+inline void launch_y_group_w(bool inv, int cb, const DevGeom& g, int nf, const cpx<T>* in,
+                             const cpx<T>* twN, cpx<T>* out, hipStream_t s) {
+    if constexpr (sizeof(T) == 4 && LOGN >= 6 && LOGN <= 8) {
+        const int wpb = cb > 0 ? cb / (512 / g.N) : 4;
+        if (wpb == 2) launch_y_group_t<T, LOGN, 2>(inv, g, nf, in, twN, out, s);
+        else if (wpb == 8) launch_y_group_t<T, LOGN, 8>(inv, g, nf, in, twN, out, s);
+        else launch_y_group_t<T, LOGN, 4>(inv, g, nf, in, twN, out, s);
+    } else {
+        const int wpb = y_group_waves<T>(g, y_group_max_waves<T, LOGN>());
+        if (wpb == 1) launch_y_group_t<T, LOGN, 1>(inv, g, nf, in, twN, out, s);
+        else if (wpb == 2) launch_y_group_t<T, LOGN, 2>(inv, g, nf, in, twN, out, s);
+        else launch_y_group_t<T, LOGN, 4>(inv, g, nf, in, twN, out, s);
+    }
 }
-inline bool launch_y_group(bool inv, const DevGeom& g, int nf, const cpx<float>* in, const cpx<float>* twN,
-                           cpx<float>* out, hipStream_t s, int cb = 0) {
-    if (g.N < 64 || g.N > 256 || g.NYc != kept_rows(g.N)) return false;
-    const int wpb = cb > 0 ? cb / (512 / g.N) : 4;
-    if (g.N == 64) launch_y_group_w<6>(inv, wpb, g, nf, in, twN, out, s);
-    else if (g.N == 128) launch_y_group_w<7>(inv, wpb, g, nf, in, twN, out, s);
-    else launch_y_group_w<8>(inv, wpb, g, nf, in, twN, out, s);
+template <typename T>
+inline bool launch_y_group(bool inv, const DevGeom& g, int nf, const cpx<T>* in, const cpx<T>* twN,
+                           cpx<T>* out, hipStream_t s, int cb = 0) {
+    if (g.N < 16 || g.N > (sizeof(T) == 8 ? 512 : 1024) || g.NYc != kept_rows(g.N)) return false;
+    switch (g.logN) {
+        case 4: launch_y_group_w<T, 4>(inv, cb, g, nf, in, twN, out, s); break;
+        case 5: launch_y_group_w<T, 5>(inv, cb, g, nf, in, twN, out, s); break;
+        case 6: launch_y_group_w<T, 6>(inv, cb, g, nf, in, twN, out, s); break;
+        case 7: launch_y_group_w<T, 7>(inv, cb, g, nf, in, twN, out, s); break;
+        case 8: launch_y_group_w<T, 8>(inv, cb, g, nf, in, twN, out, s); break;
+        case 9: launch_y_group_w<T, 9>(inv, cb, g, nf, in, twN, out, s); break;
+        default:
+            if constexpr (sizeof(T) == 4) launch_y_group_w<T, 10>(inv, cb, g, nf, in, twN, out, s);
+            break;
+    }
     return true;
 }
-inline bool launch_y_inv_group(const DevGeom& g, int nf, const cpx<float>* lev, const cpx<float>* twN,
-                               cpx<float>* hin, hipStream_t s, int cb = 0) {
-    return launch_y_group(true, g, nf, lev, twN, hin, s, cb);
+template <typename T>
+inline bool launch_y_inv_group(const DevGeom& g, int nf, const cpx<T>* lev, const cpx<T>* twN,
+                               cpx<T>* hin, hipStream_t s, int cb = 0) {
+    return launch_y_group<T>(true, g, nf, lev, twN, hin, s, cb);
 }
-inline bool launch_y_fwd_group(const DevGeom& g, int nf, const cpx<float>* hout, const cpx<float>* twN,
-                               cpx<float>* prod, hipStream_t s, int cb = 0) {
-    return launch_y_group(false, g, nf, hout, twN, prod, s, cb);
+template <typename T>
+inline bool launch_y_fwd_group(const DevGeom& g, int nf, const cpx<T>* hout, const cpx<T>* twN,
+                               cpx<T>* prod, hipStream_t s, int cb = 0) {
+    return launch_y_group<T>(false, g, nf, hout, twN, prod, s, cb);
 }
 
 }  // namespace rbc

@@ -1561,84 +1561,99 @@ __global__ void __launch_bounds__(192) k_rows512t(DevGeom g, int nblk, int per, 
     }
 }
 
-// x-rows at M = 64, 128, 256 (FP32): one group of W = M / 8 lanes per (level, y) row holding
+// x-rows at M = 16 .. 1024: one group of W = M / E lanes (E = 8; 16 at 1024) per (level, y) row holding
 // the row's three pair transforms in natural layout (fft_group), so the products form in
 // registers between the inverse and the forward transforms; 64 / W rows per wave, WPB waves per
-// block.  Same arithmetic as k_rows512t: both members of every input and product pair are
-// balanced by a power of two (pair_scale over the row, a shuffle reduction over the group).
-template <int LOGM, int WPB>
-__device__ __forceinline__ void k_rows_w_body(DevGeom g, const cpx<float>* __restrict__ hin,
-                                              const cpx<float>* __restrict__ twM, cpx<float>* __restrict__ hout) {
-    constexpr int M = 1 << LOGM, W = M / 8, G = 64 / W, RPB = WPB * G, SP = M + M / 8, KX = kept_cols(M);
-    __shared__ cpx<float> tw[M];
-    __shared__ cpx<float> scr[RPB][SP];
+// block, the nq N rows in one flat range (rows past its end are computed on the last row and not
+// stored).  Same arithmetic as k_rows512t: both members of every input and product pair are
+// balanced by a power of two (pair_scale over the row, a reduction over the group).
+// FP64 (also 16 and 32 points, and FP32 512 beside another N, 1024): the three pairs take 96
+// registers of the 256 a lane has at two waves per SIMD.  Bound: HBM for the hybrid rows, 12 nq N KX
+// values.  256^2 x 24 FP64: 101 us (3.4 TB/s; the
+// LDS radix-4 form it replaces there: 243 us); 1024 x 128 x 40 FP32: 173 us (579).
+template <typename T, int LOGM, int WPB>
+struct RowShape {
+    static constexpr int M = 1 << LOGM, E = group_elems(LOGM), W = M / E, G = 64 / W, RPB = WPB * G, SP = M + M / 8;
+    static constexpr size_t lds = ((size_t)M + (size_t)RPB * SP) * sizeof(cpx<T>);
+};
+template <typename T, int LOGM, int WPB>
+__device__ __forceinline__ void k_rows_w_body(DevGeom g, const cpx<T>* __restrict__ hin,
+                                              const cpx<T>* __restrict__ twM, cpx<T>* __restrict__ hout) {
+    using R = RowShape<T, LOGM, WPB>;
+    constexpr int M = R::M, E = R::E, W = R::W, G = R::G, RPB = R::RPB, KX = kept_cols(M);
+    __shared__ cpx<T> tw[M];
+    __shared__ cpx<T> scr[RPB][R::SP];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
     const int KXp = g.KXp, nq = g.nq, N = g.N;
-    const int y = blockIdx.x * RPB + wave * G + grp, l = blockIdx.y;
+    const int rw = blockIdx.x * RPB + wave * G + grp;
+    const bool valid = rw < nq * N;
     const size_t fstride = (size_t)nq * N * KXp;
-    const size_t roff = ((size_t)l * N + y) * KXp;
+    const size_t roff = (size_t)min(rw, nq * N - 1) * KXp;
     for (int e = threadIdx.x; e < M; e += blockDim.x) tw[e] = twM[e];
     __syncthreads();
-    cpx<float>* sb = scr[wave * G + grp];
+    cpx<T>* sb = scr[wave * G + grp];
     auto gmax = [](float x) { return group_max<W>(x); };
-    cpx<float> v[3][8];
-    float isg[3];
+    auto mag = [](T x) { return fabsf((float)x); };
+    cpx<T> v[3][E];
+    T isg[3];
 #pragma unroll
     for (int pr = 0; pr < 3; ++pr) {
-        const cpx<float>* x1 = hin + (size_t)(2 * pr) * fstride + roff;
-        const cpx<float>* x2 = hin + (size_t)(2 * pr + 1) * fstride + roff;
-        cpx<float> a[8], b[8];
+        const cpx<T>* x1 = hin + (size_t)(2 * pr) * fstride + roff;
+        const cpx<T>* x2 = hin + (size_t)(2 * pr + 1) * fstride + roff;
+        cpx<T> a[E], b[E];
         float ma = 0.f, mb = 0.f;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < E; ++r) {
             const int k = j + W * r;
             const int src = k < KX ? k : (k > M - KX ? M - k : -1);
-            a[r] = b[r] = mk(0.f, 0.f);
+            a[r] = b[r] = mk(T(0), T(0));
             if (src >= 0) {
                 a[r] = x1[src];
                 b[r] = x2[src];
                 if (src == 0) {  // a C2R ignores the imaginary part at kx = 0
-                    a[r].y = 0.f;
-                    b[r].y = 0.f;
+                    a[r].y = T(0);
+                    b[r].y = T(0);
                 }
             }
-            ma = fmaxf(ma, fmaxf(fabsf(a[r].x), fabsf(a[r].y)));
-            mb = fmaxf(mb, fmaxf(fabsf(b[r].x), fabsf(b[r].y)));
+            ma = fmaxf(ma, fmaxf(mag(a[r].x), mag(a[r].y)));
+            mb = fmaxf(mb, fmaxf(mag(b[r].x), mag(b[r].y)));
         }
-        const float sg = pair_scale(gmax(ma), gmax(mb));
-        isg[pr] = inv_pow2(sg);
+        const float sgf = pair_scale(gmax(ma), gmax(mb));
+        const T sg = sgf;
+        isg[pr] = inv_pow2(sgf);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < E; ++r) {
             const int k = j + W * r;
-            const cpx<float> bs = mk(sg * b[r].x, sg * b[r].y);
+            const cpx<T> bs = mk(sg * b[r].x, sg * b[r].y);
             if (k < KX) v[pr][r] = mk(a[r].x - bs.y, a[r].y + bs.x);               // X1 + i s X2
             else if (k > M - KX) v[pr][r] = mk(a[r].x + bs.y, -a[r].y + bs.x);     // conj(X1) + i s conj(X2)
-            else v[pr][r] = mk(0.f, 0.f);
+            else v[pr][r] = mk(T(0), T(0));
         }
     }
     fft_group<LOGM, true, 3>(v, sb, tw, j);
     // products at x = j + W r, in place, scaled by 1 / (M N)
-    const float s = 1.f / ((float)M * (float)N);
+    const T s = T(1) / (T(M) * T(N));
     float pa[3] = {0.f, 0.f, 0.f}, pb[3] = {0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const float u = v[0][r].x, vv = isg[0] * v[0][r].y, w = v[1][r].x, tx = isg[1] * v[1][r].y;
-        const float ty = v[2][r].x, tz = isg[2] * v[2][r].y;
-        v[0][r] = mk(s * (u * u + vv * vv - 2.f * w * w), s * (u * u - vv * vv));
+    for (int r = 0; r < E; ++r) {
+        const T u = v[0][r].x, vv = isg[0] * v[0][r].y, w = v[1][r].x, tx = isg[1] * v[1][r].y;
+        const T ty = v[2][r].x, tz = isg[2] * v[2][r].y;
+        v[0][r] = mk(s * (u * u + vv * vv - T(2) * w * w), s * (u * u - vv * vv));
         v[1][r] = mk(s * u * vv, s * u * w);
         v[2][r] = mk(s * vv * w, s * (u * tx + vv * ty + w * tz));
 #pragma unroll
         for (int pr = 0; pr < 3; ++pr) {
-            pa[pr] = fmaxf(pa[pr], fabsf(v[pr][r].x));
-            pb[pr] = fmaxf(pb[pr], fabsf(v[pr][r].y));
+            pa[pr] = fmaxf(pa[pr], mag(v[pr][r].x));
+            pb[pr] = fmaxf(pb[pr], mag(v[pr][r].y));
         }
     }
 #pragma unroll
     for (int pr = 0; pr < 3; ++pr) {
-        const float sg = pair_scale(gmax(pa[pr]), gmax(pb[pr]));
-        isg[pr] = inv_pow2(sg);
+        const float sgf = pair_scale(gmax(pa[pr]), gmax(pb[pr]));
+        const T sg = sgf;
+        isg[pr] = inv_pow2(sgf);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) v[pr][r].y *= sg;
+        for (int r = 0; r < E; ++r) v[pr][r].y *= sg;
     }
     fft_group<LOGM, false, 3>(v, sb, tw, j);
     // unpack X1_k = (Z_k + conj Z_{M-k}) / 2, X2_k = -i (Z_k - conj Z_{M-k}) / (2 s); Z_{M-k} of
@@ -1646,27 +1661,27 @@ __device__ __forceinline__ void k_rows_w_body(DevGeom g, const cpx<float>* __res
 #pragma unroll
     for (int pr = 0; pr < 3; ++pr) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) sb[pad8(j + W * r)] = v[pr][r];
+        for (int r = 0; r < E; ++r) sb[pad8(j + W * r)] = v[pr][r];
         wave_sync();
-        cpx<float>* o1 = hout + (size_t)(2 * pr) * fstride + roff;
-        cpx<float>* o2 = hout + (size_t)(2 * pr + 1) * fstride + roff;
+        cpx<T>* o1 = hout + (size_t)(2 * pr) * fstride + roff;
+        cpx<T>* o2 = hout + (size_t)(2 * pr + 1) * fstride + roff;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < E; ++r) {
             const int k = j + W * r;
-            if (k < KX) {
-                const cpx<float> zk = v[pr][r], zm = sb[pad8((M - k) & (M - 1))];
-                o1[k] = mk(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-                o2[k] = mk(0.5f * isg[pr] * (zk.y + zm.y), -0.5f * isg[pr] * (zk.x - zm.x));
+            if (k < KX && valid) {
+                const cpx<T> zk = v[pr][r], zm = sb[pad8((M - k) & (M - 1))];
+                o1[k] = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
+                o2[k] = mk(T(0.5) * isg[pr] * (zk.y + zm.y), T(-0.5) * isg[pr] * (zk.x - zm.x));
             }
         }
         wave_sync();  // the scratch is rewritten by the next pair
     }
 }
 
-template <int LOGM, int WPB>
-__global__ void __launch_bounds__(64 * WPB) k_rows_w(DevGeom g, const cpx<float>* __restrict__ hin,
-                                                const cpx<float>* __restrict__ twM, cpx<float>* __restrict__ hout) {
-    k_rows_w_body<LOGM, WPB>(g, hin, twM, hout);
+template <typename T, int LOGM, int WPB>
+__global__ void __launch_bounds__(64 * WPB) k_rows_w(DevGeom g, const cpx<T>* __restrict__ hin,
+                                                const cpx<T>* __restrict__ twM, cpx<T>* __restrict__ hout) {
+    k_rows_w_body<T, LOGM, WPB>(g, hin, twM, hout);
 }
 // one member's arguments of k_rows_w_batch, which runs the k_rows_w body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
@@ -1680,7 +1695,7 @@ template <int LOGM, int WPB>
 __global__ void __launch_bounds__(64 * WPB) k_rows_w_batch(const k_rows_w_args* __restrict__ tab, int zdim) {
     const int mb = blockIdx.z / zdim;
     const k_rows_w_args& a = tab[mb];
-    k_rows_w_body<LOGM, WPB>(a.g, a.hin, a.twM, a.hout);
+    k_rows_w_body<float, LOGM, WPB>(a.g, a.hin, a.twM, a.hout);
 }
 
 
@@ -2219,17 +2234,19 @@ template <>
 struct YGroup<0> {
     static constexpr int n = 3, t0 = 0, t1 = 2, t2 = -1;
     __device__ static int q(int i) { return i; }
-    __device__ static void add(int i, cpx<float> V, float kx, float ky, cpx<float>& d0, cpx<float>& d1, cpx<float>&) {
-        if (i == 0) { d0 = d0 + cscale(V, 0.5f * (kx * kx + ky * ky)); }
-        else if (i == 1) { d0 = d0 + cscale(V, 0.5f * (kx * kx - ky * ky)); d1 = d1 + cscale(V, -kx * ky); }
-        else { d0 = d0 + cscale(V, 2.f * kx * ky); d1 = d1 + cscale(V, kx * kx - ky * ky); }
+    template <typename T>
+    __device__ static void add(int i, cpx<T> V, T kx, T ky, cpx<T>& d0, cpx<T>& d1, cpx<T>&) {
+        if (i == 0) { d0 = d0 + cscale(V, T(0.5) * (kx * kx + ky * ky)); }
+        else if (i == 1) { d0 = d0 + cscale(V, T(0.5) * (kx * kx - ky * ky)); d1 = d1 + cscale(V, -kx * ky); }
+        else { d0 = d0 + cscale(V, T(2) * kx * ky); d1 = d1 + cscale(V, kx * kx - ky * ky); }
     }
 };
 template <>
 struct YGroup<1> {  // uw, vw -> D1, D3
     static constexpr int n = 2, t0 = 1, t1 = 3, t2 = -1;
     __device__ static int q(int i) { return 3 + i; }
-    __device__ static void add(int i, cpx<float> V, float kx, float ky, cpx<float>& d0, cpx<float>& d1, cpx<float>&) {
+    template <typename T>
+    __device__ static void add(int i, cpx<T> V, T kx, T ky, cpx<T>& d0, cpx<T>& d1, cpx<T>&) {
         if (i == 0) { d0 = d0 + imul(V, kx); d1 = d1 - imul(V, ky); }
         else { d0 = d0 + imul(V, ky); d1 = d1 + imul(V, kx); }
     }
@@ -2238,7 +2255,8 @@ template <>
 struct YGroup<2> {  // u.grad(theta) -> D4
     static constexpr int n = 1, t0 = 4, t1 = -1, t2 = -1;
     __device__ static int q(int) { return 5; }
-    __device__ static void add(int, cpx<float> V, float, float, cpx<float>& d0, cpx<float>&, cpx<float>&) {
+    template <typename T>
+    __device__ static void add(int, cpx<T> V, T, T, cpx<T>& d0, cpx<T>&, cpx<T>&) {
         d0 = d0 + V;
     }
 };
@@ -2246,8 +2264,8 @@ template <>
 struct YGroup<3> {  // groups 1 and 2 in one pass: uw, vw, u.grad(theta) -> D1, D3, D4
     static constexpr int n = 3, t0 = 1, t1 = 3, t2 = 4;
     __device__ static int q(int i) { return 3 + i; }
-    __device__ static void add(int i, cpx<float> V, float kx, float ky, cpx<float>& d0, cpx<float>& d1,
-                               cpx<float>& d2) {
+    template <typename T>
+    __device__ static void add(int i, cpx<T> V, T kx, T ky, cpx<T>& d0, cpx<T>& d1, cpx<T>& d2) {
         if (i == 0) { d0 = d0 + imul(V, kx); d1 = d1 - imul(V, ky); }
         else if (i == 1) { d0 = d0 + imul(V, ky); d1 = d1 + imul(V, kx); }
         else { d2 = d2 + V; }
@@ -2359,20 +2377,20 @@ __global__ void __launch_bounds__(64 * CT) k_fft_y_fwd512c2(DevGeom g, int ntile
     else y_fwd512c_body<0, CT>(lb >> 1, g, ntile, hout, tw, kxa, kya, D, fgw, tile, twl);
 }
 
-// Forward y-FFT at N = 64, 128, 256 fused with the level combinations (FP32): blockIdx.z = the
+// Forward y-FFT at N = 16 .. 1024 fused with the level combinations: blockIdx.z = the
 // combination group of YGroup (0: h, d, uv -> D0, D2; 1: uw, vw -> D1, D3 and the k = 0 values
 // of P_uw, P_vw; 2: u.grad(theta) -> D4).  A block of WPB waves handles CB kx columns of one
 // level, one group of W = N / 8 lanes per column (fft_group, natural layout); the group's
 // products are transformed in turn through the LDS tile and their combinations accumulate in
 // registers.  Writes D[t][l][p] into the level buffer (free once the inverse y-FFT has read it).
-template <int LOGN, int WPB, int GRP>
-__device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<float>* tile, const cpx<float>* tw,
-                                                 const cpx<float>* __restrict__ hout, const float* __restrict__ kxa,
-                                                 const float* __restrict__ kya, cpx<float>* __restrict__ D,
-                                                 cpx<float>* __restrict__ fgw) {
+template <typename T, int LOGN, int WPB, int GRP>
+__device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<T>* tile, const cpx<T>* tw,
+                                                 const cpx<T>* __restrict__ hout, const T* __restrict__ kxa,
+                                                 const T* __restrict__ kya, cpx<T>* __restrict__ D,
+                                                 cpx<T>* __restrict__ fgw) {
     using Gr = YGroup<GRP>;
-    constexpr int N = 1 << LOGN, W = N / 8, G = 64 / W, CB = WPB * G, S = CB + 1;
-    constexpr int NYc = kept_rows(N), a = (NYc - 1) / 2, shift = N - NYc;
+    using Y = YShape<T, LOGN, WPB>;
+    constexpr int N = Y::N, E = Y::E, W = Y::W, G = Y::G, CB = Y::CB, S = Y::S, NYc = Y::NYc, a = Y::a, shift = Y::shift;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
     const int P = g.P, nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y;
@@ -2380,32 +2398,32 @@ __device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<float>* t
     const bool cvalid = kx < KX;
     const int ncol = min(CB, KX - kx0);
     auto kyc_of = [](int n) { return n <= a ? n : (n >= N - a ? n - shift : -1); };
-    const float kxv = cvalid ? kxa[(size_t)kx * NYc] : 0.f;
-    float kyv[8];
+    const T kxv = cvalid ? kxa[(size_t)kx * NYc] : T(0);
+    T kyv[E];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
+    for (int r = 0; r < E; ++r) {
         const int kc = kyc_of(j + W * r);
-        kyv[r] = (cvalid && kc >= 0) ? kya[(size_t)kx * NYc + kc] : 0.f;
+        kyv[r] = (cvalid && kc >= 0) ? kya[(size_t)kx * NYc + kc] : T(0);
     }
-    cpx<float> d0[8], d1[8];
+    cpx<T> d0[E], d1[E];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) d0[r] = d1[r] = mk(0.f, 0.f);
+    for (int r = 0; r < E; ++r) d0[r] = d1[r] = mk(T(0), T(0));
 #pragma unroll
     for (int iq = 0; iq < Gr::n; ++iq) {
-        const cpx<float>* src = hout + ((size_t)Gr::q(iq) * nq + l) * (size_t)N * g.KXp + kx0;
+        const cpx<T>* src = hout + ((size_t)Gr::q(iq) * nq + l) * (size_t)N * g.KXp + kx0;
         for (int e = threadIdx.x; e < N * CB; e += blockDim.x) {
             const int yy = e / CB, cc = e - yy * CB;
-            tile[pad8(yy) * S + cc] = (cc < ncol) ? src[(size_t)yy * g.KXp + cc] : mk(0.f, 0.f);
+            tile[pad8(yy) * S + cc] = (cc < ncol) ? src[(size_t)yy * g.KXp + cc] : mk(T(0), T(0));
         }
         __syncthreads();
-        cpx<float> v[1][8];
+        cpx<T> v[1][E];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) v[0][r] = tile[pad8(j + W * r) * S + c];
+        for (int r = 0; r < E; ++r) v[0][r] = tile[pad8(j + W * r) * S + c];
         wave_sync();  // the column is read before it becomes the scratch
         fft_group<LOGN, false, 1, S>(v, tile + c, tw, j);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            cpx<float> unused;
+        for (int r = 0; r < E; ++r) {
+            cpx<T> unused;
             Gr::add(iq, v[0][r], kxv, kyv[r], d0[r], d1[r], unused);
         }
         if (GRP == 1 && kx == 0 && j == 0) fgw[2 * l + iq] = v[0][0];  // P_uw, P_vw at (0, 0)
@@ -2413,9 +2431,9 @@ __device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<float>* t
     }
     if (cvalid) {
         const size_t fs = (size_t)nq * P;
-        cpx<float>* o = D + (size_t)l * P + (size_t)kx * NYc;
+        cpx<T>* o = D + (size_t)l * P + (size_t)kx * NYc;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < E; ++r) {
             const int kc = kyc_of(j + W * r);
             if (kc >= 0) {
                 o[Gr::t0 * fs + kc] = d0[r];
@@ -2425,27 +2443,27 @@ __device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<float>* t
     }
 }
 
-template <int LOGN, int WPB>
-__device__ __forceinline__ void k_fft_y_fwd_wc_body(int bz, DevGeom g, const cpx<float>* __restrict__ hout,
-                                                    const cpx<float>* __restrict__ twN,
-                                                    const float* __restrict__ kxa, const float* __restrict__ kya,
-                                                    cpx<float>* __restrict__ D, cpx<float>* __restrict__ fgw) {
-    constexpr int N = 1 << LOGN, W = N / 8, G = 64 / W, CB = WPB * G, S = CB + 1;
-    __shared__ cpx<float> tw[N];
-    __shared__ cpx<float> tile[(N + N / 8) * S];
+template <typename T, int LOGN, int WPB>
+__device__ __forceinline__ void k_fft_y_fwd_wc_body(int bz, DevGeom g, const cpx<T>* __restrict__ hout,
+                                                    const cpx<T>* __restrict__ twN,
+                                                    const T* __restrict__ kxa, const T* __restrict__ kya,
+                                                    cpx<T>* __restrict__ D, cpx<T>* __restrict__ fgw) {
+    constexpr int N = 1 << LOGN, S = YShape<T, LOGN, WPB>::S;
+    __shared__ cpx<T> tw[N];
+    __shared__ cpx<T> tile[(N + N / 8) * S];
     for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
     __syncthreads();
-    if (bz == 0) y_fwd_group_comb<LOGN, WPB, 0>(g, tile, tw, hout, kxa, kya, D, fgw);
-    else if (bz == 1) y_fwd_group_comb<LOGN, WPB, 1>(g, tile, tw, hout, kxa, kya, D, fgw);
-    else y_fwd_group_comb<LOGN, WPB, 2>(g, tile, tw, hout, kxa, kya, D, fgw);
+    if (bz == 0) y_fwd_group_comb<T, LOGN, WPB, 0>(g, tile, tw, hout, kxa, kya, D, fgw);
+    else if (bz == 1) y_fwd_group_comb<T, LOGN, WPB, 1>(g, tile, tw, hout, kxa, kya, D, fgw);
+    else y_fwd_group_comb<T, LOGN, WPB, 2>(g, tile, tw, hout, kxa, kya, D, fgw);
 }
 
-template <int LOGN, int WPB>
-__global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_wc(DevGeom g, const cpx<float>* __restrict__ hout,
-                                                          const cpx<float>* __restrict__ twN,
-                                                          const float* __restrict__ kxa, const float* __restrict__ kya,
-                                                          cpx<float>* __restrict__ D, cpx<float>* __restrict__ fgw) {
-    k_fft_y_fwd_wc_body<LOGN, WPB>(blockIdx.z, g, hout, twN, kxa, kya, D, fgw);
+template <typename T, int LOGN, int WPB>
+__global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_wc(DevGeom g, const cpx<T>* __restrict__ hout,
+                                                          const cpx<T>* __restrict__ twN,
+                                                          const T* __restrict__ kxa, const T* __restrict__ kya,
+                                                          cpx<T>* __restrict__ D, cpx<T>* __restrict__ fgw) {
+    k_fft_y_fwd_wc_body<T, LOGN, WPB>(blockIdx.z, g, hout, twN, kxa, kya, D, fgw);
 }
 // one member's arguments of k_fft_y_fwd_wc_batch, which runs the k_fft_y_fwd_wc body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
@@ -2462,7 +2480,7 @@ template <int LOGN, int WPB>
 __global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_wc_batch(const k_fft_y_fwd_wc_args* __restrict__ tab, int zdim) {
     const int mb = blockIdx.z / zdim;
     const k_fft_y_fwd_wc_args& a = tab[mb];
-    k_fft_y_fwd_wc_body<LOGN, WPB>(blockIdx.z - mb * zdim, a.g, a.hout, a.twN, a.kxa, a.kya, a.D, a.fgw);
+    k_fft_y_fwd_wc_body<float, LOGN, WPB>(blockIdx.z - mb * zdim, a.g, a.hout, a.twN, a.kxa, a.kya, a.D, a.fgw);
 }
 
 
@@ -2496,16 +2514,16 @@ template <typename T>
 static bool fast512_y(const DevGeom& g) {
     return fast512_rows<T>(g);
 }
-// group (natural-layout) transforms for FP32 grids of 64, 128 and 256 points: log2 of the size,
-// or 0 when the generic kernels run
+// group (natural-layout) transforms for grids of 16 .. 1024 points (FP64: 512): log2 of the
+// size, or 0 when the generic kernels run
 template <typename T>
 static int wave_rows_log(const DevGeom& g) {
-    if (sizeof(T) != 4 || generic_fft_forced() || g.M < 64 || g.M > 256 || g.KX != kept_cols(g.M)) return 0;
+    if (generic_fft_forced() || g.M < 16 || g.M > (sizeof(T) == 8 ? 512 : 1024) || g.KX != kept_cols(g.M)) return 0;
     return g.logM;
 }
 template <typename T>
 static int wave_y_log(const DevGeom& g) {
-    if (sizeof(T) != 4 || generic_fft_forced() || g.N < 64 || g.N > 256) return 0;
+    if (generic_fft_forced() || g.N < 16 || g.N > (sizeof(T) == 8 ? 512 : 1024) || g.NYc != kept_rows(g.N)) return 0;
     return g.logN;
 }
 
@@ -2515,6 +2533,54 @@ static inline int fft_tile(int N, size_t csz) {
     if (tx > 16) tx = 16;
     if (tx < 1) tx = 1;
     return tx;
+}
+
+template <typename T, int LOGM, int WPB>
+static void launch_rows_w_t(const DevGeom& g, const Buffers& b, hipStream_t s) {
+    if constexpr (RowShape<T, LOGM, WPB>::lds <= 65536) {
+        constexpr int RPB = RowShape<T, LOGM, WPB>::RPB;
+        const dim3 gr((g.N * g.nq + RPB - 1) / RPB);
+        hipLaunchKernelGGL((k_rows_w<T, LOGM, WPB>), gr, dim3(64 * WPB), 0, s, g, (const cpx<T>*)b.hin,
+                           (const cpx<T>*)b.twM, (cpx<T>*)b.hout);
+    }
+}
+template <typename T, int LOGM>
+static void launch_rows_w(const DevGeom& g, const Buffers& b, int wpb, hipStream_t s) {
+    if constexpr (sizeof(T) == 4 && LOGM >= 6 && LOGM <= 8) {
+        if (wpb == 2) launch_rows_w_t<T, LOGM, 2>(g, b, s);
+        else if (wpb == 8) launch_rows_w_t<T, LOGM, 8>(g, b, s);
+        else launch_rows_w_t<T, LOGM, 4>(g, b, s);
+    } else {
+        // one or two waves a block while the rows are too few to give every CU a block of four
+        const int waves = (g.N * g.nq + RowShape<T, LOGM, 1>::RPB - 1) / RowShape<T, LOGM, 1>::RPB;
+        if (waves <= 512) launch_rows_w_t<T, LOGM, 1>(g, b, s);
+        else if (waves <= 1024) launch_rows_w_t<T, LOGM, 2>(g, b, s);
+        else launch_rows_w_t<T, LOGM, 4>(g, b, s);
+    }
+}
+template <typename T, int LOGN, int WPB>
+static void launch_y_fwd_wc_t(const DevGeom& g, const Buffers& b, hipStream_t s) {
+    if constexpr (YShape<T, LOGN, WPB>::lds <= 65536) {
+        constexpr int CB = YShape<T, LOGN, WPB>::CB;
+        const dim3 gr((g.KX + CB - 1) / CB, g.nq, 3);
+        hipLaunchKernelGGL((k_fft_y_fwd_wc<T, LOGN, WPB>), gr, dim3(64 * WPB), 0, s, g, (const cpx<T>*)b.hout,
+                           (const cpx<T>*)b.twN, (const T*)b.kx, (const T*)b.ky, (cpx<T>*)b.lev, (cpx<T>*)b.fgw);
+    }
+}
+template <typename T, int LOGN>
+static void launch_y_fwd_wc(const DevGeom& g, const Buffers& b, hipStream_t s) {
+    if constexpr (sizeof(T) == 4 && LOGN >= 6 && LOGN <= 8) {
+        // default: 2 waves per block at N = 64 (more blocks on the small grids), else 4
+        const int G = 512 / g.N, wpb = b.tune_ytx > 0 && b.tune_ytx / G >= 2 ? b.tune_ytx / G : (g.N <= 64 ? 2 : 4);
+        if (wpb == 2) launch_y_fwd_wc_t<T, LOGN, 2>(g, b, s);
+        else if (wpb == 8) launch_y_fwd_wc_t<T, LOGN, 8>(g, b, s);
+        else launch_y_fwd_wc_t<T, LOGN, 4>(g, b, s);
+    } else {
+        const int wpb = y_group_waves<T>(g, y_group_max_waves<T, LOGN>());
+        if (wpb == 1) launch_y_fwd_wc_t<T, LOGN, 1>(g, b, s);
+        else if (wpb == 2) launch_y_fwd_wc_t<T, LOGN, 2>(g, b, s);
+        else launch_y_fwd_wc_t<T, LOGN, 4>(g, b, s);
+    }
 }
 
 template <typename T>
@@ -2564,8 +2630,8 @@ void Launch<T>::fft_y_inv(const DevGeom& g, const Buffers& b, hipStream_t s) {
                            (const cpx<float>*)b.lev, (const cpx<float>*)b.twP, (cpx<float>*)b.hin);
         return;
     }
-    if (wave_y_log<T>(g) && launch_y_inv_group(g, 6, (const cpx<float>*)b.lev, (const cpx<float>*)b.twN,
-                                               (cpx<float>*)b.hin, s, b.tune_ytx))
+    if (wave_y_log<T>(g) &&
+        launch_y_inv_group<T>(g, 6, (const cpx<T>*)b.lev, (const cpx<T>*)b.twN, (cpx<T>*)b.hin, s, b.tune_ytx))
         return;
     const int TX = b.tune_ytx > 0 ? b.tune_ytx : fft_tile(g.N, sizeof(cpx<T>));
     dim3 grid((g.KX + TX - 1) / TX, g.nq, 6);
@@ -2583,23 +2649,19 @@ void Launch<T>::rows(const DevGeom& g, const Buffers& b, hipStream_t s) {
         return;
     }
     if (const int lg = wave_rows_log<T>(g)) {
-        const int wpb = b.tune_rows_threads > 0 ? b.tune_rows_threads / 64 : 4;
-        if (g.N % (wpb * 512 / g.M) == 0) {
-            const dim3 gr(g.N / (wpb * 512 / g.M), g.nq);
-#define RBC_ROWSW(LG, WPBV)                                                                                        \
-    hipLaunchKernelGGL((k_rows_w<LG, WPBV>), gr, dim3(64 * WPBV), 0, s, g, (const cpx<float>*)b.hin,                \
-                       (const cpx<float>*)b.twM, (cpx<float>*)b.hout)
-#define RBC_ROWSW_L(LG)              \
-    if (wpb == 2) RBC_ROWSW(LG, 2);  \
-    else if (wpb == 8) RBC_ROWSW(LG, 8); \
-    else RBC_ROWSW(LG, 4)
-            if (lg == 6) { RBC_ROWSW_L(6); }
-            else if (lg == 7) { RBC_ROWSW_L(7); }
-            else { RBC_ROWSW_L(8); }
-#undef RBC_ROWSW_L
-#undef RBC_ROWSW
-            return;
+        const int tuned = b.tune_rows_threads > 0 ? b.tune_rows_threads / 64 : 4;
+        switch (lg) {
+            case 4: launch_rows_w<T, 4>(g, b, 4, s); break;
+            case 5: launch_rows_w<T, 5>(g, b, 4, s); break;
+            case 6: launch_rows_w<T, 6>(g, b, tuned, s); break;
+            case 7: launch_rows_w<T, 7>(g, b, tuned, s); break;
+            case 8: launch_rows_w<T, 8>(g, b, tuned, s); break;
+            case 9: launch_rows_w<T, 9>(g, b, 4, s); break;
+            default:
+                if constexpr (sizeof(T) == 4) launch_rows_w<T, 10>(g, b, 4, s);
+                break;
         }
+        return;
     }
     const int nth = b.tune_rows_threads > 0 ? b.tune_rows_threads : 256;
     // rows per block: RB M = 512 for M >= 64 (at most 8 rows, at most nth / 32 so that a row keeps
@@ -2632,23 +2694,21 @@ void Launch<T>::fft_y_fwd(const DevGeom& g, const Buffers& b, hipStream_t s) {
                            (const float*)b.ky, (cpx<float>*)b.lev, (cpx<float>*)b.fgw);
         return;
     }
-    if (wave_y_log<T>(g) && g.NYc == kept_rows(g.N)) {
-        // default: 2 waves per block at N = 64 (more blocks on the small grids), else 4
-        const int G = 512 / g.N, wpb = b.tune_ytx > 0 && b.tune_ytx / G >= 2 ? b.tune_ytx / G : (g.N <= 64 ? 2 : 4);
-        const dim3 gr((g.KX + wpb * G - 1) / (wpb * G), g.nq, 3);
-#define RBC_YFWDC(LG, WPBV)                                                                                        \
-    hipLaunchKernelGGL((k_fft_y_fwd_wc<LG, WPBV>), gr, dim3(64 * WPBV), 0, s, g, (const cpx<float>*)b.hout,        \
-                       (const cpx<float>*)b.twN, (const float*)b.kx, (const float*)b.ky, (cpx<float>*)b.lev,   \
-                       (cpx<float>*)b.fgw)
-#define RBC_YFWDC_L(LG)                  \
-    if (wpb == 2) RBC_YFWDC(LG, 2);      \
-    else if (wpb == 8) RBC_YFWDC(LG, 8); \
-    else RBC_YFWDC(LG, 4)
-        if (g.N == 64) { RBC_YFWDC_L(6); }
-        else if (g.N == 128) { RBC_YFWDC_L(7); }
-        else { RBC_YFWDC_L(8); }
-#undef RBC_YFWDC_L
-#undef RBC_YFWDC
+    // columns of 16 and 32 points: a wave takes 32 or 16 of them, so the fused form, whose blocks go
+    // through a group's products in turn, needs enough columns (32 x 32 x 8 FP64, 480 columns: 12.0
+    // us against 7.5 us for the generic transform and k_combine)
+    if (wave_y_log<T>(g) && (g.N >= 64 || g.nq * g.KX >= 4096)) {
+        switch (g.logN) {
+            case 4: launch_y_fwd_wc<T, 4>(g, b, s); break;
+            case 5: launch_y_fwd_wc<T, 5>(g, b, s); break;
+            case 6: launch_y_fwd_wc<T, 6>(g, b, s); break;
+            case 7: launch_y_fwd_wc<T, 7>(g, b, s); break;
+            case 8: launch_y_fwd_wc<T, 8>(g, b, s); break;
+            case 9: launch_y_fwd_wc<T, 9>(g, b, s); break;
+            default:
+                if constexpr (sizeof(T) == 4) launch_y_fwd_wc<T, 10>(g, b, s);
+                break;
+        }
         return;
     }
     {
@@ -2918,8 +2978,8 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
     const Buffers& b0 = *m[0].b;
     // the single-run path these kernels stand for: FP32 storage on the matrix cores, group
     // transforms in both directions, the register group update
-    if (b0.mma < 0 || g.L > 32 || !wave_rows_log<float>(g) || !wave_y_log<float>(g) || g.NYc != kept_rows(g.N) ||
-        fast512_rows<float>(g) || fast512_y<float>(g)) {
+    const bool sized = g.M >= 64 && g.M <= 256 && g.N >= 64 && g.N <= 256;
+    if (b0.mma < 0 || g.L > 32 || !sized || !wave_rows_log<float>(g) || !wave_y_log<float>(g)) {
         why = "not on the batched path (FP32/BF16X3 storage, 64..256-point group transforms, L <= 32)";
         return nullptr;
     }
@@ -3042,7 +3102,8 @@ void batch_step(const StepBatch* sb, hipStream_t s) {
     }
     {
         const int wpb = sb->rows_wpb;
-        const dim3 gr(g.N / (wpb * 512 / g.M), g.nq, B);
+        const int rpb = wpb * 512 / g.M;
+        const dim3 gr((g.N * g.nq + rpb - 1) / rpb, 1, B);
 #define RBC_RWB(LG, WPBV) hipLaunchKernelGGL((k_rows_w_batch<LG, WPBV>), gr, dim3(64 * WPBV), 0, s, sb->rw, 1)
 #define RBC_RWB_L(LG)                \
     if (wpb == 2) RBC_RWB(LG, 2);      \

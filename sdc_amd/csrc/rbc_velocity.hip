@@ -1082,7 +1082,7 @@ void velocity_grid(rbc_ctx* c, const GridWork& w) {
     gt.nq = w.nz;
     if (c->rsz == 8) launch_vel_levels<double>(c, gt, w.nz, w.zb, w.spec);
     else launch_vel_levels<float>(c, gt, w.nz, w.zb, w.spec);
-    if (!launch_y_inv_group(gt, 3, (const cpx<float>*)w.spec, (const cpx<float>*)w.twN, w.hyb, c->stream)) {
+    if (!launch_y_inv_group<float>(gt, 3, (const cpx<float>*)w.spec, (const cpx<float>*)w.twN, w.hyb, c->stream)) {
         int TX = (int)(65536 / (2 * (size_t)gt.N * sizeof(cpx<float>)));
         TX = std::max(1, std::min(16, TX));
         dim3 gy((gt.KX + TX - 1) / TX, w.nz, 3);
