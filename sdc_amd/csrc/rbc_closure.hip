@@ -36,8 +36,7 @@ constexpr int OFF_B2 = OFF_W2 + NH * NH;    // [NH]
 constexpr int OFF_W3 = OFF_B2 + NH;         // [NOUT][NH]
 constexpr int OFF_B3 = OFF_W3 + NOUT * NH;  // [NOUT]
 constexpr int NW = OFF_B3 + NOUT;           // 4931 parameters
-constexpr int kTrainBlocks = 256;  // partial gradients of a batch, at most
-constexpr int kTrainWaves = 8;     // waves per block
+constexpr int kTrainParts = 512;  // partial gradients of a batch, at most: one block each
 
 struct Norm {
     float in_mean[NIN], in_inv[NIN];  // x_n = (x - mean) * inv
@@ -559,315 +558,303 @@ int infer_blocks(int npts) {
 }
 
 // Training: gradient of the mean squared error (normalised targets, mean over points and outputs)
-// over `batch` points, on the matrix cores.  A wave takes 32 points at a time (columns of the
-// 32x32 tiles) and runs the three 64 x 64 products of the two hidden layers with
-// v_mfma_f32_32x32x2_f32: H2 = W2 H1, D1 = W2^T D2, G2 += D2 H1^T -- FP32 operands and sums, as a
-// scalar loop would have.  In the accumulator layout a lane holds one point and 32 hidden units
-// (rows 8 (r / 4) + 4 h + r % 4 of tile t, h = lane / 32); used in register order as a B operand that
-// is the K order the W2 fragments are stored in (w2f, w2t), so activations go from layer to layer
-// without leaving the registers.  The sums over points (G2, and G1, G3, the biases on the VALU)
-// need units across lanes: each factor is transposed once through the wave's LDS tile.
+// over `batch` points, on the matrix cores.  Block bp sums the batch points [bp per, (bp + 1) per) in
+// order, 32 at a time: four waves, each with 16 of the 64 hidden units (rows) and all 32 points
+// (columns, two tiles) of the products A2 = W2 H1, D1 = W2^T D2 and G2 += D2 H1^T, as
+// v_mfma_f32_16x16x4_f32.  That instruction is the FMA chain c + a0 b0 + .. + a3 b3, each step
+// rounded, and every sum here runs over the same terms in the same order, FMA for FMA, as a
+// scalar loop over units and points would.  A wave keeps its rows of W1, W2 and W2^T as A operands in
+// registers; the activations are exchanged through LDS tiles [unit][point], from which the sums over
+// points on the VALU (G1, G3 and the biases, one unit per lane, split over the waves) read too.
 //
-// Bound: 200 MFMAs of 64 cycles per 32 points, 12 us for 65,536 points on 1,024 SIMDs at two waves
-// each (LDS: 33 KiB of weight fragments and 9 KiB per wave).  One block of 8 waves per CU: the
-// gradients of its waves are added in LDS in a fixed order, so 256 partials leave the chip
-// instead of one per wave.  Groups go to blocks first, then to waves, so that small batches still
-// spread over the CUs.  65,536 points: 35 us (a scalar form, one point per wave at a time and 512
-// one-wave blocks, took 307 us).
-constexpr int kTP = 36;                      // row stride of the transposing tile (32 points + pad)
-constexpr int kTrainThreads = 64 * kTrainWaves;
-constexpr int NGV = 64 + 2 * NIN + 4 + 2 * NOUT + NOUT;  // gradient values per lane in the block's reduction
-// fragments (2 x 16 KiB) and the waves' tiles; the reduction reuses the same memory
-constexpr size_t kTrainLds =
-    std::max<size_t>((size_t)2 * NH * NH + (size_t)kTrainWaves * NH * kTP, (size_t)(kTrainWaves / 2) * NGV * 64) *
-    sizeof(float);
+// Bound: 100 MFMAs of 32 cycles per wave and 32 points, with LDS reads of the B operands (one per MFMA)
+// and six LDS barriers between; 512 blocks, two or more a CU, run past each other's barriers.  65,536
+// points: 41 us (a scalar form, one point per wave at a time and 512 one-wave blocks, took 307 us).
+constexpr int kTP = 36;  // tile row stride: 32 points and a pad that spreads rows and columns over the banks
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(kTrainThreads) k_mlp_train(int count, int batch, int random, uint64_t seed,
-                                                             uint64_t step, const uint16_t* __restrict__ wbf, Norm nm,
-                                                             const float* __restrict__ X, const float* __restrict__ Y,
-                                                             float* __restrict__ gpart, double* __restrict__ lpart) {
-    extern __shared__ float smem[];
-    __shared__ float b1s[NH], b2s[NH], w3s[NOUT * NH], b3s[NOUT];
-    __shared__ float w1s[NH * NIN];
-    __shared__ float xs[kTrainWaves][32][NIN + 4];  // a group's inputs and dy[0..2]
-    __shared__ double lsum[kTrainWaves];
+__device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// the value of another lane of the quad (DPP quad_perm)
+template <int CTRL>
+__device__ __forceinline__ float quad_swap(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_mlp_train(int count, int batch, int per, int random, uint64_t seed,
+                                                   uint64_t step, const uint16_t* __restrict__ wbf, Norm nm,
+                                                   const float* __restrict__ X, const float* __restrict__ Y,
+                                                   float* __restrict__ gpart, double* __restrict__ lpart) {
+#pragma clang fp contract(off)
+    __shared__ float H1[NH * kTP], H2[NH * kTP], D2[NH * kTP], S1[NH * kTP];  // S1 = W2^T D2
+    __shared__ uint32_t wl[(NW + 1) / 2];  // the BF16 weights, for the operand gathers below
+    // by point: a group's inputs, two groups in turn; targets; twice the errors; dy for the units < 32
+    // and for the others
+    __shared__ float xs[2][NIN * kTP], ts[2][NOUT][32], e2[NOUT][32], dys[2][NOUT][32];
+    __shared__ double lsum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int c = lane & 31, h = lane >> 5;
-    float* w2f = smem;                // [tile row][tile col][r / 4][lane][r % 4]: W2[32 t2 + c][unit(t, r, h)]
-    float* w2t = smem + NH * NH;      // same with W2 transposed
-    float* tile = smem + 2 * NH * NH + wave * NH * kTP;  // [unit][point]
-    for (int i = tid; i < NH * NH; i += kTrainThreads) {
-        const int r4 = i & 3, l = (i >> 2) & 63, rq = (i >> 8) & 3, t = (i >> 10) & 1, t2 = i >> 11;
-        const int row = 32 * t2 + (l & 31), unit = 32 * t + 8 * rq + 4 * (l >> 5) + r4;
-        w2f[i] = bf16_bits_to_f32(wbf[OFF_W2 + row * NH + unit]);
-        w2t[i] = bf16_bits_to_f32(wbf[OFF_W2 + unit * NH + row]);
-    }
-    for (int i = tid; i < NH * NIN; i += kTrainThreads) w1s[i] = bf16_bits_to_f32(wbf[OFF_W1 + i]);
-    for (int i = tid; i < NOUT * NH; i += kTrainThreads) w3s[i] = bf16_bits_to_f32(wbf[OFF_W3 + i]);
-    if (tid < NH) {
-        b1s[tid] = bf16_bits_to_f32(wbf[OFF_B1 + tid]);
-        b2s[tid] = bf16_bits_to_f32(wbf[OFF_B2 + tid]);
-    }
-    if (tid < NOUT) b3s[tid] = bf16_bits_to_f32(wbf[OFF_B3 + tid]);
-    __syncthreads();
-    const float inv_outs = 1.0f / ((float)batch * NOUT);
-    const int ngroups = (batch + 31) / 32;
-    f32x16 g2[2][2] = {};
-    float g1[2][NIN] = {}, gb1[2] = {}, gb2[2] = {}, g3[2][NOUT] = {}, gb3[NOUT] = {};
-    double loss = 0.0;
-    // rows of the accumulator layout into the [unit][point] tile; points 16 h + 4 q .. + 3 of unit
-    // 32 t + c from it
-    auto put = [&](const f32x16 (&d)[2]) {
-        wave_sync();
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) tile[(32 * t + 8 * (r >> 2) + 4 * h + (r & 3)) * kTP + c] = d[t][r];
-        wave_sync();
-    };
-    auto points = [&](int t, int q) { return *(const f32x4*)(tile + (32 * t + c) * kTP + 16 * h + 4 * q); };
-    for (int gi = wave * gridDim.x + blockIdx.x; gi < ngroups; gi += kTrainWaves * gridDim.x) {  // wave-uniform
-        const int bi = gi * 32 + c;
-        const bool valid = bi < batch;
-        size_t idx = valid ? (size_t)bi : 0;
+    const int c = lane & 15, kq = lane >> 4;  // column of a tile; k of a step, and row group 4 kq + r
+    const int row0 = 16 * wave;               // the wave's units
+    const int pt = tid >> 3, j = tid & 7;
+    const int p0 = blockIdx.x * per, p1 = min(batch, p0 + per);
+    // the thread's input j of point pt (and target j < 3); past the range: point 0 or a drawn one, dropped
+    float xr, yr;
+    auto fetch = [&](int g0) {
+        const int bi = g0 + pt;
+        size_t idx = bi < p1 ? (size_t)bi : 0;
         if (random)
             idx = (size_t)(mix64(seed * 0x100000001B3ull + step * 0x9E3779B1ull + (uint64_t)bi) % (uint64_t)count);
-        // every lane loads (row 0 or a drawn row where the batch has ended) and drops it if not valid
-        const f32x4 xr = *(const f32x4*)(X + idx * NIN + 4 * h);
-        float yr[NOUT];
+        xr = X[idx * NIN + j];
+        yr = Y[idx * NOUT + (j < NOUT ? j : 0)];
+    };
+    fetch(p0);
+    for (int i = tid; i < (NW + 1) / 2; i += 256) wl[i] = reinterpret_cast<const uint32_t*>(wbf)[i];
+    __syncthreads();
+    auto wb = [&](int i) { return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(wl)[i]); };
+    float aW1[2], aW2[16], aW2t[16], b1r[4], b2r[4], w3r[NOUT][4], b3[NOUT];
 #pragma unroll
-        for (int o = 0; o < NOUT; ++o) yr[o] = Y[idx * NOUT + o];
-        float xv[4];
+    for (int s = 0; s < 2; ++s) aW1[s] = wb(OFF_W1 + (row0 + c) * NIN + 4 * s + kq);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float z = (xr[e] - nm.in_mean[4 * h + e]) * nm.in_inv[4 * h + e];
-            xv[e] = valid ? z : 0.f;
-            xs[wave][c][4 * h + e] = xv[e];
+    for (int s = 0; s < 16; ++s) {
+        aW2[s] = wb(OFF_W2 + (row0 + c) * NH + 4 * s + kq);
+        aW2t[s] = wb(OFF_W2 + (4 * s + kq) * NH + row0 + c);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        b1r[r] = wb(OFF_B1 + row0 + 4 * kq + r);
+        b2r[r] = wb(OFF_B2 + row0 + 4 * kq + r);
+#pragma unroll
+        for (int o = 0; o < NOUT; ++o) w3r[o][r] = wb(OFF_W3 + o * NH + row0 + 4 * kq + r);
+    }
+    // the output sums: thread (point tid / 8, sum k01, j4) takes the unit pairs (u, u + 32), u = j4 + 4 m
+    const int k01 = (tid >> 2) & 1, j4 = tid & 3;
+    float w3a[NOUT][8], w3b[NOUT][8], w3u[NOUT];  // of the fused member of a pair, of the other
+#pragma unroll
+    for (int o = 0; o < NOUT; ++o) {
+        b3[o] = wb(OFF_B3 + o);
+        w3u[o] = wb(OFF_W3 + o * NH + lane);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            w3a[o][m] = wb(OFF_W3 + o * NH + 32 * k01 + j4 + 4 * m);
+            w3b[o][m] = wb(OFF_W3 + o * NH + 32 * (1 - k01) + j4 + 4 * m);
         }
-        f32x16 h1[2], h2[2];
+    }
+    const float inv_outs = 1.0f / ((float)batch * NOUT);
+    f32x4 g2[4] = {};
+    float g1[2] = {}, gb1 = 0.f, gb2 = 0.f, g3 = 0.f, gb3 = 0.f;
+    double loss = 0.0;
+    float mean = 0.f, inv = 0.f, scale = 1.f;  // of the thread's input and target
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            f32x16 a = {};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                a = __builtin_amdgcn_mfma_f32_32x32x2f32(w1s[(32 * t + c) * NIN + 4 * h + e], xv[e], a, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) h1[t][r] = tanh_fast(a[r] + b1s[32 * t + 8 * (r >> 2) + 4 * h + (r & 3)]);
+    for (int i = 0; i < NIN; ++i)
+        if (j == i) {
+            mean = nm.in_mean[i];
+            inv = nm.in_inv[i];
+            if (i < NOUT) scale = nm.out_scale[i < NOUT ? i : 0];
         }
-        // 64 x 64 times 64 x 32: fragments from LDS, four K steps a read
-        auto product = [&](const float* frag, const f32x16 (&b)[2], f32x16 (&out)[2]) {
-            out[0] = out[1] = f32x16{};
+    auto rows = [&](float* tile, const f32x4 (&d)[2]) {  // accumulators -> [unit][point]
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+        for (int n = 0; n < 2; ++n)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const f32x4 a0 = *(const f32x4*)(frag + ((t * 4 + q) * 64 + lane) * 4);
-                    const f32x4 a1 = *(const f32x4*)(frag + ((8 + t * 4 + q) * 64 + lane) * 4);
+            for (int r = 0; r < 4; ++r) tile[(row0 + 4 * kq + r) * kTP + 16 * n + c] = d[n][r];
+    };
+    auto product = [&](const float (&a)[16], const float* tile, f32x4 (&d)[2]) {  // d += A tile
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        out[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], b[t][4 * q + e], out[0], 0, 0, 0);
-                        out[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], b[t][4 * q + e], out[1], 0, 0, 0);
-                    }
-                }
-        };
-        asm volatile("" ::: "memory");  // the tables are read where they are used, not held in registers
-        product(w2f, h1, h2);
-        asm volatile("" ::: "memory");
-        float y[NOUT] = {};
+        for (int s = 0; s < 16; ++s)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+            for (int n = 0; n < 2; ++n) d[n] = mfma16(a[s], tile[(4 * s + kq) * kTP + 16 * n + c], d[n]);
+    };
+    int slot = 0;
+    for (int g0 = p0; g0 < p1; g0 += 32, slot ^= 1) {
+        {
+            const float z = (xr - mean) * inv;
+            xs[slot][j * kTP + pt] = g0 + pt < p1 ? z : 0.f;
+            if (j < NOUT) ts[slot][j][pt] = yr / scale;
+        }
+        if (g0 + 32 < p1) fetch(g0 + 32);
+        lds_barrier();
+        f32x4 h1[2], h2[2], d[2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int unit = 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-                h2[t][r] = tanh_fast(h2[t][r] + b2s[unit]);
+        for (int n = 0; n < 2; ++n) {
 #pragma unroll
-                for (int o = 0; o < NOUT; ++o) y[o] += w3s[o * NH + unit] * h2[t][r];
+            for (int r = 0; r < 4; ++r) h1[n][r] = b1r[r];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) h1[n] = mfma16(aW1[s], xs[slot][(4 * s + kq) * kTP + 16 * n + c], h1[n]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h1[n][r] = tanh_fast(h1[n][r]);
+        }
+        rows(H1, h1);
+        lds_barrier();
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h2[n][r] = b2r[r];
+        product(aW2, H1, h2);
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h2[n][r] = tanh_fast(h2[n][r]);
+        rows(H2, h2);
+        lds_barrier();
+        {
+            // y_o = sum_u w3[o][u] h2[u]: units u and u + 32 first (one of the two products fused into
+            // the add: the lower one in sum 0, the upper one in sum 1), then 16, 8, 4, 2, 1 apart.  The
+            // units below 32 take their dy from sum 0, the others from sum 1; the loss is sum 0's.
+            float ha[8], hb[8];
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                ha[m] = H2[(32 * k01 + j4 + 4 * m) * kTP + pt];
+                hb[m] = H2[(32 * (1 - k01) + j4 + 4 * m) * kTP + pt];
             }
-        float dy[NOUT];
+            float dy[NOUT], er2[NOUT];
 #pragma unroll
-        for (int o = 0; o < NOUT; ++o) {
-            y[o] += __shfl_xor(y[o], 32);
-            const float err = y[o] + b3s[o] - yr[o] / nm.out_scale[o], e = valid ? err : 0.f;
-            dy[o] = 2.f * e * inv_outs;
-            loss += (double)e * e;  // both lane halves: halved where it is written
-            gb3[o] += dy[o];
-            xs[wave][c][NIN + o] = dy[o];
-        }
-        asm volatile("" ::: "memory");
-        f32x16 d[2];
+            for (int o = 0; o < NOUT; ++o) {
+                float v[8];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+                for (int m = 0; m < 8; ++m) v[m] = __builtin_fmaf(ha[m], w3a[o][m], hb[m] * w3b[o][m]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int unit = 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
-                float s = 0.f;
+                for (int x = 4; x > 0; x >>= 1)
 #pragma unroll
-                for (int o = 0; o < NOUT; ++o) s += w3s[o * NH + unit] * dy[o];
-                d[t][r] = s * (1.f - h2[t][r] * h2[t][r]);
+                    for (int m = 0; m < x; ++m) v[m] = v[m] + v[m + x];
+                float y = v[0];
+                y = y + quad_swap<0x4E>(y);  // 2 lanes apart
+                y = y + quad_swap<0xB1>(y);  // 1
+                const float d0 = (y + b3[o]) - ts[slot][o][pt], er = g0 + pt < p1 ? d0 : 0.f;
+                loss += (double)er * er;  // every thread of the point: one counts below
+                er2[o] = 2.f * er;
+                dy[o] = er2[o] * inv_outs;
             }
-        put(h2);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 u0 = points(0, q), u1 = points(1, q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
+            if (j4 == 0) {
 #pragma unroll
                 for (int o = 0; o < NOUT; ++o) {
-                    const float v = xs[wave][16 * h + 4 * q + e][NIN + o];
-                    g3[0][o] += v * u0[e];
-                    g3[1][o] += v * u1[e];
-                }
-        }
-        put(d);
-        f32x4 dt[2][4];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) dt[t][q] = points(t, q);
-        put(h1);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 u0 = points(0, q), u1 = points(1, q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int t2 = 0; t2 < 2; ++t2) {
-                    g2[t2][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(dt[t2][q][e], u0[e], g2[t2][0], 0, 0, 0);
-                    g2[t2][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(dt[t2][q][e], u1[e], g2[t2][1], 0, 0, 0);
-                    gb2[t2] += dt[t2][q][e];
-                }
-        }
-        asm volatile("" ::: "memory");
-        product(w2t, d, h2);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) d[t][r] = h2[t][r] * (1.f - h1[t][r] * h1[t][r]);
-        put(d);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 u0 = points(0, q), u1 = points(1, q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                gb1[0] += u0[e];
-                gb1[1] += u1[e];
-#pragma unroll
-                for (int i = 0; i < NIN; ++i) {
-                    const float v = xs[wave][16 * h + 4 * q + e][i];
-                    g1[0][i] += v * u0[e];
-                    g1[1][i] += v * u1[e];
+                    dys[k01][o][pt] = dy[o];
+                    if (k01 == 0) e2[o][pt] = er2[o];
                 }
             }
         }
-        wave_sync();  // xs is rewritten by the next group
-    }
-    // the waves' gradients, added pairwise in a fixed order (upper half to lower half)
-    float v[NGV];
-    {
-        int n = 0;
+        lds_barrier();
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2)
+        for (int n = 0; n < 2; ++n) {
+            float dy[NOUT];
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+            for (int o = 0; o < NOUT; ++o) dy[o] = dys[wave >> 1][o][16 * n + c];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) v[n++] = g2[t2][t][r];
+            for (int r = 0; r < 4; ++r) {
+                float s = 0.f;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int i = 0; i < NIN; ++i) v[n++] = g1[t][i];
-            v[n++] = gb1[t];
-            v[n++] = gb2[t];
-#pragma unroll
-            for (int o = 0; o < NOUT; ++o) v[n++] = g3[t][o];
+                for (int o = 0; o < NOUT; ++o) s = __builtin_fmaf(w3r[o][r], dy[o], s);
+                d[n][r] = __builtin_fmaf(-h2[n][r], h2[n][r], 1.f) * s;
+            }
         }
+        rows(D2, d);
+        // sums over points of the output layer, unit = lane: wave o < 3 has g3[o] and gb3[o], wave 3 gb2
+        auto four = [](const float* q) { return *(const f32x4*)q; };
+        if (wave < NOUT) {
 #pragma unroll
-        for (int o = 0; o < NOUT; ++o) v[n++] = gb3[o];
+            for (int q = 0; q < 8; ++q) {
+                const f32x4 u = four(H2 + lane * kTP + 4 * q), dy = four(&dys[lane >> 5][wave][4 * q]);
+                const f32x4 ee = four(&e2[wave][4 * q]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    g3 = __builtin_fmaf(u[e], dy[e], g3);
+                    gb3 = __builtin_fmaf(inv_outs, ee[e], gb3);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const f32x4 u = four(H2 + lane * kTP + 4 * q);
+                f32x4 v = {};
+#pragma unroll
+                for (int o = 0; o < NOUT; ++o) {
+                    const f32x4 dy = four(&dys[lane >> 5][o][4 * q]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(w3u[o], dy[e], v[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) gb2 = __builtin_fmaf(__builtin_fmaf(-u[e], u[e], 1.f), v[e], gb2);
+            }
+        }
+        lds_barrier();
+        d[0] = d[1] = f32x4{};
+        product(aW2t, D2, d);
+        rows(S1, d);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {  // points 4 s + kq
+            const float a = D2[(row0 + c) * kTP + 4 * s + kq];
+#pragma unroll
+            for (int n = 0; n < 4; ++n) g2[n] = mfma16(a, H1[(16 * n + c) * kTP + 4 * s + kq], g2[n]);
+        }
+        lds_barrier();
+        // sums over points of the input layer, unit = lane: wave w has inputs 2 w and 2 w + 1, wave 0 gb1
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const f32x4 u = four(H1 + lane * kTP + 4 * q), v = four(S1 + lane * kTP + 4 * q);
+            const f32x4 x0 = four(&xs[slot][2 * wave * kTP + 4 * q]), x1 = four(&xs[slot][(2 * wave + 1) * kTP + 4 * q]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float f = __builtin_fmaf(-u[e], u[e], 1.f), d1 = f * v[e];
+                gb1 = __builtin_fmaf(f, v[e], gb1);  // wave 0's is written
+                g1[0] = __builtin_fmaf(d1, x0[e], g1[0]);
+                g1[1] = __builtin_fmaf(d1, x1[e], g1[1]);
+            }
+        }
     }
+    float* gp = gpart + (size_t)blockIdx.x * NW;
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) gp[OFF_W2 + (row0 + 4 * kq + r) * NH + 16 * n + c] = g2[n][r];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) gp[OFF_W1 + lane * NIN + 2 * wave + i] = g1[i];
+    if (wave < NOUT) {
+        gp[OFF_W3 + wave * NH + lane] = g3;
+        if (lane == 0) gp[OFF_B3 + wave] = gb3;
+    } else {
+        gp[OFF_B2 + lane] = gb2;
+    }
+    if (wave == 0) gp[OFF_B1 + lane] = gb1;
+    if (j != 0) loss = 0.0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
     if (lane == 0) lsum[wave] = loss;
-#pragma unroll
-    for (int half = kTrainWaves / 2; half > 0; half >>= 1) {
-        __syncthreads();
-        if (wave >= half && wave < 2 * half) {
-#pragma unroll
-            for (int n = 0; n < NGV; ++n) smem[((wave - half) * NGV + n) * 64 + lane] = v[n];
-        }
-        __syncthreads();
-        if (wave < half) {
-#pragma unroll
-            for (int n = 0; n < NGV; ++n) v[n] += smem[(wave * NGV + n) * 64 + lane];
-        }
-    }
-    if (wave != 0) return;
-    float* gp = gpart + (size_t)blockIdx.x * NW;
-    int n = 0;
-#pragma unroll
-    for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r)
-                gp[OFF_W2 + (32 * t2 + 8 * (r >> 2) + 4 * h + (r & 3)) * NH + 32 * t + c] = v[n++];
-    // per-unit values: the two lane halves hold sums over different points
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int i = 0; i < NIN + 2 + NOUT; ++i, ++n) {
-            const float s = v[n] + __shfl_xor(v[n], 32);
-            const int unit = 32 * t + c;
-            const int at = i < NIN ? OFF_W1 + unit * NIN + i
-                                   : (i == NIN ? OFF_B1 + unit
-                                               : (i == NIN + 1 ? OFF_B2 + unit : OFF_W3 + (i - NIN - 2) * NH + unit));
-            if (h == 0) gp[at] = s;
-        }
-    }
-#pragma unroll
-    for (int o = 0; o < NOUT; ++o, ++n) {
-        float s = v[n];
-        for (int k = 16; k > 0; k >>= 1) s += __shfl_xor(s, k);
-        if (lane == 0) gp[OFF_B3 + o] = s;
-    }
-    if (lane == 0) {
-        double s = 0.0;
-        for (int w = 0; w < kTrainWaves; ++w) s += lsum[w];
-        lpart[blockIdx.x] = 0.5 * s / ((double)batch * NOUT);
-    }
+    __syncthreads();
+    if (tid == 0) lpart[blockIdx.x] = (lsum[0] + lsum[1] + lsum[2] + lsum[3]) / ((double)batch * NOUT);
 }
 
-// The batch gradient: FP64 sum of the blocks' partials in a fixed order (32 parameters a block, 8
-// threads each take every 8th partial), the batch loss into lossbuf[slot], and, with ADAM, the Adam
+// The batch gradient: FP64 sum of the blocks' partials in a fixed order (32 parameters a block, 16
+// threads each take every 16th partial), the batch loss into lossbuf[slot], and, with ADAM, the Adam
 // update (Kingma & Ba 2015) of the FP32 master weights and their BF16 copies in the same launch.
-// Bound: 5 MB of partials; 155 blocks with 8 partial rows in flight each (5.5 us; one thread per
+// Bound: 10 MB of partials; 155 blocks with 16 partial rows in flight each (6.5 us; one thread per
 // parameter over 512 partials, 20 blocks, took 137 us and Adam a launch of 5 us more).
 struct AdamStep {
     float lr, beta1, beta2, eps, c1, c2;
 };
 template <bool ADAM>
-__global__ void __launch_bounds__(256) k_grad_finish(int nblk, const float* __restrict__ gpart,
+__global__ void __launch_bounds__(512) k_grad_finish(int npart, const float* __restrict__ gpart,
                                                      const double* __restrict__ lpart, float* __restrict__ grad,
                                                      double* __restrict__ lossbuf, int slot, AdamStep ad,
                                                      float* __restrict__ wm, float* __restrict__ m1,
                                                      float* __restrict__ m2, uint16_t* __restrict__ wbf) {
-    __shared__ double part[8][32];
+    __shared__ double part[16][32];
     const int c = threadIdx.x & 31, row = threadIdx.x >> 5, i = blockIdx.x * 32 + c;
     double s = 0.0;
     if (i < NW) {
 #pragma unroll 8
-        for (int b = row; b < nblk; b += 8) s += gpart[(size_t)b * NW + i];
+        for (int b = row; b < npart; b += 16) s += gpart[(size_t)b * NW + i];
     }
     part[row][c] = s;
     __syncthreads();
-    if (blockIdx.x == 0 && threadIdx.x >= 192) {  // the last wave: the loss
+    if (blockIdx.x == 0 && threadIdx.x >= 448) {  // the last wave: the loss
         double l = 0.0;
-        for (int b = threadIdx.x - 192; b < nblk; b += 64) l += lpart[b];
+        for (int b = threadIdx.x - 448; b < npart; b += 64) l += lpart[b];
         for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-        if (threadIdx.x == 192) lossbuf[slot] = l;
+        if (threadIdx.x == 448) lossbuf[slot] = l;
     }
     if (row != 0 || i >= NW) return;
-    for (int r = 1; r < 8; ++r) s += part[r][c];
+    for (int r = 1; r < 16; ++r) s += part[r][c];
     const float gr = (float)s;
     grad[i] = gr;
     if (ADAM) {
@@ -884,10 +871,10 @@ __global__ void __launch_bounds__(256) k_grad_finish(int nblk, const float* __re
 // gradient partials of `batch` points of (X, Y); returns the number of partials
 int launch_train(hipStream_t s, int count, int batch, int random, uint64_t seed, uint64_t step, const uint16_t* wbf,
                  const Norm& nm, const float* X, const float* Y, float* gpart, double* lpart) {
-    const int nblk = std::min(kTrainBlocks, (batch + 31) / 32);
-    hipLaunchKernelGGL(k_mlp_train, dim3(nblk), dim3(kTrainThreads), kTrainLds, s, count, batch, random, seed, step,
+    const int per = (batch + kTrainParts - 1) / kTrainParts, np = (batch + per - 1) / per;
+    hipLaunchKernelGGL(k_mlp_train, dim3(np), dim3(256), 0, s, count, batch, per, random, seed, step,
                        wbf, nm, X, Y, gpart, lpart);
-    return nblk;
+    return np;
 }
 
 // per-column sums and sums of squares (FP64) of a row-major [n][nc] array, per block
@@ -959,8 +946,8 @@ struct rbc_closure {
     float* grad = nullptr;
     float* m1 = nullptr;
     float* m2 = nullptr;
-    float* gpart = nullptr;           // [kTrainBlocks][NW]
-    double* lpart = nullptr;          // [kTrainBlocks]
+    float* gpart = nullptr;           // [kTrainParts][NW]
+    double* lpart = nullptr;          // [kTrainParts]
     double* lossbuf = nullptr;        // [lossbuf_n]
     int lossbuf_n = 0;
     int adam_t = 0;
@@ -1308,12 +1295,12 @@ int rbc_closure_create(rbc_ctx* c, int nz, int capacity_points, rbc_closure** ou
         cl->DX = (float*)cl->al((size_t)capacity_points * NIN * sizeof(float));
         cl->DY = (float*)cl->al((size_t)capacity_points * NOUT * sizeof(float));
         cl->wm = (float*)cl->al(NW * sizeof(float));
-        cl->wbf = (uint16_t*)cl->al(NW * sizeof(uint16_t));
+        cl->wbf = (uint16_t*)cl->al((NW + 1) * sizeof(uint16_t));  // read in pairs
         cl->grad = (float*)cl->al(NW * sizeof(float));
         cl->m1 = (float*)cl->al(NW * sizeof(float));
         cl->m2 = (float*)cl->al(NW * sizeof(float));
-        cl->gpart = (float*)cl->al((size_t)kTrainBlocks * NW * sizeof(float));
-        cl->lpart = (double*)cl->al(kTrainBlocks * sizeof(double));
+        cl->gpart = (float*)cl->al((size_t)kTrainParts * NW * sizeof(float));
+        cl->lpart = (double*)cl->al(kTrainParts * sizeof(double));
         for (int i = 0; i < 11; ++i) cl->snap.push_back(cl->al(snap_bytes(c, i)));
         // Glorot-uniform initial weights from SplitMix64, zero biases
         std::vector<float> w0(NW, 0.f);
@@ -1543,8 +1530,8 @@ int rbc_closure_gradient(rbc_closure* cl, int n, const float* X, const float* Y,
         HIPCHK(hipMalloc(&lb, sizeof(double)));
         HIPCHK(hipMemcpy(dx, X, (size_t)n * NIN * sizeof(float), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(dy, Y, (size_t)n * NOUT * sizeof(float), hipMemcpyHostToDevice));
-        const int nblk = launch_train(c->stream, n, n, 0, 0, 0, cl->wbf, cl->nm, dx, dy, cl->gpart, cl->lpart);
-        hipLaunchKernelGGL(k_grad_finish<false>, dim3((NW + 31) / 32), dim3(256), 0, c->stream, nblk,
+        const int np = launch_train(c->stream, n, n, 0, 0, 0, cl->wbf, cl->nm, dx, dy, cl->gpart, cl->lpart);
+        hipLaunchKernelGGL(k_grad_finish<false>, dim3((NW + 31) / 32), dim3(512), 0, c->stream, np,
                            (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, lb, 0, AdamStep{}, nullptr,
                            nullptr, nullptr, nullptr);
         HIPCHK(hipGetLastError());
@@ -1577,12 +1564,12 @@ int rbc_closure_train(rbc_closure* cl, int steps, int batch, double lr, unsigned
         const float* X = cl->DX + (size_t)first * NIN;
         const float* Y = cl->DY + (size_t)first * NOUT;
         for (int s = 0; s < steps; ++s) {
-            const int nblk = launch_train(c->stream, n, batch, 1, seed, (uint64_t)(cl->adam_t + 1), cl->wbf, cl->nm, X,
+            const int np = launch_train(c->stream, n, batch, 1, seed, (uint64_t)(cl->adam_t + 1), cl->wbf, cl->nm, X,
                                           Y, cl->gpart, cl->lpart);
             cl->adam_t++;
             const float b1 = 0.9f, b2 = 0.999f;
             const float c1 = 1.f - std::pow(b1, (float)cl->adam_t), c2 = 1.f - std::pow(b2, (float)cl->adam_t);
-            hipLaunchKernelGGL(k_grad_finish<true>, dim3((NW + 31) / 32), dim3(256), 0, c->stream, nblk,
+            hipLaunchKernelGGL(k_grad_finish<true>, dim3((NW + 31) / 32), dim3(512), 0, c->stream, np,
                                (const float*)cl->gpart, (const double*)cl->lpart, cl->grad, cl->lossbuf, s,
                                AdamStep{(float)lr, b1, b2, 1e-8f, c1, c2}, cl->wm, cl->m1, cl->m2, cl->wbf);
         }
