@@ -227,6 +227,7 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
         d.KXp = (p->M == 512 && p->N == 512) ? (g.KX + 7) & ~7 : (g.KX + 3) & ~3;
         d.NYc = NYc;
         d.P = g.P();
+        d.PS = (d.P + 15) & ~15;
         d.logM = 0;
         while ((1 << d.logM) < p->M) ++d.logM;
         d.logN = 0;
@@ -261,10 +262,10 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
         b.XoG = c->dalloc(L * cs);
         b.OoF = c->dalloc(L * cs);
         b.OoG = c->dalloc(L * cs);
-        b.lev = c->dalloc((size_t)6 * nq * P * cs);
+        b.lev = c->dalloc((size_t)6 * nq * d.PS * cs);
         b.hin = c->dalloc((size_t)6 * nq * d.N * d.KXp * cs);
         b.hout = c->dalloc((size_t)7 * nq * d.N * d.KXp * cs);
-        b.prod = c->dalloc((size_t)7 * nq * P * cs);
+        b.prod = c->dalloc((size_t)7 * nq * d.PS * cs);
         b.fgw = c->dalloc((size_t)2 * nq * cs);
         b.refstage = c->dalloc((size_t)(d.M / 2 + 1) * d.N * L * 16);
         // zero-initialise state and padding once (not in any step: nothing is memset later)
@@ -301,21 +302,26 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
         b.prtab = c->dalloc(pr.size() * c->rsz);
         upload_reals(c.get(), b.evtab, ev);
         upload_reals(c.get(), b.prtab, pr);
-        // matrix-core operand tables in fragment order (see k_eval_mma / k_project_mma)
+        // matrix-core operand tables.  RBC_NO_MFMA=1 in the environment keeps the plain VALU sums (the
+        // tests pin the matrix-core forms against them).
+        const char* no = getenv("RBC_NO_MFMA");
+        if (p->precision != RBC_BF16X3 && !(no && no[0] == '1')) {
+            std::vector<double> evP, prP;
+            vertical_tables(p->L, nq, d.PS, c->rsz == 8, ev, pr, evP, prP);
+            b.evP = c->dalloc(evP.size() * c->rsz);
+            b.prP = c->dalloc(prP.size() * c->rsz);
+            upload_reals(c.get(), b.evP, evP);
+            upload_reals(c.get(), b.prP, prP);
+        }
+        // BF16X3: in fragment order (see k_eval_mma / k_project_mma)
         {
-            const char* no = getenv("RBC_NO_MFMA");
-            const bool off = no && no[0] == '1';
-            if (p->precision == RBC_BF16X3) b.mma = 1;
-            else if (p->precision == RBC_F32 && p->L <= 32 && !off) b.mma = 0;
-            // the matrix-core projection addresses one level combination (2 nq P floats) with
-            // 32-bit buffer offsets
-            if (b.mma >= 0 && (double)nq * P * 8.0 >= 2147483648.0) {
-                if (p->precision == RBC_BF16X3)
-                    return fail(nullptr, RBC_ERR_ARG, "BF16X3: grid too large for the 32-bit projection offsets");
-                b.mma = -1;
-            }
-            if (b.mma >= 0) {
-                const int K = b.mma == 0 ? 2 : 16, KPL = K / 2;
+            b.bf16x3 = p->precision == RBC_BF16X3;
+            // the BF16X3 projection addresses one level combination (2 nq P floats) with 32-bit
+            // buffer offsets
+            if (b.bf16x3 && (double)nq * d.PS * 8.0 >= 2147483648.0)
+                return fail(nullptr, RBC_ERR_ARG, "BF16X3: grid too large for the 32-bit projection offsets");
+            if (b.bf16x3) {
+                const int K = 16, KPL = K / 2;
                 b.ev_nlt = (nq + 31) / 32;
                 b.ev_nks = ((int)L + K - 1) / K;
                 b.pr_nks = (nq + K - 1) / K;
@@ -327,11 +333,8 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
                             for (int ln = 0; ln < 64; ++ln)
                                 for (int e = 0; e < KPL; ++e) {
                                     const int l = lt * 32 + (ln & 31), m = s * K + KPL * (ln >> 5) + e;
-                                    // FP32 (KPL = 1): the four tables interleaved, one float4 per (tile,
-                                    // k-step, lane); BF16X3: [table][tile][k-step][lane][KPL]
                                     const size_t at =
-                                        b.mma == 0 ? ((((size_t)lt * b.ev_nks + s) * 64 + ln) * 4 + t)
-                                                   : ((((size_t)t * b.ev_nlt + lt) * b.ev_nks + s) * 64 + ln) * KPL + e;
+                                        ((((size_t)t * b.ev_nlt + lt) * b.ev_nks + s) * 64 + ln) * KPL + e;
                                     if (l < nq && m < (int)L) eA[at] = B(evt[t], m, l);
                                 }
                 std::vector<double> pA((size_t)5 * b.pr_nks * 64 * KPL, 0.0);

@@ -1229,6 +1229,7 @@ int rbc_closure_create(rbc_ctx* c, int nz, int capacity_points, rbc_closure** ou
     cl->cap = capacity_points;
     cl->gz = c->dg;
     cl->gz.nq = nz;
+    cl->gz.PS = c->dg.P;
     try {
         hipSetDevice(c->p.device);
         const DevGeom& g = cl->gz;

@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(256) k_fft_y_inv(DevGeom g, int TX, const cpx<
                                                    cpx<T>* __restrict__ hin) {
     extern __shared__ unsigned char smem_raw[];
     cpx<T>* a = reinterpret_cast<cpx<T>*>(smem_raw);
-    const int N = g.N, NYc = g.NYc, P = g.P, nq = g.nq;
+    const int N = g.N, NYc = g.NYc, nq = g.nq;
     cpx<T>* b = a + (size_t)TX * N;
     const int ftile = blockIdx.x;
     const int l = blockIdx.y, field = blockIdx.z;
@@ -383,7 +383,7 @@ __global__ void __launch_bounds__(256) k_fft_y_inv(DevGeom g, int TX, const cpx<
     const int ncol = min(TX, g.KX - kx0);
     for (int e = threadIdx.x; e < TX * N; e += blockDim.x) a[e] = mk<T>(0, 0);
     __syncthreads();
-    const cpx<T>* src = lev + ((size_t)field * nq + l) * P;
+    const cpx<T>* src = lev + ((size_t)field * nq + l) * g.PS;
     for (int e = threadIdx.x; e < ncol * NYc; e += blockDim.x) {
         const int c = e / NYc, kyc = e - c * NYc;
         a[c * N + rows[kyc]] = src[(size_t)(kx0 + c) * NYc + kyc];
@@ -406,7 +406,7 @@ __global__ void __launch_bounds__(256) k_fft_y_fwd(DevGeom g, int TX, const cpx<
                                                    cpx<T>* __restrict__ prod) {
     extern __shared__ unsigned char smem_raw[];
     cpx<T>* a = reinterpret_cast<cpx<T>*>(smem_raw);
-    const int N = g.N, NYc = g.NYc, P = g.P, nq = g.nq;
+    const int N = g.N, NYc = g.NYc, nq = g.nq;
     cpx<T>* b = a + (size_t)TX * N;
     const int kx0 = blockIdx.x * TX;
     const int l = blockIdx.y, q = blockIdx.z;
@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(256) k_fft_y_fwd(DevGeom g, int TX, const cpx<
     }
     __syncthreads();
     cpx<T>* r = lds_fft(a, b, g.logN, TX, twN, false);
-    cpx<T>* dst = prod + ((size_t)q * nq + l) * P;
+    cpx<T>* dst = prod + ((size_t)q * nq + l) * g.PS;
     for (int e = threadIdx.x; e < ncol * NYc; e += blockDim.x) {
         const int c = e / NYc, kyc = e - c * NYc;
         dst[(size_t)(kx0 + c) * NYc + kyc] = r[c * N + rows[kyc]];
@@ -445,12 +445,12 @@ __device__ __forceinline__ void k_fft_y_inv_w_body(int bz, DevGeom g, const cpx<
     __shared__ cpx<T> tw[N];
     __shared__ cpx<T> tile[(N + N / 8) * S];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
-    const int P = g.P, nq = g.nq, KX = g.KX;
+    const int nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y, field = bz;
     const int c = wave * G + grp, kx = kx0 + c;
     for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
     __syncthreads();
-    const cpx<T>* src = lev + ((size_t)field * nq + l) * P + (size_t)kx * NYc;
+    const cpx<T>* src = lev + ((size_t)field * nq + l) * g.PS + (size_t)kx * NYc;
     cpx<T> v[1][E];
 #pragma unroll
     for (int r = 0; r < E; ++r) {
@@ -502,7 +502,7 @@ __global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_w(DevGeom g, const cpx<T
     __shared__ cpx<T> tw[N];
     __shared__ cpx<T> tile[(N + N / 8) * S];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
-    const int P = g.P, nq = g.nq, KX = g.KX;
+    const int nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y, q = blockIdx.z;
     const int c = wave * G + grp, kx = kx0 + c;
     const int ncol = min(CB, KX - kx0);
@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_w(DevGeom g, const cpx<T
     wave_sync();  // the column is read before it becomes the scratch
     fft_group<LOGN, false, 1, S>(v, tile + c, tw, j);
     if (kx < KX) {
-        cpx<T>* dst = prod + ((size_t)q * nq + l) * P + (size_t)kx * NYc;
+        cpx<T>* dst = prod + ((size_t)q * nq + l) * g.PS + (size_t)kx * NYc;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
             const int n = j + W * r;
@@ -599,6 +599,36 @@ template <typename T>
 inline bool launch_y_fwd_group(const DevGeom& g, int nf, const cpx<T>* hout, const cpx<T>* twN,
                                cpx<T>* prod, hipStream_t s, int cb = 0) {
     return launch_y_group<T>(false, g, nf, hout, twN, prod, s, cb);
+}
+
+// mean flow (nonlinear...cu:920-1003): N_F = -<uw, S'>_{k=0}, N_G = -<vw, S'>_{k=0}, times -1/Pr
+template <typename T>
+__device__ __forceinline__ void mean_flow_projection(const DevGeom& g, const cpx<T>* __restrict__ fgw,
+                                                     const T* __restrict__ prtab, T Pr, cpx<T>* NF, cpx<T>* NG) {
+    // threads 0 .. 63: lane = (level parity, m) for L <= 32 (the two halves of the wave
+    // take alternate levels and are added at the end), lane = m for L <= 64
+    const int L = g.L, nq = g.nq;
+    if (threadIdx.x >= 64) return;
+    const int G = L <= 32 ? 2 : 1, m = threadIdx.x % (64 / G), par = threadIdx.x / (64 / G);
+    cpx<T> sF = mk<T>(0, 0), sG = sF;
+    if (m < L) {
+#pragma unroll 4
+        for (int l = par; l < nq; l += G) {
+            const T sp = prtab[(size_t)l * 5 * L + 4 * L + m];
+            sF = sF + cscale(fgw[2 * l], sp);
+            sG = sG + cscale(fgw[2 * l + 1], sp);
+        }
+    }
+    if (G == 2) {
+        sF.x += __shfl_xor(sF.x, 32);
+        sF.y += __shfl_xor(sF.y, 32);
+        sG.x += __shfl_xor(sG.x, 32);
+        sG.y += __shfl_xor(sG.y, 32);
+    }
+    if (par == 0 && m < L) {
+        NF[m] = cscale(sF, T(1) / Pr);
+        NG[m] = cscale(sG, T(1) / Pr);
+    }
 }
 
 }  // namespace rbc

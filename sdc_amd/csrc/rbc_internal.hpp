@@ -68,6 +68,8 @@ int build_factors(const Geometry& g, double Lx, double Ly, double Ra, double Pr,
 // ---------------------------------------------------------------------------------------
 struct DevGeom {
     int M, N, L, nq, KX, KXp, NYc, P;
+    int PS;  // row stride of the level arrays [q][l][p]: P rounded up to 16 in the context's own, so that the 16 modes a
+             // wave writes or reads of a level are whole 128-byte lines; other arrays of this form set their own
     int logM, logN;
     double Lx, Ly;
 };
@@ -91,10 +93,10 @@ struct Buffers {
     void* OoF;
     void* OoG;
     // level space
-    void* lev;    // 6 * nq * P complex  [field][l][p]
+    void* lev;    // 6 * nq * PS complex  [field][l][p] (rows of PS)
     void* hin;    // 6 * nq * N * KXp complex  [field][l][y][kx]
     void* hout;   // 7 * nq * N * KXp complex  [prod][l][y][kx]
-    void* prod;   // 7 * nq * P complex  [prod][l][p] (generic path only)
+    void* prod;   // 7 * nq * PS complex  [prod][l][p] (generic path only)
     // the projection's five level combinations live in `lev` (free once the inverse y-FFT has
     // consumed it): [5][l][p] complex; fgw[l] = (P_uw, P_vw) at k = 0 for the mean flow
     void* fgw;    // nq * 2 complex
@@ -124,11 +126,16 @@ struct Buffers {
     // non-finite value (0 = none), health[1] = steps finished since create (both written by the
     // last block of the end-of-step kernel only)
     int* health;
-    // matrix-core vertical transforms (FP32 storage): -1 = off, 0 = FP32 MFMA, 1 = BF16 x3
-    int mma = -1;
+    // BF16 x3 vertical transforms (RBC_BF16X3)
+    bool bf16x3 = false;
     void* evA = nullptr;  // [4][ev_nlt][ev_nks][64][KPL] floats (C', C, S, S')
     void* prA = nullptr;  // [5][pr_nks][64][KPL] floats (wC', wC'', wC, wS, wS')
     int ev_nlt = 0, ev_nks = 0, pr_nks = 0;
+    // operand tables of the FP64 / FP32 matrix-core transforms (rbc_vertical.hip), in the real type: parity-
+    // folded [4][level tiles][k-steps][64][2] (C', C, S, S') and [32-mode halves][k-steps][5][64][2] (wC', wC'',
+    // wC, wS, wS'); FP32 up to L = 32 [level tiles][k-steps][64][4] and 2 x [level pairs][64][4]
+    void* evP = nullptr;
+    void* prP = nullptr;
     // launch shapes of the generic (non-512) FFT kernels; 0 = built-in choice.  Set by the
     // ensemble autotuner; the arithmetic per element does not depend on them.
     int tune_ytx = 0;           // kx columns per block of the y-FFTs
@@ -170,6 +177,11 @@ enum PlaneOp { PLANE_CAPTURE = 0, PLANE_FREEZE = 1, PLANE_HEAT = 2, PLANE_SCALE 
 // context's real type (rsz = 4 or 8); enqueued on s
 void field_from_ref64(const DevGeom& g, int rsz, const void* ref, void* dst, hipStream_t s);
 void field_to_ref64(const DevGeom& g, int rsz, const void* src, void* ref, hipStream_t s);
+
+// Operand tables of the matrix-core vertical transforms (rbc_vertical.hip) from the level tables ev [l][4][m]
+// and pr [l][5][m].
+void vertical_tables(int L, int nq, int PS, bool f64, const std::vector<double>& ev, const std::vector<double>& pr,
+                   std::vector<double>& evP, std::vector<double>& prP);
 
 template <typename T>
 struct Launch {

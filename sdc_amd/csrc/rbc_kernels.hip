@@ -13,6 +13,7 @@
 
 #include "rbc_ctx.hpp"
 #include "rbc_device.hpp"
+#include "rbc_vertical.hpp"
 
 namespace rbc {
 
@@ -60,7 +61,7 @@ __global__ void __launch_bounds__(256) k_eval(DevGeom g, int LG, int nblk, int p
     if (p >= P) return;
     const T kx = kxa[p], ky = kya[p];
     const T k2 = kx * kx + ky * ky;
-    const size_t plane = (size_t)P;
+    const size_t plane = (size_t)g.PS;
     constexpr int LB = 4;  // levels per pass over the mode data
     for (int l0 = lbeg + wave * LB; l0 < lend; l0 += 4 * LB) {
         cpx<T> Fp[LB], Fc[LB], Gs[LB], Ts[LB], Tz[LB];
@@ -265,10 +266,10 @@ template <typename T>
 __global__ void __launch_bounds__(256) k_combine(DevGeom g, const cpx<T>* __restrict__ prod,
                                                  const T* __restrict__ kxa, const T* __restrict__ kya,
                                                  cpx<T>* __restrict__ D, cpx<T>* __restrict__ fgw) {
-    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t P = g.P, fs = (size_t)g.nq * P;
-    if (e >= fs) return;
-    const size_t p = e % P;
+    const size_t e0 = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t P = g.P, fs = (size_t)g.nq * g.PS;
+    if (e0 >= g.nq * P) return;
+    const size_t l = e0 / P, p = e0 - l * P, e = l * g.PS + p;
     const T kx = kxa[p], ky = kya[p];
     cpx<T> d[5];
 #pragma unroll
@@ -278,102 +279,9 @@ __global__ void __launch_bounds__(256) k_combine(DevGeom g, const cpx<T>* __rest
 #pragma unroll
     for (int t = 0; t < 5; ++t) D[t * fs + e] = d[t];
     if (p == 0) {
-        const size_t l = e / P;
         fgw[2 * l] = prod[3 * fs + e];
         fgw[2 * l + 1] = prod[4 * fs + e];
     }
-}
-
-// mean flow (nonlinear...cu:920-1003): N_F = -<uw, S'>_{k=0}, N_G = -<vw, S'>_{k=0}, times -1/Pr
-template <typename T>
-__device__ __forceinline__ void mean_flow_projection(const DevGeom& g, const cpx<T>* __restrict__ fgw,
-                                                     const T* __restrict__ prtab, T Pr, cpx<T>* NF, cpx<T>* NG) {
-    // first wave of block 0: lane = (level parity, m) for L <= 32 (the two halves of the wave
-    // take alternate levels and are added at the end), lane = m for L <= 64
-    const int L = g.L, nq = g.nq;
-    if (blockIdx.x != 0 || threadIdx.x >= 64) return;
-    const int G = L <= 32 ? 2 : 1, m = threadIdx.x % (64 / G), par = threadIdx.x / (64 / G);
-    cpx<T> sF = mk<T>(0, 0), sG = sF;
-    if (m < L) {
-#pragma unroll 4
-        for (int l = par; l < nq; l += G) {
-            const T sp = prtab[(size_t)l * 5 * L + 4 * L + m];
-            sF = sF + cscale(fgw[2 * l], sp);
-            sG = sG + cscale(fgw[2 * l + 1], sp);
-        }
-    }
-    if (G == 2) {
-        sF.x += __shfl_xor(sF.x, 32);
-        sF.y += __shfl_xor(sF.y, 32);
-        sG.x += __shfl_xor(sG.x, 32);
-        sG.y += __shfl_xor(sG.y, 32);
-    }
-    if (par == 0 && m < L) {
-        NF[m] = cscale(sF, T(1) / Pr);
-        NG[m] = cscale(sG, T(1) / Pr);
-    }
-}
-
-// Variant for L <= 4 * MCH: per round of 4 levels the block stages the combinations of 4 levels
-// of its 64 modes in LDS; every wave then accumulates its own MCH vertical modes.
-template <typename T, int MCH>
-__global__ void __launch_bounds__(256) k_project_lds(DevGeom g, const cpx<T>* __restrict__ D,
-                                                     const cpx<T>* __restrict__ fgw, const T* __restrict__ prtab,
-                                                     const T* __restrict__ kxa, const T* __restrict__ kya, T Pr,
-                                                     cpx<T>* __restrict__ Nt, cpx<T>* __restrict__ Nf,
-                                                     cpx<T>* __restrict__ Ng, cpx<T>* __restrict__ NF,
-                                                     cpx<T>* __restrict__ NG) {
-    constexpr int LV = 4;
-    __shared__ cpx<T> sD[LV][5][64];
-    const int L = g.L, P = g.P, nq = g.nq;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = blockIdx.x * 64 + lane;
-    const bool valid = p < P;
-    const int pc = valid ? p : 0;
-    const T kx = kxa[pc], ky = kya[pc];
-    const T k2 = kx * kx + ky * ky;
-    const size_t fs = (size_t)nq * P;
-    const T mt = T(-1), mp = T(-1) / Pr;
-    const int mb = wave * MCH;
-    cpx<T> af[MCH], ag[MCH], at[MCH];
-#pragma unroll
-    for (int i = 0; i < MCH; ++i) af[i] = ag[i] = at[i] = mk<T>(0, 0);
-    for (int l0 = 0; l0 < nq; l0 += LV) {
-        const int ls = l0 + wave;
-        if (ls < nq) {
-#pragma unroll
-            for (int t = 0; t < 5; ++t) sD[wave][t][lane] = D[t * fs + (size_t)ls * P + pc];
-        }
-        __syncthreads();
-        for (int lv = 0; lv < LV && l0 + lv < nq; ++lv) {
-            const T* tb = prtab + (size_t)(l0 + lv) * 5 * L;  // wC', wC'', wC, wS, wS'
-            const cpx<T> A = sD[lv][0][lane], Bf = sD[lv][1][lane], Ag = sD[lv][2][lane];
-            const cpx<T> Bg = sD[lv][3][lane], At = sD[lv][4][lane];
-#pragma unroll
-            for (int i = 0; i < MCH; ++i) {
-                const int m = mb + i;
-                if (m < L) {
-                    const T cp = tb[m], cpp = tb[L + m], cv = tb[2 * L + m], sv = tb[3 * L + m], sp = tb[4 * L + m];
-                    af[i] = af[i] + cscale(A, cp) + cscale(Bf, cpp + k2 * cv);
-                    ag[i] = ag[i] + cscale(Ag, sv) + cscale(Bg, sp);
-                    at[i] = at[i] + cscale(At, sv);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    if (valid) {
-#pragma unroll
-        for (int i = 0; i < MCH; ++i) {
-            const int m = mb + i;
-            if (m < L) {
-                Nt[(size_t)p * L + m] = cscale(at[i], mt);
-                Nf[(size_t)p * L + m] = cscale(af[i], mp);
-                Ng[(size_t)p * L + m] = cscale(ag[i], mp);
-            }
-        }
-    }
-    mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
 }
 
 // General L: block = 64 modes; wave w accumulates vertical modes m = w*MCH + 4*MCH*i.
@@ -391,14 +299,14 @@ __global__ void __launch_bounds__(256) k_project(DevGeom g, const cpx<T>* __rest
     const int pc = valid ? p : 0;
     const T kx = kxa[pc], ky = kya[pc];
     const T k2 = kx * kx + ky * ky;
-    const size_t fs = (size_t)nq * P;
+    const size_t fs = (size_t)nq * g.PS;
     const T mt = T(-1), mp = T(-1) / Pr;
     for (int mb = wave * MCH; mb < L; mb += 4 * MCH) {
         cpx<T> af[MCH], ag[MCH], at[MCH];
 #pragma unroll
         for (int i = 0; i < MCH; ++i) af[i] = ag[i] = at[i] = mk<T>(0, 0);
         for (int l = 0; l < nq; ++l) {
-            const cpx<T>* src = D + (size_t)l * P + pc;
+            const cpx<T>* src = D + (size_t)l * g.PS + pc;
             const cpx<T> A = src[0], Bf = src[fs], Ag = src[2 * fs], Bg = src[3 * fs], At = src[4 * fs];
             const T* tb = prtab + (size_t)l * 5 * L;
 #pragma unroll
@@ -424,7 +332,7 @@ __global__ void __launch_bounds__(256) k_project(DevGeom g, const cpx<T>* __rest
             }
         }
     }
-    mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
+    if (blockIdx.x == 0) mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1717,7 +1625,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) k
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int NYc = NYC512;
     constexpr int a = (NYc - 1) / 2, shift = 512 - NYc;  // kept rows [0, a] U [512 - a, 511]
-    const int P = g.P, KX = g.KX;
+    const int KX = g.KX;
     for (int e = threadIdx.x; e < TwByPass::size; e += 512) twl[e] = tw[e];  // tw: in TwByPass order
     lds_barrier();
     const int range = (nblk + 7) / 8, xcd = blockIdx.x & 7;
@@ -1725,7 +1633,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) k
     auto load = [&](int lb, cpx<float> (&v)[8]) {
         const int tix = lb % ntile, rest = lb / ntile;
         const int kx = tix * YT + wave;
-        const cpx<float>* src = lev + (size_t)rest * P + (size_t)kx * NYc;  // rest = field * nq + l
+        const cpx<float>* src = lev + (size_t)rest * g.PS + (size_t)kx * NYc;  // rest = field * nq + l
 #pragma unroll
         for (int r = 0; r < 8; ++r) {
             const int n = lane + 64 * r;
@@ -1763,9 +1671,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6))) k
 }
 
 // =======================================================================================
-// Vertical transforms on the matrix cores (FP32 storage).  MM = 0: v_mfma_f32_32x32x2f32
-// (K = 2 per instruction); MM = 1: BF16 hi/lo split, v_mfma_f32_32x32x16_bf16 (K = 16),
-// a*b ~ ah*bh + ah*bl + al*bh with FP32 accumulation.
+// Vertical transforms of RBC_BF16X3 on the matrix cores: BF16 hi/lo split,
+// v_mfma_f32_32x32x16_bf16 (K = 16), a*b ~ ah*bh + ah*bl + al*bh with FP32 accumulation.
 // Operand layouts (wave64): A (32 x K) lane l holds row l%32, k = KPL*(l/32) + e;
 // B (K x 32) lane l holds column l%32, k = KPL*(l/32) + e; D (32 x 32) lane l, register r
 // holds column l%32, row 8*(r/4) + 4*(l/32) + r%4.  KPL = K/2 elements per lane.
@@ -1780,17 +1687,7 @@ __device__ __forceinline__ float bf16_to_f32(__bf16 h) {
     return __uint_as_float((unsigned)__builtin_bit_cast(unsigned short, h) << 16);
 }
 
-template <int MM>
-struct Mma;
-template <>
-struct Mma<0> {
-    static constexpr int K = 2, KPL = 1;
-    __device__ static __forceinline__ void run(f32x16& c, const float* a, const float* b) {
-        c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], b[0], c, 0, 0, 0);
-    }
-};
-template <>
-struct Mma<1> {
+struct Mma {
     static constexpr int K = 16, KPL = 8;
     __device__ static __forceinline__ void run(f32x16& c, const float* a, const float* b) {
         bf16x8 ah, al, bh, bl;
@@ -1810,10 +1707,9 @@ struct Mma<1> {
 // Evaluation on the matrix cores: D[level][column] = sum_m A_t[level][m] B_f[m][column], with
 // columns = (mode, re/im) of 16 modes per wave and 4 tables C', C, S, S' applied to f, f, g,
 // theta, theta (5 chains).  Block = 64 modes (4 waves); the block's mode data is staged in
-// LDS as [field][m][128 columns].  evA: [NLT][NKS][64][4 tables] floats for FP32 (KPL = 1, one
-// float4 per lane and k-step), [4][NLT][NKS][64][KPL] for BF16X3; ALDS: the block's A operands are
+// LDS as [field][m][128 columns].  evA: [4][NLT][NKS][64][KPL]; ALDS: the block's A operands are
 // copied to LDS with the modes (when both fit in 64 KiB).
-template <int MM, bool ALDS>
+template <bool ALDS>
 __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int per,
                                                 const cpx<float>* __restrict__ Xt,
                                                 const cpx<float>* __restrict__ Xf, const cpx<float>* __restrict__ Xg,
@@ -1821,7 +1717,7 @@ __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int
                                                 const float* __restrict__ evA, const float* __restrict__ evtab,
                                                 const float* __restrict__ kxa, const float* __restrict__ kya,
                                                 cpx<float>* __restrict__ lev) {
-    using MT = Mma<MM>;
+    using MT = Mma;
     extern __shared__ float sX[];  // 3 * 128 * (Lp + 1) modes, then sA: the block's A operands
     const int L = g.L, P = g.P, nq = g.nq;
     const int Lp = nks * MT::K;
@@ -1838,16 +1734,11 @@ __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int
     // A operands of the block's level tile, [4][nks][64][KPL], copied next to the modes
     float* sA = sX + 3 * 128 * LP;
     if (ALDS) {
-        if constexpr (MM == 0) {  // the tile's interleaved tables are one contiguous piece
-            const float4* src = reinterpret_cast<const float4*>(evA) + (size_t)lt_block * nks * 64;
-            for (int e = threadIdx.x; e < nks * 64; e += 256) reinterpret_cast<float4*>(sA)[e] = src[e];
-        } else {
-            const int na = nks * 64 * MT::KPL / 4;  // float4 per table
-            for (int e = threadIdx.x; e < 4 * na; e += 256) {
-                const int t = e / na, i = e - t * na;
-                reinterpret_cast<float4*>(sA)[e] =
-                    reinterpret_cast<const float4*>(evA + ((size_t)t * nlt + lt_block) * nks * 64 * MT::KPL)[i];
-            }
+        const int na = nks * 64 * MT::KPL / 4;  // float4 per table
+        for (int e = threadIdx.x; e < 4 * na; e += 256) {
+            const int t = e / na, i = e - t * na;
+            reinterpret_cast<float4*>(sA)[e] =
+                reinterpret_cast<const float4*>(evA + ((size_t)t * nlt + lt_block) * nks * 64 * MT::KPL)[i];
         }
     }
     // mean flow u, v (sum_m C_m F_m, sum_m C_m G_m) at the block's 32 levels, for mode p = 0
@@ -1899,27 +1790,18 @@ __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int
     const bool pvalid = p < P;
     const int pc = pvalid ? p : 0;
     const float kx = kxa[pc], ky = kya[pc], k2 = kx * kx + ky * ky;
-    const size_t fs = (size_t)nq * P;
+    const size_t fs = (size_t)nq * g.PS;
     {
         const int lt = lt_block;
         f32x16 cFp = {}, cFc = {}, cGs = {}, cTs = {}, cTz = {};
         for (int s = 0; s < nks; ++s) {
             float a[4][MT::KPL], bt[MT::KPL], bf[MT::KPL], bg[MT::KPL];
-            if constexpr (MM == 0) {  // FP32: one float4 holds the lane's value of the four tables
-                const float4 av = ALDS ? reinterpret_cast<const float4*>(sA)[s * 64 + lane]
-                                       : reinterpret_cast<const float4*>(evA)[((size_t)lt * nks + s) * 64 + lane];
-                a[0][0] = av.x;
-                a[1][0] = av.y;
-                a[2][0] = av.z;
-                a[3][0] = av.w;
-            } else {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float* src = ALDS ? sA + (((size_t)t * nks + s) * 64 + lane) * MT::KPL
-                                            : evA + ((((size_t)t * nlt + lt) * nks + s) * 64 + lane) * MT::KPL;
+            for (int t = 0; t < 4; ++t) {
+                const float* src = ALDS ? sA + (((size_t)t * nks + s) * 64 + lane) * MT::KPL
+                                        : evA + ((((size_t)t * nlt + lt) * nks + s) * 64 + lane) * MT::KPL;
 #pragma unroll
-                    for (int e = 0; e < MT::KPL; ++e) a[t][e] = src[e];
-                }
+                for (int e = 0; e < MT::KPL; ++e) a[t][e] = src[e];
             }
 #pragma unroll
             for (int e = 0; e < MT::KPL; ++e) {
@@ -1954,7 +1836,7 @@ __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int
                 v += comp ? mG.y : mG.x;
             }
             if (pvalid && l < nq) {
-                float* o = reinterpret_cast<float*>(lev) + ((size_t)l * P + p) * 2 + comp;
+                float* o = reinterpret_cast<float*>(lev) + ((size_t)l * g.PS + p) * 2 + comp;
                 o[0 * 2 * fs] = u;
                 o[1 * 2 * fs] = v;
                 o[2 * 2 * fs] = w;
@@ -1966,7 +1848,7 @@ __device__ __forceinline__ void k_eval_mma_body(DevGeom g, int nlt, int nks, int
     }
 }
 
-template <int MM, bool ALDS>
+template <bool ALDS>
 __global__ void __launch_bounds__(256) k_eval_mma(DevGeom g, int nlt, int nks, int per,
                                                   const cpx<float>* __restrict__ Xt,
                                                   const cpx<float>* __restrict__ Xf, const cpx<float>* __restrict__ Xg,
@@ -1974,7 +1856,7 @@ __global__ void __launch_bounds__(256) k_eval_mma(DevGeom g, int nlt, int nks, i
                                                   const float* __restrict__ evA, const float* __restrict__ evtab,
                                                   const float* __restrict__ kxa, const float* __restrict__ kya,
                                                   cpx<float>* __restrict__ lev) {
-    k_eval_mma_body<MM, ALDS>(g, nlt, nks, per, Xt, Xf, Xg, XF, XG, evA, evtab, kxa, kya, lev);
+    k_eval_mma_body<ALDS>(g, nlt, nks, per, Xt, Xf, Xg, XF, XG, evA, evtab, kxa, kya, lev);
 }
 // one member's arguments of k_eval_mma_batch, which runs the k_eval_mma body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
@@ -1994,11 +1876,11 @@ struct k_eval_mma_args {
     const float* kya;
     cpx<float>* lev;
 };
-template <int MM, bool ALDS>
+template <bool ALDS>
 __global__ void __launch_bounds__(256) k_eval_mma_batch(const k_eval_mma_args* __restrict__ tab, int zdim) {
     const int mb = blockIdx.z / zdim;
     const k_eval_mma_args& a = tab[mb];
-    k_eval_mma_body<MM, ALDS>(a.g, a.nlt, a.nks, a.per, a.Xt, a.Xf, a.Xg, a.XF, a.XG, a.evA, a.evtab, a.kxa, a.kya,
+    k_eval_mma_body<ALDS>(a.g, a.nlt, a.nks, a.per, a.Xt, a.Xf, a.Xg, a.XF, a.XG, a.evA, a.evtab, a.kxa, a.kya,
                               a.lev);
 }
 
@@ -2010,7 +1892,7 @@ __global__ void __launch_bounds__(256) k_eval_mma_batch(const k_eval_mma_args* _
 // m < L <= 32); the KS waves of a group split the level sum into contiguous k-step ranges and
 // add their partial sums through LDS in fixed order (KS > 1 gives small grids more waves in
 // flight).
-template <int MM, int WPB, int KS>
+template <int WPB, int KS>
 __device__ __forceinline__ void k_project_mma_body(DevGeom g, int nks, const float* __restrict__ Dfl,
                                                    const cpx<float>* __restrict__ fgw, const float* __restrict__ prA,
                                                    const float* __restrict__ prtab, const float* __restrict__ kxa,
@@ -2018,13 +1900,9 @@ __device__ __forceinline__ void k_project_mma_body(DevGeom g, int nks, const flo
                                                    cpx<float>* __restrict__ Nt, cpx<float>* __restrict__ Nf,
                                                    cpx<float>* __restrict__ Ng, cpx<float>* __restrict__ NF,
                                                    cpx<float>* __restrict__ NG) {
-    using MT = Mma<MM>;
+    using MT = Mma;
     constexpr int OS = 66;               // staging row (2L <= 64 floats plus 2 to spread banks)
-    // the FP32 form of the large grids stages one field at a time: 17 KB of LDS per block and
-    // (with the hint on the kernel) 125 registers, so that 4 blocks fit a CU and a 512^2 x 32
-    // projection (917 blocks) has all its blocks resident at once
-    constexpr int NST = (MM == 0 && WPB == 4) ? 1 : 3;
-    __shared__ float sO[WPB][NST][16 * OS];  // per wave: [field][mode][OS] staging for the write-out
+    __shared__ float sO[WPB][3][16 * OS];  // per wave: [field][mode][OS] staging for the write-out
     __shared__ f32x16 sPart[KS > 1 ? (KS - 1) * WPB : 1][KS > 1 ? 4 : 1][64];  // partials of waves wk > 0
     const int L = g.L, P = g.P, nq = g.nq;
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) % WPB, wk = (threadIdx.x >> 6) / WPB;
@@ -2034,21 +1912,21 @@ __device__ __forceinline__ void k_project_mma_body(DevGeom g, int nks, const flo
     const bool pvalid = p < P;
     const int pc = pvalid ? p : 0;
     const float kx = kxa[pc], ky = kya[pc], k2 = kx * kx + ky * ky;
-    const size_t ffs = (size_t)2 * nq * P;  // floats per combination
+    const size_t ffs = (size_t)2 * nq * g.PS;  // floats per combination
     f32x16 cF1 = {}, cF2 = {}, cG = {}, cT = {};
     const int spw = (nks + KS - 1) / KS, sbeg = wk * spw, send = min(nks, sbeg + spw);
     // Operands through buffer loads: a descriptor per level combination (its 2 nq P floats; a
     // level past nq, whose table entries are zero, lies outside the range and reads as 0) and
     // one for the tables, so that each load is a 32-bit offset that grows by a constant per
     // k-step, with no 64-bit address arithmetic.  Byte offsets stay below 2^31 (rbc_create
-    // keeps the matrix-core forms only for grids where 2 nq P floats fit).
+    // refuses larger grids).
     __amdgpu_buffer_rsrc_t rD[5];
 #pragma unroll
     for (int t = 0; t < 5; ++t)
         rD[t] = __builtin_amdgcn_make_buffer_rsrc((void*)(Dfl + t * ffs), (short)0, (int)(ffs * 4), 0x00020000);
     const __amdgpu_buffer_rsrc_t rA =
         __builtin_amdgcn_make_buffer_rsrc((void*)prA, (short)0, 5 * nks * 64 * MT::KPL * 4, 0x00020000);
-    const int dbase = (2 * pc + comp) * 4, dstep = 2 * P * 4;  // bytes: column, one level
+    const int dbase = (2 * pc + comp) * 4, dstep = 2 * g.PS * 4;  // bytes: column, one level
     auto fetch = [&](int s, float (&a)[5][MT::KPL], float (&b)[5][MT::KPL]) {
 #pragma unroll
         for (int e = 0; e < MT::KPL; ++e) {
@@ -2071,41 +1949,7 @@ __device__ __forceinline__ void k_project_mma_body(DevGeom g, int nks, const flo
         MT::run(cG, a[4], b[3]);   // wS'  . D3
         MT::run(cT, a[3], b[4]);   // wS   . D4
     };
-    // FP32: batches of U k-steps, the next batch's operands (tables and data, issued together)
-    // loading while the current batch runs on the matrix cores (loads return in issue order,
-    // so a batch waits for its own only).  Two buffers taken in turn over a loop unrolled twice,
-    // so that no buffer is copied (a copy would wait for its loads).  A load past the wave's
-    // range is harmless and unused: a step of another wave's range, or past the end of a
-    // descriptor, which reads as 0.
-    constexpr int U = 2;
-    int s = sbeg;
-    if constexpr (MM == 0) {
-        float a0[U][5][MT::KPL], b0[U][5][MT::KPL], a1[U][5][MT::KPL], b1[U][5][MT::KPL];
-        auto load = [&](int s0, float (&a)[U][5][MT::KPL], float (&b)[U][5][MT::KPL]) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) fetch(s0 + u, a[u], b[u]);
-        };
-        auto run = [&](const float (&a)[U][5][MT::KPL], const float (&b)[U][5][MT::KPL]) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) step(a[u], b[u]);
-        };
-        load(s, a0, b0);
-        for (; s + 2 * U <= send; s += 2 * U) {
-            __builtin_amdgcn_sched_barrier(0);
-            load(s + U, a1, b1);
-            __builtin_amdgcn_sched_barrier(0);
-            run(a0, b0);
-            __builtin_amdgcn_sched_barrier(0);
-            load(s + 2 * U, a0, b0);
-            __builtin_amdgcn_sched_barrier(0);
-            run(a1, b1);
-        }
-        if (s + U <= send) {  // one more whole batch, already loaded
-            run(a0, b0);
-            s += U;
-        }
-    }
-    for (; s < send; ++s) {
+    for (int s = sbeg; s < send; ++s) {
         float a[5][MT::KPL], b[5][MT::KPL];
         fetch(s, a, b);
         step(a, b);
@@ -2133,54 +1977,31 @@ __device__ __forceinline__ void k_project_mma_body(DevGeom g, int nks, const flo
     const int lm = j >> 1;  // local mode 0..15 within the wave
     const int pw0 = blockIdx.x * 16 * WPB + wave * 16;
     // 16 modes x L complex per field written contiguously ([p][m] layout) through the wave's
-    // staging rows: all three fields at once, or (NST = 1) one after another, not unrolled, so
-    // that one field's values are live at a time
-    if constexpr (NST == 3) {
+    // staging rows
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = 8 * (r >> 2) + 4 * half + (r & 3);
-            if (m < L) {
-                sO[wave][0][lm * OS + 2 * m + comp] = mt * cT[r];
-                sO[wave][1][lm * OS + 2 * m + comp] = mp * (cF1[r] + k2 * cF2[r]);
-                sO[wave][2][lm * OS + 2 * m + comp] = mp * cG[r];
-            }
-        }
-        wave_sync();
-        for (int e = lane; e < 16 * 2 * L; e += 64) {
-            const int lmode = e / (2 * L), q = e - lmode * 2 * L;
-            const int pp = pw0 + lmode;
-            if (pp < P) {
-                reinterpret_cast<float*>(Nt)[(size_t)pp * 2 * L + q] = sO[wave][0][lmode * OS + q];
-                reinterpret_cast<float*>(Nf)[(size_t)pp * 2 * L + q] = sO[wave][1][lmode * OS + q];
-                reinterpret_cast<float*>(Ng)[(size_t)pp * 2 * L + q] = sO[wave][2][lmode * OS + q];
-            }
-        }
-    } else {
-        float* so = sO[wave][0];
-#pragma unroll 1
-        for (int fld = 0; fld < 3; ++fld) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = 8 * (r >> 2) + 4 * half + (r & 3);
-                if (m < L)
-                    so[lm * OS + 2 * m + comp] =
-                        fld == 0 ? mt * cT[r] : (fld == 1 ? mp * (cF1[r] + k2 * cF2[r]) : mp * cG[r]);
-            }
-            wave_sync();
-            float* out = reinterpret_cast<float*>(fld == 0 ? Nt : (fld == 1 ? Nf : Ng));
-            for (int e = lane; e < 16 * 2 * L; e += 64) {
-                const int lmode = e / (2 * L), q = e - lmode * 2 * L;
-                const int pp = pw0 + lmode;
-                if (pp < P) out[(size_t)pp * 2 * L + q] = so[lmode * OS + q];
-            }
-            wave_sync();  // the rows are read before the next field is staged
+    for (int r = 0; r < 16; ++r) {
+        const int m = 8 * (r >> 2) + 4 * half + (r & 3);
+        if (m < L) {
+            sO[wave][0][lm * OS + 2 * m + comp] = mt * cT[r];
+            sO[wave][1][lm * OS + 2 * m + comp] = mp * (cF1[r] + k2 * cF2[r]);
+            sO[wave][2][lm * OS + 2 * m + comp] = mp * cG[r];
         }
     }
-    mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
+    wave_sync();
+    for (int e = lane; e < 16 * 2 * L; e += 64) {
+        const int lmode = e / (2 * L), q = e - lmode * 2 * L;
+        const int pp = pw0 + lmode;
+        if (pp < P) {
+            reinterpret_cast<float*>(Nt)[(size_t)pp * 2 * L + q] = sO[wave][0][lmode * OS + q];
+            reinterpret_cast<float*>(Nf)[(size_t)pp * 2 * L + q] = sO[wave][1][lmode * OS + q];
+            reinterpret_cast<float*>(Ng)[(size_t)pp * 2 * L + q] = sO[wave][2][lmode * OS + q];
+        }
+    }
+    if (blockIdx.x == 0) mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
 }
 
-template <int MM, int WPB, int KS>
-__global__ void __launch_bounds__(64 * WPB * KS) __attribute__((amdgpu_waves_per_eu(MM == 0 && WPB == 4 ? 4 : 1)))
+template <int WPB, int KS>
+__global__ void __launch_bounds__(64 * WPB * KS)
 k_project_mma(DevGeom g, int nks, const float* __restrict__ Dfl,
                                                      const cpx<float>* __restrict__ fgw, const float* __restrict__ prA,
                                                      const float* __restrict__ prtab, const float* __restrict__ kxa,
@@ -2188,7 +2009,7 @@ k_project_mma(DevGeom g, int nks, const float* __restrict__ Dfl,
                                                      cpx<float>* __restrict__ Nt, cpx<float>* __restrict__ Nf,
                                                      cpx<float>* __restrict__ Ng, cpx<float>* __restrict__ NF,
                                                      cpx<float>* __restrict__ NG) {
-    k_project_mma_body<MM, WPB, KS>(g, nks, Dfl, fgw, prA, prtab, kxa, kya, Pr, Nt, Nf, Ng, NF, NG);
+    k_project_mma_body<WPB, KS>(g, nks, Dfl, fgw, prA, prtab, kxa, kya, Pr, Nt, Nf, Ng, NF, NG);
 }
 // one member's arguments of k_project_mma_batch, which runs the k_project_mma body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
@@ -2208,12 +2029,12 @@ struct k_project_mma_args {
     cpx<float>* NF;
     cpx<float>* NG;
 };
-template <int MM, int WPB, int KS>
-__global__ void __launch_bounds__(64 * WPB * KS) __attribute__((amdgpu_waves_per_eu(MM == 0 && WPB == 4 ? 4 : 1)))
+template <int WPB, int KS>
+__global__ void __launch_bounds__(64 * WPB * KS)
 k_project_mma_batch(const k_project_mma_args* __restrict__ tab, int zdim) {
     const int mb = blockIdx.z / zdim;
     const k_project_mma_args& a = tab[mb];
-    k_project_mma_body<MM, WPB, KS>(a.g, a.nks, a.Dfl, a.fgw, a.prA, a.prtab, a.kxa, a.kya, a.Pr, a.Nt, a.Nf, a.Ng,
+    k_project_mma_body<WPB, KS>(a.g, a.nks, a.Dfl, a.fgw, a.prA, a.prtab, a.kxa, a.kya, a.Pr, a.Nt, a.Nf, a.Ng,
                                     a.NF, a.NG);
 }
 
@@ -2291,7 +2112,7 @@ __device__ __forceinline__ void y_fwd512c_body(int lb, const DevGeom& g, int nti
         for (int e = threadIdx.x; e < TwByPass::size; e += 64 * CT) twl[e] = tw[e];  // tw: in TwByPass order
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int NYc = NYC512;
-    const int P = g.P, nq = g.nq, KX = g.KX;
+    const int nq = g.nq, KX = g.KX;
     const int tix = lb % ntile, l = lb / ntile;
     const int kx0 = tix * CT;
     constexpr int a = (NYc - 1) / 2, shift = 512 - NYc;
@@ -2343,11 +2164,11 @@ __device__ __forceinline__ void y_fwd512c_body(int lb, const DevGeom& g, int nti
         __syncthreads();  // the tile is rewritten for the next product
     }
     if (cvalid) {
-        const size_t fs = (size_t)nq * P;
+        const size_t fs = (size_t)nq * g.PS;
 #pragma unroll
         for (int r = 0; r < 8; ++r)
             if (kyc[r] >= 0) {
-                cpx<float>* o = D + (size_t)l * P + (size_t)kxc * NYc + kyc[r];
+                cpx<float>* o = D + (size_t)l * g.PS + (size_t)kxc * NYc + kyc[r];
                 o[G::t0 * fs] = d0[r];
                 if (G::t1 >= 0) o[G::t1 * fs] = d1[r];
                 if (G::t2 >= 0) o[G::t2 * fs] = d2[r];
@@ -2392,7 +2213,7 @@ __device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<T>* tile,
     using Y = YShape<T, LOGN, WPB>;
     constexpr int N = Y::N, E = Y::E, W = Y::W, G = Y::G, CB = Y::CB, S = Y::S, NYc = Y::NYc, a = Y::a, shift = Y::shift;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
-    const int P = g.P, nq = g.nq, KX = g.KX;
+    const int nq = g.nq, KX = g.KX;
     const int kx0 = blockIdx.x * CB, l = blockIdx.y;
     const int c = wave * G + grp, kx = kx0 + c;
     const bool cvalid = kx < KX;
@@ -2430,8 +2251,8 @@ __device__ __forceinline__ void y_fwd_group_comb(const DevGeom& g, cpx<T>* tile,
         __syncthreads();  // the tile is refilled by the next product
     }
     if (cvalid) {
-        const size_t fs = (size_t)nq * P;
-        cpx<T>* o = D + (size_t)l * P + (size_t)kx * NYc;
+        const size_t fs = (size_t)nq * g.PS;
+        cpx<T>* o = D + (size_t)l * g.PS + (size_t)kx * NYc;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
             const int kc = kyc_of(j + W * r);
@@ -2535,6 +2356,15 @@ static inline int fft_tile(int N, size_t csz) {
     return tx;
 }
 
+// LDS of the BF16X3 evaluation: the A operands go there with the modes only while the block stays
+// within 64 KiB
+static size_t eval_mma_mode_lds(const Buffers& b) { return (size_t)3 * 128 * (b.ev_nks * Mma::K + 1) * sizeof(float); }
+static size_t eval_mma_table_lds(const Buffers& b) { return (size_t)4 * b.ev_nks * 64 * Mma::KPL * sizeof(float); }
+static bool eval_mma_tables_in_lds(const Buffers& b) { return eval_mma_mode_lds(b) + eval_mma_table_lds(b) <= 65536; }
+static size_t eval_mma_lds(const Buffers& b) {
+    return eval_mma_mode_lds(b) + (eval_mma_tables_in_lds(b) ? eval_mma_table_lds(b) : 0);
+}
+
 template <typename T, int LOGM, int WPB>
 static void launch_rows_w_t(const DevGeom& g, const Buffers& b, hipStream_t s) {
     if constexpr (RowShape<T, LOGM, WPB>::lds <= 65536) {
@@ -2586,28 +2416,21 @@ static void launch_y_fwd_wc(const DevGeom& g, const Buffers& b, hipStream_t s) {
 template <typename T>
 void Launch<T>::eval(const DevGeom& g, const Buffers& b, void* const X[3], const void* XF, const void* XG,
                      hipStream_t s) {
-    if (sizeof(T) == 4 && b.mma >= 0) {
-        const int K = b.mma == 0 ? 2 : 16;
-        const size_t sx = (size_t)3 * 128 * (b.ev_nks * K + 1) * sizeof(float);
-        const size_t sa = (size_t)4 * b.ev_nks * 64 * (K / 2) * sizeof(float);
-        // the A operands go to LDS with the modes only while the block stays within 64 KiB: at
-        // 66.7 KiB (512^2 x 32; 2 blocks per CU instead of 3) the evaluation took 103 us against 97
-        const bool alds = sx + sa <= 65536;
-        const size_t smm = alds ? sx + sa : sx;
+    if (b.evP) {
+        launch_eval<T>(eval_args<T>(g, b, X, XF, XG), nullptr, 1, s);
+        return;
+    }
+    if (sizeof(T) == 4 && b.bf16x3) {
+        const size_t smm = eval_mma_lds(b);
         const int nblk = ((g.P + 63) / 64) * b.ev_nlt, per = (nblk + 7) / 8;
         dim3 grid(8 * per);
-#define RBC_EVAL_MMA(MMV, ALDSV)                                                                                 \
-    hipLaunchKernelGGL((k_eval_mma<MMV, ALDSV>), grid, dim3(256), smm, s, g, b.ev_nlt, b.ev_nks, per,             \
+#define RBC_EVAL_MMA(ALDSV)                                                                                      \
+    hipLaunchKernelGGL((k_eval_mma<ALDSV>), grid, dim3(256), smm, s, g, b.ev_nlt, b.ev_nks, per,                  \
                        (const cpx<float>*)X[0], (const cpx<float>*)X[1], (const cpx<float>*)X[2],                \
                        (const cpx<float>*)XF, (const cpx<float>*)XG, (const float*)b.evA, (const float*)b.evtab, \
                        (const float*)b.kx, (const float*)b.ky, (cpx<float>*)b.lev)
-        if (b.mma == 0) {
-            if (alds) RBC_EVAL_MMA(0, true);
-            else RBC_EVAL_MMA(0, false);
-        } else {
-            if (alds) RBC_EVAL_MMA(1, true);
-            else RBC_EVAL_MMA(1, false);
-        }
+        if (eval_mma_tables_in_lds(b)) RBC_EVAL_MMA(true);
+        else RBC_EVAL_MMA(false);
 #undef RBC_EVAL_MMA
         return;
     }
@@ -2728,30 +2551,23 @@ void Launch<T>::project(const DevGeom& g, const Buffers& b, double Pr, void* con
                         hipStream_t s) {
     constexpr int MCH = sizeof(T) == 8 ? 4 : 8;
     dim3 grid((g.P + 63) / 64);
-    if (sizeof(T) == 4 && b.mma >= 0) {
+    if (b.prP) {
+        launch_project<T>(project_args<T>(g, b, Pr, Nout, NFo, NGo), nullptr, 1, s);
+        return;
+    }
+    if (sizeof(T) == 4 && b.bf16x3) {
         // when 64-mode blocks would leave most of the 256 CUs idle: 16-mode blocks whose four
         // waves split the level sum
         const bool small = (g.P + 63) / 64 < 512;
         const dim3 gr = small ? dim3((g.P + 15) / 16) : grid, bl = dim3(256);
-#define RBC_PROJECT_MMA(MMV, WPBV)                                                                              \
-    hipLaunchKernelGGL((k_project_mma<MMV, WPBV, 4 / WPBV>), gr, bl, 0, s, g, b.pr_nks, (const float*)b.lev,      \
+#define RBC_PROJECT_MMA(WPBV)                                                                                   \
+    hipLaunchKernelGGL((k_project_mma<WPBV, 4 / WPBV>), gr, bl, 0, s, g, b.pr_nks, (const float*)b.lev,           \
                        (const cpx<float>*)b.fgw, (const float*)b.prA, (const float*)b.prtab, (const float*)b.kx,   \
                        (const float*)b.ky, (float)Pr, (cpx<float>*)Nout[0], (cpx<float>*)Nout[1],                \
                        (cpx<float>*)Nout[2], (cpx<float>*)NFo, (cpx<float>*)NGo)
-        if (b.mma == 0) {
-            if (small) RBC_PROJECT_MMA(0, 1);
-            else RBC_PROJECT_MMA(0, 4);
-        } else {
-            if (small) RBC_PROJECT_MMA(1, 1);
-            else RBC_PROJECT_MMA(1, 4);
-        }
+        if (small) RBC_PROJECT_MMA(1);
+        else RBC_PROJECT_MMA(4);
 #undef RBC_PROJECT_MMA
-        return;
-    }
-    if (g.L <= 4 * MCH) {
-        hipLaunchKernelGGL((k_project_lds<T, MCH>), grid, dim3(256), 0, s, g, (const cpx<T>*)b.lev,
-                           (const cpx<T>*)b.fgw, (const T*)b.prtab, (const T*)b.kx, (const T*)b.ky, (T)Pr,
-                           (cpx<T>*)Nout[0], (cpx<T>*)Nout[1], (cpx<T>*)Nout[2], (cpx<T>*)NFo, (cpx<T>*)NGo);
         return;
     }
     hipLaunchKernelGGL((k_project<T, MCH>), grid, dim3(256), 0, s, g, (const cpx<T>*)b.lev, (const cpx<T>*)b.fgw,
@@ -2877,6 +2693,7 @@ void Launch<T>::penalty(const DevGeom& g, const Buffers& b, const Penalty& pen, 
     // the generic y-transforms with the L modes in place of the levels, ten fields
     DevGeom gp = g;
     gp.nq = g.L;
+    gp.PS = g.P;
     const int TX = fft_tile(g.N, sizeof(cpx<T>));
     const size_t sm = (size_t)2 * TX * g.N * sizeof(cpx<T>);
     const dim3 gy((g.KX + TX - 1) / TX, g.L, 10);
@@ -2901,6 +2718,7 @@ void Launch<T>::plane_op(const DevGeom& g, const Buffers& b, int op, int nf, con
                        (const cpx<T>*)X[2], (cpx<T>*)spec);
     DevGeom gp = g;
     gp.nq = g.L;
+    gp.PS = g.P;
     const int TX = fft_tile(g.N, sizeof(cpx<T>));
     const size_t sm = (size_t)2 * TX * g.N * sizeof(cpx<T>);
     const dim3 gy((g.KX + TX - 1) / TX, g.L, nf);
@@ -2935,7 +2753,7 @@ template struct Launch<double>;
 struct StepBatch {
     int B = 0;
     DevGeom g;            // the class geometry (launch shapes; Lx, Ly come from each member's table)
-    int mma = 0;          // 0: FP32 MFMA, 1: BF16 x3
+    bool bf16x3 = false;  // BF16X3 vertical transforms (ev, pj); else those of rbc_vertical.hip (pev, ppj)
     bool alds = false;    // evaluation operand tables in LDS
     size_t ev_smem = 0;   // evaluation dynamic LDS
     int ev_blocks = 0;    // evaluation blocks per member (XCD-ordered 1-D grid)
@@ -2949,6 +2767,10 @@ struct StepBatch {
     k_rows_w_args* rw = nullptr;
     k_fft_y_fwd_wc_args* yf = nullptr;
     k_project_mma_args* pj = nullptr;
+    EvalArgs<float>* pev = nullptr;
+    ProjectArgs<float>* ppj = nullptr;
+    EvalArgs<float> pev0;  // the first member's, for the launch shape
+    ProjectArgs<float> ppj0;
     k_update32_args<float>* up = nullptr;
     k_finish_args<float>* fi = nullptr;
 };
@@ -2964,7 +2786,7 @@ static A* upload_table(const std::vector<A>& v) {
 void batch_destroy(StepBatch* sb) {
     if (!sb) return;
     for (void* p : {(void*)sb->ev, (void*)sb->yi, (void*)sb->rw, (void*)sb->yf, (void*)sb->pj, (void*)sb->up,
-                    (void*)sb->fi})
+                    (void*)sb->fi, (void*)sb->pev, (void*)sb->ppj})
         if (p) hipFree(p);
     delete sb;
 }
@@ -2979,7 +2801,7 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
     // the single-run path these kernels stand for: FP32 storage on the matrix cores, group
     // transforms in both directions, the register group update
     const bool sized = g.M >= 64 && g.M <= 256 && g.N >= 64 && g.N <= 256;
-    if (b0.mma < 0 || g.L > 32 || !sized || !wave_rows_log<float>(g) || !wave_y_log<float>(g)) {
+    if (!(b0.bf16x3 || b0.evP) || g.L > 32 || !sized || !wave_rows_log<float>(g) || !wave_y_log<float>(g)) {
         why = "not on the batched path (FP32/BF16X3 storage, 64..256-point group transforms, L <= 32)";
         return nullptr;
     }
@@ -2998,7 +2820,7 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
         const DevGeom& h = *x.g;
         const Buffers& b = *x.b;
         if (h.M != g.M || h.N != g.N || h.L != g.L || h.nq != g.nq || h.KX != g.KX || h.KXp != g.KXp ||
-            h.NYc != g.NYc || h.P != g.P || b.mma != b0.mma || b.ev_nlt != b0.ev_nlt || b.ev_nks != b0.ev_nks ||
+            h.NYc != g.NYc || h.P != g.P || b.bf16x3 != b0.bf16x3 || !b.evP != !b0.evP || b.ev_nlt != b0.ev_nlt || b.ev_nks != b0.ev_nks ||
             b.pr_nks != b0.pr_nks || b.tune_ytx != b0.tune_ytx || b.tune_rows_threads != b0.tune_rows_threads) {
             why = "members differ in launch shape";
             return nullptr;
@@ -3007,21 +2829,18 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
     StepBatch* sb = new StepBatch;
     sb->B = (int)m.size();
     sb->g = g;
-    sb->mma = b0.mma;
+    sb->bf16x3 = b0.bf16x3;
     sb->yi_wpb = yi_wpb;
     sb->yf_wpb = yf_wpb;
     sb->rows_wpb = rows_wpb;
-    {
-        const int K = b0.mma == 0 ? 2 : 16;
-        const size_t sx = (size_t)3 * 128 * (b0.ev_nks * K + 1) * sizeof(float);
-        const size_t sa = (size_t)4 * b0.ev_nks * 64 * (K / 2) * sizeof(float);
-        sb->alds = sx + sa <= 65536;
-        sb->ev_smem = sb->alds ? sx + sa : sx;
-    }
+    sb->alds = eval_mma_tables_in_lds(b0);
+    sb->ev_smem = eval_mma_lds(b0);
     const int nblk = ((g.P + 63) / 64) * b0.ev_nlt, per = (nblk + 7) / 8;
     sb->ev_blocks = 8 * per;
     sb->small_proj = (g.P + 63) / 64 < 512;
     std::vector<k_eval_mma_args> ev;
+    std::vector<EvalArgs<float>> pev;
+    std::vector<ProjectArgs<float>> ppj;
     std::vector<k_fft_y_inv_w_args> yi;
     std::vector<k_rows_w_args> rw;
     std::vector<k_fft_y_fwd_wc_args> yf;
@@ -3032,16 +2851,21 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
         const DevGeom& h = *x.g;
         const Buffers& b = *x.b;
         using C = cpx<float>;
-        ev.push_back({h, b.ev_nlt, b.ev_nks, per, (const C*)b.X[0], (const C*)b.X[1], (const C*)b.X[2],
-                      (const C*)b.XF, (const C*)b.XG, (const float*)b.evA, (const float*)b.evtab,
-                      (const float*)b.kx, (const float*)b.ky, (C*)b.lev});
+        if (b.bf16x3) {
+            ev.push_back({h, b.ev_nlt, b.ev_nks, per, (const C*)b.X[0], (const C*)b.X[1], (const C*)b.X[2],
+                          (const C*)b.XF, (const C*)b.XG, (const float*)b.evA, (const float*)b.evtab,
+                          (const float*)b.kx, (const float*)b.ky, (C*)b.lev});
+            pj.push_back({h, b.pr_nks, (const float*)b.lev, (const C*)b.fgw, (const float*)b.prA,
+                          (const float*)b.prtab, (const float*)b.kx, (const float*)b.ky, (float)x.Pr, (C*)b.Nn[0],
+                          (C*)b.Nn[1], (C*)b.Nn[2], (C*)b.NF, (C*)b.NG});
+        } else {
+            pev.push_back(eval_args<float>(h, b, b.X, b.XF, b.XG));
+            ppj.push_back(project_args<float>(h, b, x.Pr, b.Nn, b.NF, b.NG));
+        }
         yi.push_back({h, (const C*)b.lev, (const C*)b.twN, (C*)b.hin});
         rw.push_back({h, (const C*)b.hin, (const C*)b.twM, (C*)b.hout});
         yf.push_back({h, (const C*)b.hout, (const C*)b.twN, (const float*)b.kx, (const float*)b.ky, (C*)b.lev,
                       (C*)b.fgw});
-        pj.push_back({h, b.pr_nks, (const float*)b.lev, (const C*)b.fgw, (const float*)b.prA, (const float*)b.prtab,
-                      (const float*)b.kx, (const float*)b.ky, (float)x.Pr, (C*)b.Nn[0], (C*)b.Nn[1], (C*)b.Nn[2],
-                      (C*)b.NF, (C*)b.NG});
         // AB2 coefficients: a batch only runs members that have their history
         const float a_cur = (float)(1.5 * x.dt), a_prev = (float)(-0.5 * x.dt);
         up.push_back({h, b.nchunk, x.L0, x.L1, x.stride, (float)x.Pr, (float)x.dt, a_cur, a_prev, 1, b.cgrp, b.cbeg,
@@ -3053,11 +2877,18 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
         sb->nchunk_max = std::max(sb->nchunk_max, b.nchunk);
     }
     try {
-        sb->ev = upload_table(ev);
+        if (b0.bf16x3) {
+            sb->ev = upload_table(ev);
+            sb->pj = upload_table(pj);
+        } else {
+            sb->pev0 = pev[0];
+            sb->ppj0 = ppj[0];
+            sb->pev = upload_table(pev);
+            sb->ppj = upload_table(ppj);
+        }
         sb->yi = upload_table(yi);
         sb->rw = upload_table(rw);
         sb->yf = upload_table(yf);
-        sb->pj = upload_table(pj);
         sb->up = upload_table(up);
         sb->fi = upload_table(fi);
     } catch (const HipError&) {
@@ -3072,18 +2903,12 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
 void batch_step(const StepBatch* sb, hipStream_t s) {
     const DevGeom& g = sb->g;
     const int B = sb->B;
-    {
+    if (sb->bf16x3) {
         const dim3 gr(sb->ev_blocks, 1, B);
-#define RBC_EVB(MMV, ALDSV) \
-    hipLaunchKernelGGL((k_eval_mma_batch<MMV, ALDSV>), gr, dim3(256), sb->ev_smem, s, sb->ev, 1)
-        if (sb->mma == 0) {
-            if (sb->alds) RBC_EVB(0, true);
-            else RBC_EVB(0, false);
-        } else {
-            if (sb->alds) RBC_EVB(1, true);
-            else RBC_EVB(1, false);
-        }
-#undef RBC_EVB
+        if (sb->alds) hipLaunchKernelGGL((k_eval_mma_batch<true>), gr, dim3(256), sb->ev_smem, s, sb->ev, 1);
+        else hipLaunchKernelGGL((k_eval_mma_batch<false>), gr, dim3(256), sb->ev_smem, s, sb->ev, 1);
+    } else {
+        launch_eval<float>(sb->pev0, sb->pev, B, s);
     }
     const int G = 512 / g.N;
     {
@@ -3129,18 +2954,12 @@ void batch_step(const StepBatch* sb, hipStream_t s) {
 #undef RBC_YFB_L
 #undef RBC_YFB
     }
-    {
+    if (sb->bf16x3) {
         const dim3 gr(sb->small_proj ? (g.P + 15) / 16 : (g.P + 63) / 64, 1, B);
-#define RBC_PJB(MMV, WPBV) \
-    hipLaunchKernelGGL((k_project_mma_batch<MMV, WPBV, 4 / WPBV>), gr, dim3(256), 0, s, sb->pj, 1)
-        if (sb->mma == 0) {
-            if (sb->small_proj) RBC_PJB(0, 1);
-            else RBC_PJB(0, 4);
-        } else {
-            if (sb->small_proj) RBC_PJB(1, 1);
-            else RBC_PJB(1, 4);
-        }
-#undef RBC_PJB
+        if (sb->small_proj) hipLaunchKernelGGL((k_project_mma_batch<1, 4>), gr, dim3(256), 0, s, sb->pj, 1);
+        else hipLaunchKernelGGL((k_project_mma_batch<4, 1>), gr, dim3(256), 0, s, sb->pj, 1);
+    } else {
+        launch_project<float>(sb->ppj0, sb->ppj, B, s);
     }
     {
         const dim3 gr((sb->nchunk_max + 3) / 4, 1, B);

@@ -1079,6 +1079,7 @@ void set_heights(rbc_ctx* c, GridWork& w, const std::vector<double>& z) {
 // velocity grid at the heights of w (spectral -> y-FFT -> x C2R), on the context's stream
 void velocity_grid(rbc_ctx* c, const GridWork& w) {
     DevGeom gt = c->dg;
+    gt.PS = gt.P;
     gt.nq = w.nz;
     if (c->rsz == 8) launch_vel_levels<double>(c, gt, w.nz, w.zb, w.spec);
     else launch_vel_levels<float>(c, gt, w.nz, w.zb, w.spec);
