@@ -41,10 +41,10 @@ def stage_bytes(st, cs, nprod):
         # forward y-FFT reads the product rows and writes the 5 level combinations
         "fft_y_fwd": (nprod * nq * H + 5 * nq * P) * cs,
         "project": (5 * nq * P + 3 * L * P) * cs,
-        # state, N and history in/out; factor records once per |k|^2 group
+        # state, N and history in/out; factor records once per |k|^2 group (the kx = 0 column's mirror,
+        # F and G ride along: the "finish" stage is empty)
         "update": (9 * L * P + 6 * L * P) * cs + st.n_unique_k * (2 * L * L + L * L // 2) * (cs // 2),
-        # make_real of the kx = 0 column and the F, G update
-        "finish": 2 * 3 * st.ky_kept * L * cs + 8 * L * cs,
+        "finish": 0,
     }
 
 
@@ -83,8 +83,7 @@ def fft_product_stage(st, stages, cs):
 # matrix-core kernels, with the same memory traffic)
 STAGE_KERNELS = {"eval": ["k_eval_mma<0, false>"], "fft_y_inv": ["k_fft_y_inv512"], "rows_products": ["k_rows512t"],
                  "fft_y_fwd": ["k_fft_y_fwd512c2<8>"],
-                 "project": ["k_project_mma<0, 4, 1>"], "update": ["k_update32<float, 32>"],
-                 "finish": ["k_finish<float>"]}
+                 "project": ["k_project_mma<0, 4, 1>"], "update": ["k_update<float, 32, 32, 0>"], "finish": []}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "hbm_traffic_512x512x32_f32.md")
 
 

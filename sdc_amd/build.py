@@ -14,7 +14,8 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libsdc_rbc.so")
 
 SOURCES = ["rbc_setup.cpp", "rbc_abi.cpp", "rbc_io.cpp", "rbc_ensemble.cpp", "rbc_driver.cpp", "rbc_kernels.hip",
-           "rbc_vertical.hip", "rbc_velocity.hip", "rbc_closure.hip"]
+           "rbc_vertical.hip", "rbc_update.hip",
+           "rbc_velocity.hip", "rbc_closure.hip"]
 RUN_EXE = os.path.join(HERE, "rbc_run")
 EXTRACT_EXE = os.path.join(HERE, "rbc_extract_vel")
 ARCH = os.environ.get("SDC_AMD_ARCH", "gfx950")

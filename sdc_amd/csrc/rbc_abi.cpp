@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "rbc_ctx.hpp"
+#include "rbc_update.hpp"
 
 using namespace rbc;
 
@@ -113,10 +114,12 @@ void one_step(rbc_ctx* c, bool timed) {
     if (timed) HIPCHK(hipEventRecord(c->ev[0], c->stream));
     nonlinear_into<T>(c, c->b.X, c->b.XF, c->b.XG, c->b.Nn, c->b.NF, c->b.NG, timed ? 0 : -1);
     if (c->post_nonlinear) c->post_nonlinear(c, c->post_user);
-    Launch<T>::update(c->dg, c->b, c->fac.ngroups(), c->fac.L0, c->fac.L1, c->fac.stride, c->p.Pr, c->p.dt, sc,
-                      UPD_STEP, c->b.X, c->b.Nn, c->b.Rp, c->stream);
+    Buffers& b = c->b;
+    launch_update<T>(update_args<T>(c->dg, b, c->fac.L0, c->fac.L1, c->fac.stride, c->p.Pr, c->p.dt, sc, b.X, b.Nn, b.Rp,
+                                    b.XF, b.XG, b.NF, b.NG, b.RpF, b.RpG),
+                     UPD_STEP, nullptr, 0, 1, c->stream);
     if (timed) HIPCHK(hipEventRecord(c->ev[6], c->stream));
-    Launch<T>::finish(c->dg, c->b, c->p.Pr, c->p.dt, sc, c->stream);  // make_real + F, G update
+    // stage "finish" (make_real and F, G) is part of the group update
     if (timed) HIPCHK(hipEventRecord(c->ev[7], c->stream));
     HIPCHK(hipGetLastError());
     c->have_hist = true;
@@ -387,17 +390,14 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
         upload_reals(c.get(), b.k2, c->fac.k2);
         b.rows = (int*)c->dalloc(g.rows.size() * sizeof(int));
         HIPCHK(hipMemcpy(b.rows, g.rows.data(), g.rows.size() * sizeof(int), hipMemcpyHostToDevice));
-        b.gstart = (int*)c->dalloc(c->fac.group_start.size() * sizeof(int));
         b.gmem = (int*)c->dalloc(c->fac.members.size() * sizeof(int));
-        HIPCHK(hipMemcpy(b.gstart, c->fac.group_start.data(), c->fac.group_start.size() * sizeof(int),
-                         hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(b.gmem, c->fac.members.data(), c->fac.members.size() * sizeof(int), hipMemcpyHostToDevice));
-        {  // chunks of at most kChunk members per wave of the group update: a wave runs its members
+        {  // chunks of members, one chunk per wave of the group update: a wave runs its members
            // one after another, so small grids (few modes, a few thousand waves at most) take one
            // member per wave; larger grids take 4, which matches the usual group size (the
            // (+-kx, +-ky) images of a mode) and shares the group's matrix loads (measured at
            // 512^2 x 32: 98 us with 4, 103 us with 2, 116 us with 8 members per chunk)
-            const int kChunk = g.P() >= 8192 ? 4 : 1;
+            const int kChunk = g.P() >= 8192 ? kUpdateChunk : 1;
             std::vector<int> cg, cb;
             const auto& gs = c->fac.group_start;
             for (int gi = 0; gi + 1 < (int)gs.size(); ++gi)
@@ -522,22 +522,17 @@ namespace {
 template <typename T>
 void op_core_t(rbc_ctx* c, int which, void** outs, void** oF, void** oG) {
     Buffers& b = c->b;
-    StepCoef sc{0.0, 0.0, 0};
+    const auto args = update_args<T>(c->dg, b, c->fac.L0, c->fac.L1, c->fac.stride, c->p.Pr, c->p.dt, {0.0, 0.0, 0}, b.Xo,
+                                     b.Xo, b.Oo, b.XoF, b.XoG, b.XoF, b.XoG, b.OoF, b.OoG);
     for (int i = 0; i < 3; ++i) outs[i] = b.Oo[i];
     *oF = b.OoF;
     *oG = b.OoG;
     if (which == 0) {
         nonlinear_into<T>(c, b.Xo, b.XoF, b.XoG, b.Oo, b.OoF, b.OoG, -1);
     } else if (which == 1) {  // inverse B: N in Xo -> R in Oo
-        Launch<T>::update(c->dg, b, c->fac.ngroups(), c->fac.L0, c->fac.L1, c->fac.stride, c->p.Pr, c->p.dt, sc,
-                          UPD_INVB, b.Xo, b.Xo, b.Oo, c->stream);
-        Launch<T>::update_FG(c->dg, c->p.Pr, c->p.dt, sc, UPD_INVB, b.XoF, b.XoG, b.XoF, b.XoG, b.OoF, b.OoG,
-                             c->stream);
+        launch_update<T>(args, UPD_INVB, nullptr, 0, 1, c->stream);
     } else {  // implicit: in place on Xo
-        Launch<T>::update(c->dg, b, c->fac.ngroups(), c->fac.L0, c->fac.L1, c->fac.stride, c->p.Pr, c->p.dt, sc,
-                          UPD_IMPLICIT, b.Xo, b.Xo, b.Oo, c->stream);
-        Launch<T>::update_FG(c->dg, c->p.Pr, c->p.dt, sc, UPD_IMPLICIT, b.XoF, b.XoG, b.XoF, b.XoG, b.OoF, b.OoG,
-                             c->stream);
+        launch_update<T>(args, UPD_IMPLICIT, nullptr, 0, 1, c->stream);
         for (int i = 0; i < 3; ++i) outs[i] = b.Xo[i];
         *oF = b.XoF;
         *oG = b.XoG;

@@ -112,9 +112,8 @@ struct Buffers {
     void* ky;     // P real
     void* k2;     // P real
     int* rows;    // NYc kept rows
-    int* gstart;  // ngroups + 1
     int* gmem;    // P
-    // work chunks of at most kChunk members of one group (a group's chunks are consecutive):
+    // work chunks of at most kUpdateChunk members of one group (a group's chunks are consecutive):
     // chunk c covers members [cbeg[c], cbeg[c+1]) of group cgrp[c]
     int* cgrp;
     int* cbeg;
@@ -124,7 +123,7 @@ struct Buffers {
     int nred;
     // step health: health[0] = 1 + the step count at which the end-of-step check first saw a
     // non-finite value (0 = none), health[1] = steps finished since create (both written by the
-    // last block of the end-of-step kernel only)
+    // wave of the k = 0 mode in the group update only)
     int* health;
     // BF16 x3 vertical transforms (RBC_BF16X3)
     bool bf16x3 = false;
@@ -168,6 +167,9 @@ struct StepCoef {
     int use_prev;
 };
 
+// members per wave of the group update, at most
+constexpr int kUpdateChunk = 4;
+
 enum UpdateMode { UPD_STEP = 0, UPD_INVB = 1, UPD_IMPLICIT = 2 };
 
 // plane operators on the state's mode planes (freeze_operator.cu, masktemp.cu, masking.cu)
@@ -197,16 +199,6 @@ struct Launch {
     // stage 5: vertical projection -> N (theta, f, g, F, G), scaled as the reference does
     static void project(const DevGeom& g, const Buffers& b, double Pr, void* const Nout[3],
                         void* NFo, void* NGo, hipStream_t s);
-    // stage 6: per-|k|^2 group update: inverse B, AB2 combine, implicit Euler
-    static void update(const DevGeom& g, const Buffers& b, int ngroups, int L0, int L1,
-                       int stride, double Pr, double dt, StepCoef sc, int mode,
-                       void* const Xio[3], void* const Nin[3], void* const Rp[3], hipStream_t s);
-    // F and G (mean flow) update
-    static void update_FG(const DevGeom& g, double Pr, double dt, StepCoef sc, int mode,
-                          void* XF, void* XG, const void* NF, const void* NG, void* RpF,
-                          void* RpG, hipStream_t s);
-    // make_real of X and the F, G update of a time step (mode UPD_STEP) in one launch
-    static void finish(const DevGeom& g, const Buffers& b, double Pr, double dt, StepCoef sc, hipStream_t s);
     // make_real on the kx = 0 column (util.cu make_real)
     static void make_real(const DevGeom& g, const Buffers& b, void* const X[3], hipStream_t s);
     static void nusselt(const DevGeom& g, const Buffers& b, const void* ia1, hipStream_t s);

@@ -13,6 +13,7 @@
 
 #include "rbc_ctx.hpp"
 #include "rbc_device.hpp"
+#include "rbc_update.hpp"
 #include "rbc_vertical.hpp"
 
 namespace rbc {
@@ -335,341 +336,6 @@ __global__ void __launch_bounds__(256) k_project(DevGeom g, const cpx<T>* __rest
     if (blockIdx.x == 0) mean_flow_projection(g, fgw, prtab, Pr, NF, NG);
 }
 
-// ---------------------------------------------------------------------------------------
-// Stage 6: group update.  One block (64 lanes) per |k|^2 group; lanes 0..31 serve parity
-// class 0 and 32..63 class 1 (rows of the class matrices, looped when a class is larger).
-// Per member mode:
-//   mode UPD_STEP:     R = B^-1 N;  X += a_cur R;  X += a_prev R_prev;  X = C^-1 X;  R_prev = R
-//   mode UPD_INVB:     out = B^-1 N              (inverse_B_matrix::calculate_inverse)
-//   mode UPD_IMPLICIT: out = C^-1 X              (linear_implicit_operator::calculate_operator)
-// g uses its diagonal factors (inverse_B_matrix.cu:276-300, linear_implicit_operator.cu:419-458).
-// ---------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(64) k_update(DevGeom g, int L0, int L1, int stride, T Pr, T dt, T a_cur,
-                                               T a_prev, int use_prev, int mode,
-                                               const int* __restrict__ gstart, const int* __restrict__ gmem,
-                                               const T* __restrict__ gmat, const T* __restrict__ k2a,
-                                               cpx<T>* __restrict__ Xt, cpx<T>* __restrict__ Xf,
-                                               cpx<T>* __restrict__ Xg, const cpx<T>* __restrict__ Nt,
-                                               const cpx<T>* __restrict__ Nf, const cpx<T>* __restrict__ Ng,
-                                               cpx<T>* __restrict__ Rt, cpx<T>* __restrict__ Rf,
-                                               cpx<T>* __restrict__ Rg) {
-    extern __shared__ unsigned char smem_raw[];
-    const int L = g.L;
-    cpx<T>* rhs = reinterpret_cast<cpx<T>*>(smem_raw);  // 2L: [class0 theta, f][class1 theta, f]
-    cpx<T>* nfv = rhs + 2 * L;                          // L: N_f reordered by class
-    const int grp = blockIdx.x;
-    const int b0 = gstart[grp], b1 = gstart[grp + 1];
-    const int lane = threadIdx.x;
-    const int cls = lane >> 5, cl = lane & 31;
-    const int Lc = cls ? L1 : L0, nc = 2 * Lc;
-    const int n0 = 2 * L0;
-    const T* Cinv = gmat + (size_t)grp * stride + (cls ? (size_t)n0 * n0 : 0);
-    const T* Binv = gmat + (size_t)grp * stride + (size_t)n0 * n0 + (size_t)(2 * L1) * (2 * L1) +
-                    (cls ? (size_t)L0 * L0 : 0);
-    const int rbase = cls ? 2 * L0 : 0;  // offset of this class in rhs
-    for (int mi = b0; mi < b1; ++mi) {
-        const int p = gmem[mi];
-        const size_t base = (size_t)p * L;
-        const T k2 = k2a[p];
-        // ---- gather: class c holds modes m = c, c+2, ... ; rhs = [theta_c | f_c]
-        for (int e = lane; e < L; e += 64) {
-            const int c = e & 1, idx = e >> 1;
-            const int off = (c ? 2 * L0 : 0);
-            const int Lcc = c ? L1 : L0;
-            if (mode == UPD_STEP) {
-                rhs[off + idx] = Xt[base + e];
-                rhs[off + Lcc + idx] = Xf[base + e];
-                nfv[off / 2 + idx] = Nf[base + e];
-            } else if (mode == UPD_INVB) {
-                nfv[off / 2 + idx] = Nf[base + e];
-            } else {
-                rhs[off + idx] = Xt[base + e];
-                rhs[off + Lcc + idx] = Xf[base + e];
-            }
-        }
-        __syncthreads();
-        // ---- inverse B on f (class matvec), theta x2, and the AB2 combine
-        if (mode != UPD_IMPLICIT) {
-            for (int r = cl; r < Lc; r += 32) {
-                const int m = cls + 2 * r;
-                cpx<T> rf = mk<T>(0, 0);
-                for (int j = 0; j < Lc; ++j) rf = rf + cscale(nfv[rbase / 2 + j], Binv[(size_t)j * Lc + r]);
-                const cpx<T> rt = cscale(Nt[base + m], T(2));
-                if (mode == UPD_INVB) {
-                    Rt[base + m] = rt;
-                    Rf[base + m] = rf;
-                } else {
-                    cpx<T> xt = rhs[rbase + r], xf = rhs[rbase + Lc + r];
-                    xt = xt + cscale(rt, a_cur);
-                    xf = xf + cscale(rf, a_cur);
-                    if (use_prev) {
-                        xt = xt + cscale(Rt[base + m], a_prev);
-                        xf = xf + cscale(Rf[base + m], a_prev);
-                    }
-                    Rt[base + m] = rt;
-                    Rf[base + m] = rf;
-                    rhs[rbase + r] = xt;
-                    rhs[rbase + Lc + r] = xf;
-                }
-            }
-            __syncthreads();
-        }
-        // ---- implicit Euler: x = C^-1 rhs per class
-        if (mode != UPD_INVB) {
-            cpx<T> outv[4];
-            int cnt = 0;
-            for (int r = cl; r < nc && cnt < 4; r += 32, ++cnt) {
-                cpx<T> acc = mk<T>(0, 0);
-                for (int j = 0; j < nc; ++j) acc = acc + cscale(rhs[rbase + j], Cinv[(size_t)j * nc + r]);
-                outv[cnt] = acc;
-            }
-            cnt = 0;
-            for (int r = cl; r < nc && cnt < 4; r += 32, ++cnt) {
-                const int m = cls + 2 * (r < Lc ? r : r - Lc);
-                if (r < Lc) Xt[base + m] = outv[cnt];
-                else Xf[base + m] = outv[cnt];
-            }
-        }
-        // ---- g: diagonal factors
-        for (int m = lane; m < L; m += 64) {
-            const T mpi = T(m + 1) * T(M_PI);
-            if (mode == UPD_INVB) {
-                Rg[base + m] = (k2 != T(0)) ? cscale(Ng[base + m], T(-2) * Pr / k2) : mk<T>(0, 0);
-            } else if (mode == UPD_IMPLICIT) {
-                Xg[base + m] = (k2 != T(0)) ? cscale(Xg[base + m], T(1) / (T(1) + dt * Pr * (k2 + mpi * mpi)))
-                                            : mk<T>(0, 0);
-            } else {
-                const cpx<T> rg = (k2 != T(0)) ? cscale(Ng[base + m], T(-2) * Pr / k2) : mk<T>(0, 0);
-                cpx<T> xg = Xg[base + m] + cscale(rg, a_cur);
-                if (use_prev) xg = xg + cscale(Rg[base + m], a_prev);
-                Rg[base + m] = rg;
-                Xg[base + m] = (k2 != T(0)) ? cscale(xg, T(1) / (T(1) + dt * Pr * (k2 + mpi * mpi))) : mk<T>(0, 0);
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// Group update for L <= 32 with the class matrices held in registers: one wave per group
-// (4 groups per block), lane (class c, row r) keeps row r of C^-1 (n_c <= NC values) and of
-// B^-1_f (L_c <= NC / 2 values) for every member of the group; NC = 32, or 16 for L <= 16.
-// Same arithmetic and rounding order as k_update; mode UPD_STEP only.
-template <typename T, int NC>
-__device__ __forceinline__ void k_update32_body(DevGeom g, int nchunk, int L0, int L1, int stride, T Pr, T dt,
-                                                T a_cur, T a_prev, int use_prev, const int* __restrict__ cgrp,
-                                                const int* __restrict__ cbeg,
-                                                const int* __restrict__ gmem, const T* __restrict__ gmat,
-                                                const T* __restrict__ k2a, cpx<T>* __restrict__ Xt,
-                                                cpx<T>* __restrict__ Xf, cpx<T>* __restrict__ Xg,
-                                                const cpx<T>* __restrict__ Nt, const cpx<T>* __restrict__ Nf,
-                                                const cpx<T>* __restrict__ Ng, cpx<T>* __restrict__ Rt,
-                                                cpx<T>* __restrict__ Rf, cpx<T>* __restrict__ Rg) {
-    __shared__ cpx<T> shm[4][2][2][32];  // [wave][class][0: N_f, 1: rhs][j]
-    // the wave index as a wave-uniform value: chunk, group and member indices then live in
-    // scalar registers and come from scalar loads, which the vector loads do not wait for
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ch = blockIdx.x * 4 + wave;  // one chunk (<= kChunk members of one group) per wave
-    if (ch >= nchunk) return;               // whole wave leaves; no block-wide barrier below
-    const int grp = cgrp[ch];
-    const int L = g.L;
-    const int cls = lane >> 5, r = lane & 31;
-    const int Lc = cls ? L1 : L0, nc = 2 * Lc, n0 = 2 * L0;
-    const T* rec = gmat + (size_t)grp * stride;
-    const T* Cinv = rec + (cls ? (size_t)n0 * n0 : 0);
-    const T* Binv = rec + (size_t)n0 * n0 + (size_t)(2 * L1) * (2 * L1) + (cls ? (size_t)L0 * L0 : 0);
-    // Every load below is issued by every lane (lanes outside the class read element 0 of a
-    // valid array and discard it), and the matrix-vector sums run over the full 16 / 32 terms
-    // with zero matrix entries and zero LDS slots beyond the class size: no branch depends on
-    // the class sizes, so the compiler can keep the next member's loads in flight across the
-    // current member's arithmetic.  The extra terms add exact zeros (bit-identical sums).
-    T crow[NC], brow[NC / 2];
-    {
-        const T* csrc = nc > 0 ? Cinv : rec;
-        const T* bsrc = Lc > 0 ? Binv : rec;
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-            const bool in = j < nc && r < nc;
-            const T v = csrc[in ? (size_t)j * nc + r : 0];
-            crow[j] = in ? v : T(0);
-        }
-#pragma unroll
-        for (int j = 0; j < NC / 2; ++j) {
-            const bool in = j < Lc && r < Lc;
-            const T v = bsrc[in ? (size_t)j * Lc + r : 0];
-            brow[j] = in ? v : T(0);
-        }
-    }
-    cpx<T>* snf = shm[wave][cls][0];
-    cpx<T>* srhs = shm[wave][cls][1];
-    for (int e = r; e < 64; e += 32) shm[wave][cls][e >> 5][e & 31] = mk<T>(0, 0);  // slots beyond the class stay 0
-    const int b0 = cbeg[ch], b1 = cbeg[ch + 1];
-    const bool tf = r < Lc, gl = lane < L;
-    const int m = tf ? cls + 2 * r : 0;  // theta/f mode of this lane (element 0 outside the class)
-    const int mg = gl ? lane : 0;        // g mode of this lane
-    // one member's loads (issued together)
-    struct Member {
-        cpx<T> nf, xt, xf, nt, rt, rf, ng, xg, rg;
-        T k2;
-        size_t base;
-    };
-    auto fetch = [&](int mi, Member& d) {
-        const int p = gmem[mi];
-        d.base = (size_t)p * L;
-        d.k2 = k2a[p];
-        d.nf = Nf[d.base + m];
-        d.xt = Xt[d.base + m];
-        d.xf = Xf[d.base + m];
-        d.nt = Nt[d.base + m];
-        d.rt = Rt[d.base + m];  // read also without history (then unused)
-        d.rf = Rf[d.base + m];
-        d.ng = Ng[d.base + mg];
-        d.xg = Xg[d.base + mg];
-        d.rg = Rg[d.base + mg];
-    };
-    auto update = [&](const Member& d) {
-        const size_t base = d.base;
-        const T k2 = d.k2;
-        if (tf) snf[r] = d.nf;
-        wave_sync();
-        if (tf) {
-            cpx<T> rf = mk<T>(0, 0);
-#pragma unroll
-            for (int j = 0; j < NC / 2; ++j) rf = rf + cscale(snf[j], brow[j]);
-            const cpx<T> rt = cscale(d.nt, T(2));
-            cpx<T> x1 = d.xt + cscale(rt, a_cur), x2 = d.xf + cscale(rf, a_cur);
-            if (use_prev) {
-                x1 = x1 + cscale(d.rt, a_prev);
-                x2 = x2 + cscale(d.rf, a_prev);
-            }
-            Rt[base + m] = rt;
-            Rf[base + m] = rf;
-            srhs[r] = x1;
-            srhs[Lc + r] = x2;
-        }
-        wave_sync();
-        if (r < nc) {
-            cpx<T> acc = mk<T>(0, 0);
-#pragma unroll
-            for (int j = 0; j < NC; ++j) acc = acc + cscale(srhs[j], crow[j]);
-            const int mm = cls + 2 * (r < Lc ? r : r - Lc);
-            if (r < Lc) Xt[base + mm] = acc;
-            else Xf[base + mm] = acc;
-        }
-        // g: diagonal factors, one vertical mode per lane
-        if (gl) {
-            const T mpi = T(lane + 1) * T(M_PI);
-            const cpx<T> rg = (k2 != T(0)) ? cscale(d.ng, T(-2) * Pr / k2) : mk<T>(0, 0);
-            cpx<T> x3 = d.xg + cscale(rg, a_cur);
-            if (use_prev) x3 = x3 + cscale(d.rg, a_prev);
-            Rg[base + lane] = rg;
-            Xg[base + lane] = (k2 != T(0)) ? cscale(x3, T(1) / (T(1) + dt * Pr * (k2 + mpi * mpi))) : mk<T>(0, 0);
-        }
-        wave_sync();
-    };
-    // Members of a chunk (at most kMaxChunk) two ahead: member mi + 2's loads are in flight while
-    // member mi is computed.  Three register sets taken in turn over a fully unrolled loop, so
-    // that no set is copied (a copy would wait for its loads); loads return in issue order, so
-    // member mi waits for its own only.
-    constexpr int kMaxChunk = 4;
-    Member d[3];
-    if (b0 < b1) fetch(b0, d[0]);
-    if (b0 + 1 < b1) fetch(b0 + 1, d[1]);
-#pragma unroll
-    for (int u = 0; u < kMaxChunk; ++u) {
-        if (b0 + u >= b1) break;
-        if (b0 + u + 2 < b1 && u + 2 < kMaxChunk) fetch(b0 + u + 2, d[(u + 2) % 3]);
-        update(d[u % 3]);
-    }
-    for (int mi = b0 + kMaxChunk; mi < b1; ++mi) {  // longer chunks (the host makes none): in turn
-        Member e;
-        fetch(mi, e);
-        update(e);
-    }
-}
-
-template <typename T, int NC>
-__global__ void __launch_bounds__(256) k_update32(DevGeom g, int nchunk, int L0, int L1, int stride, T Pr, T dt,
-                                                  T a_cur, T a_prev, int use_prev, const int* __restrict__ cgrp,
-                                                  const int* __restrict__ cbeg,
-                                                  const int* __restrict__ gmem, const T* __restrict__ gmat,
-                                                  const T* __restrict__ k2a, cpx<T>* __restrict__ Xt,
-                                                  cpx<T>* __restrict__ Xf, cpx<T>* __restrict__ Xg,
-                                                  const cpx<T>* __restrict__ Nt, const cpx<T>* __restrict__ Nf,
-                                                  const cpx<T>* __restrict__ Ng, cpx<T>* __restrict__ Rt,
-                                                  cpx<T>* __restrict__ Rf, cpx<T>* __restrict__ Rg) {
-    k_update32_body<T, NC>(g, nchunk, L0, L1, stride, Pr, dt, a_cur, a_prev, use_prev, cgrp, cbeg, gmem, gmat, k2a, Xt,
-                       Xf, Xg, Nt, Nf, Ng, Rt, Rf, Rg);
-}
-// one member's arguments of k_update32_batch, which runs the k_update32 body for member
-// blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
-template <typename T>
-struct k_update32_args {
-    DevGeom g;
-    int nchunk;
-    int L0;
-    int L1;
-    int stride;
-    T Pr;
-    T dt;
-    T a_cur;
-    T a_prev;
-    int use_prev;
-    const int* cgrp;
-    const int* cbeg;
-    const int* gmem;
-    const T* gmat;
-    const T* k2a;
-    cpx<T>* Xt;
-    cpx<T>* Xf;
-    cpx<T>* Xg;
-    const cpx<T>* Nt;
-    const cpx<T>* Nf;
-    const cpx<T>* Ng;
-    cpx<T>* Rt;
-    cpx<T>* Rf;
-    cpx<T>* Rg;
-};
-template <typename T, int NC>
-__global__ void __launch_bounds__(256) k_update32_batch(const k_update32_args<T>* __restrict__ tab, int zdim) {
-    const int mb = blockIdx.z / zdim;
-    const k_update32_args<T>& a = tab[mb];
-    k_update32_body<T, NC>(a.g, a.nchunk, a.L0, a.L1, a.stride, a.Pr, a.dt, a.a_cur, a.a_prev, a.use_prev, a.cgrp, a.cbeg,
-                       a.gmem, a.gmat, a.k2a, a.Xt, a.Xf, a.Xg, a.Nt, a.Nf, a.Ng, a.Rt, a.Rf, a.Rg);
-}
-
-
-// F, G: inverse B = 2 Pr (imag 0), implicit factor 1/(1 + dt Pr (m pi)^2) (imag 0); thread m.
-template <typename T>
-__device__ __forceinline__ void update_FG_mode(int m, int L, T Pr, T dt, T a_cur, T a_prev, int use_prev, int mode,
-                                               cpx<T>* XF, cpx<T>* XG, const cpx<T>* NF, const cpx<T>* NG,
-                                               cpx<T>* RF, cpx<T>* RG) {
-    if (m >= L) return;
-    const T mpi = T(m + 1) * T(M_PI);
-    const T fac = T(1) / (T(1) + dt * Pr * mpi * mpi);
-    cpx<T>* X[2] = {XF, XG};
-    const cpx<T>* Nn[2] = {NF, NG};
-    cpx<T>* R[2] = {RF, RG};
-    for (int i = 0; i < 2; ++i) {
-        if (mode == UPD_INVB) {
-            R[i][m] = mk(T(2) * Pr * Nn[i][m].x, T(0));
-        } else if (mode == UPD_IMPLICIT) {
-            X[i][m] = mk(fac * X[i][m].x, T(0));
-        } else {
-            const cpx<T> r = mk(T(2) * Pr * Nn[i][m].x, T(0));
-            cpx<T> x = X[i][m] + cscale(r, a_cur);
-            if (use_prev) x = x + cscale(R[i][m], a_prev);
-            R[i][m] = r;
-            X[i][m] = mk(fac * x.x, T(0));
-        }
-    }
-}
-template <typename T>
-__global__ void k_update_FG(int L, T Pr, T dt, T a_cur, T a_prev, int use_prev, int mode, cpx<T>* XF,
-                            cpx<T>* XG, const cpx<T>* NF, const cpx<T>* NG, cpx<T>* RF, cpx<T>* RG) {
-    update_FG_mode<T>(threadIdx.x, L, Pr, dt, a_cur, a_prev, use_prev, mode, XF, XG, NF, NG, RF, RG);
-}
-
 // make_real (util.cu): on the kx = 0 column set row r (0 < r < N/2) to conj(row N - r), and
 // clear the imaginary part of (0, 0).  Kept rows are symmetric, so source and target are
 // both kept or both removed.
@@ -691,87 +357,6 @@ __global__ void k_make_real(DevGeom g, const int* __restrict__ rows, cpx<T>* X0,
         X[(size_t)kyc * L + m] = conjg(s);
     }
 }
-
-// the end of a time step in one launch: make_real on the blocks before the last, the F, G
-// update (mode UPD_STEP) and the health check on the last block.  A non-finite coefficient
-// anywhere in the state reaches every mode within one nonlinear evaluation (each Fourier mode
-// of a product sums every grid point), so the mean modes theta(0,0), F and G, which the last
-// block reads anyway, show it by the end of the step that consumed it.  health[1] counts the
-// steps; health[0] keeps 1 + the count of the first step that ended non-finite.
-template <typename T>
-__device__ __forceinline__ void k_finish_body(DevGeom g, const int* __restrict__ rows, cpx<T>* X0, cpx<T>* X1,
-                                              cpx<T>* X2, T Pr, T dt, T a_cur, T a_prev, int use_prev, cpx<T>* XF,
-                                              cpx<T>* XG, const cpx<T>* NF, const cpx<T>* NG, cpx<T>* RF,
-                                              cpx<T>* RG, int* __restrict__ health) {
-    if (blockIdx.x == gridDim.x - 1) {
-        update_FG_mode<T>(threadIdx.x, g.L, Pr, dt, a_cur, a_prev, use_prev, UPD_STEP, XF, XG, NF, NG, RF, RG);
-        int bad = 0;
-        if ((int)threadIdx.x < g.L) {
-            const int m = threadIdx.x;
-            // theta(0,0) real parts only: the make_real blocks clear its imaginary parts meanwhile
-            bad = !(isfinite(XF[m].x) && isfinite(XG[m].x) && isfinite(X0[m].x));
-        }
-        bad = __syncthreads_or(bad);
-        if (threadIdx.x == 0) {
-            const int n = health[1];
-            if (bad && health[0] == 0) health[0] = n + 1;
-            health[1] = n + 1;
-        }
-        return;
-    }
-    const int L = g.L, NYc = g.NYc, N = g.N;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= 3 * NYc * L) return;
-    const int fld = e / (NYc * L), rem = e - fld * NYc * L;
-    const int kyc = rem / L, m = rem - kyc * L;
-    cpx<T>* X = fld == 0 ? X0 : (fld == 1 ? X1 : X2);
-    const int row = rows[kyc];
-    if (row == 0) {
-        X[m].y = T(0);
-    } else if (row < N / 2) {
-        const int src = NYc - kyc;
-        const cpx<T> s = X[(size_t)src * L + m];
-        X[(size_t)kyc * L + m] = conjg(s);
-    }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_finish(DevGeom g, const int* __restrict__ rows, cpx<T>* X0, cpx<T>* X1,
-                                                cpx<T>* X2, T Pr, T dt, T a_cur, T a_prev, int use_prev, cpx<T>* XF,
-                                                cpx<T>* XG, const cpx<T>* NF, const cpx<T>* NG, cpx<T>* RF,
-                                                cpx<T>* RG, int* __restrict__ health) {
-    k_finish_body<T>(g, rows, X0, X1, X2, Pr, dt, a_cur, a_prev, use_prev, XF, XG, NF, NG, RF, RG, health);
-}
-// one member's arguments of k_finish_batch, which runs the k_finish body for member
-// blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
-template <typename T>
-struct k_finish_args {
-    DevGeom g;
-    const int* rows;
-    cpx<T>* X0;
-    cpx<T>* X1;
-    cpx<T>* X2;
-    T Pr;
-    T dt;
-    T a_cur;
-    T a_prev;
-    int use_prev;
-    cpx<T>* XF;
-    cpx<T>* XG;
-    const cpx<T>* NF;
-    const cpx<T>* NG;
-    cpx<T>* RF;
-    cpx<T>* RG;
-    int* health;
-};
-template <typename T>
-__global__ void __launch_bounds__(256) k_finish_batch(const k_finish_args<T>* __restrict__ tab, int zdim) {
-    const int mb = blockIdx.z / zdim;
-    const k_finish_args<T>& a = tab[mb];
-    k_finish_body<T>(a.g, a.rows, a.X0, a.X1, a.X2, a.Pr, a.dt, a.a_cur, a.a_prev, a.use_prev, a.XF, a.XG, a.NF, a.NG,
-                     a.RF, a.RG, a.health);
-}
-
 
 // ---------------------------------------------------------------------------------------
 // Device-resident exchange with the reference layout ((M/2+1) x N x L complex, kx fastest,
@@ -2576,51 +2161,10 @@ void Launch<T>::project(const DevGeom& g, const Buffers& b, double Pr, void* con
 }
 
 template <typename T>
-void Launch<T>::update(const DevGeom& g, const Buffers& b, int ngroups, int L0, int L1, int stride, double Pr,
-                       double dt, StepCoef sc, int mode, void* const Xio[3], void* const Nin[3], void* const Rp[3],
-                       hipStream_t s) {
-    if (mode == UPD_STEP && g.L <= 32) {
-#define RBC_UPD32(NCV)                                                                                            \
-    hipLaunchKernelGGL((k_update32<T, NCV>), dim3((b.nchunk + 3) / 4), dim3(256), 0, s, g, b.nchunk, L0, L1,       \
-                       stride, (T)Pr, (T)dt, (T)sc.a_cur, (T)sc.a_prev, sc.use_prev, b.cgrp, b.cbeg, b.gmem,           \
-                       (const T*)b.gmat,                                                                               \
-                       (const T*)b.k2, (cpx<T>*)Xio[0], (cpx<T>*)Xio[1], (cpx<T>*)Xio[2], (const cpx<T>*)Nin[0],       \
-                       (const cpx<T>*)Nin[1], (const cpx<T>*)Nin[2], (cpx<T>*)Rp[0], (cpx<T>*)Rp[1], (cpx<T>*)Rp[2])
-        if (g.L <= 16) RBC_UPD32(16);
-        else RBC_UPD32(32);
-#undef RBC_UPD32
-        return;
-    }
-    const size_t sm = (size_t)3 * g.L * sizeof(cpx<T>);
-    hipLaunchKernelGGL(k_update<T>, dim3(ngroups), dim3(64), sm, s, g, L0, L1, stride, (T)Pr, (T)dt,
-                       (T)sc.a_cur, (T)sc.a_prev, sc.use_prev, mode, b.gstart, b.gmem, (const T*)b.gmat,
-                       (const T*)b.k2, (cpx<T>*)Xio[0], (cpx<T>*)Xio[1], (cpx<T>*)Xio[2], (const cpx<T>*)Nin[0],
-                       (const cpx<T>*)Nin[1], (const cpx<T>*)Nin[2], (cpx<T>*)Rp[0], (cpx<T>*)Rp[1],
-                       (cpx<T>*)Rp[2]);
-}
-
-template <typename T>
-void Launch<T>::update_FG(const DevGeom& g, double Pr, double dt, StepCoef sc, int mode, void* XF, void* XG,
-                          const void* NF, const void* NG, void* RpF, void* RpG, hipStream_t s) {
-    hipLaunchKernelGGL(k_update_FG<T>, dim3(1), dim3(64 * ((g.L + 63) / 64)), 0, s, g.L, (T)Pr, (T)dt,
-                       (T)sc.a_cur, (T)sc.a_prev, sc.use_prev, mode, (cpx<T>*)XF, (cpx<T>*)XG,
-                       (const cpx<T>*)NF, (const cpx<T>*)NG, (cpx<T>*)RpF, (cpx<T>*)RpG);
-}
-
-template <typename T>
 void Launch<T>::make_real(const DevGeom& g, const Buffers& b, void* const X[3], hipStream_t s) {
     const int n = 3 * g.NYc * g.L;
     hipLaunchKernelGGL(k_make_real<T>, dim3((n + 255) / 256), dim3(256), 0, s, g, b.rows, (cpx<T>*)X[0],
                        (cpx<T>*)X[1], (cpx<T>*)X[2]);
-}
-
-template <typename T>
-void Launch<T>::finish(const DevGeom& g, const Buffers& b, double Pr, double dt, StepCoef sc, hipStream_t s) {
-    const int n = 3 * g.NYc * g.L;
-    hipLaunchKernelGGL(k_finish<T>, dim3((n + 255) / 256 + 1), dim3(256), 0, s, g, b.rows, (cpx<T>*)b.X[0],
-                       (cpx<T>*)b.X[1], (cpx<T>*)b.X[2], (T)Pr, (T)dt, (T)sc.a_cur, (T)sc.a_prev, sc.use_prev,
-                       (cpx<T>*)b.XF, (cpx<T>*)b.XG, (const cpx<T>*)b.NF, (const cpx<T>*)b.NG, (cpx<T>*)b.RpF,
-                       (cpx<T>*)b.RpG, b.health);
 }
 
 template <typename T>
@@ -2771,8 +2315,8 @@ struct StepBatch {
     ProjectArgs<float>* ppj = nullptr;
     EvalArgs<float> pev0;  // the first member's, for the launch shape
     ProjectArgs<float> ppj0;
-    k_update32_args<float>* up = nullptr;
-    k_finish_args<float>* fi = nullptr;
+    UpdateArgs<float>* up = nullptr;
+    UpdateArgs<float> up0;
 };
 
 template <typename A>
@@ -2786,7 +2330,7 @@ static A* upload_table(const std::vector<A>& v) {
 void batch_destroy(StepBatch* sb) {
     if (!sb) return;
     for (void* p : {(void*)sb->ev, (void*)sb->yi, (void*)sb->rw, (void*)sb->yf, (void*)sb->pj, (void*)sb->up,
-                    (void*)sb->fi, (void*)sb->pev, (void*)sb->ppj})
+                    (void*)sb->pev, (void*)sb->ppj})
         if (p) hipFree(p);
     delete sb;
 }
@@ -2845,8 +2389,7 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
     std::vector<k_rows_w_args> rw;
     std::vector<k_fft_y_fwd_wc_args> yf;
     std::vector<k_project_mma_args> pj;
-    std::vector<k_update32_args<float>> up;
-    std::vector<k_finish_args<float>> fi;
+    std::vector<UpdateArgs<float>> up;
     for (const BatchMember& x : m) {
         const DevGeom& h = *x.g;
         const Buffers& b = *x.b;
@@ -2867,13 +2410,8 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
         yf.push_back({h, (const C*)b.hout, (const C*)b.twN, (const float*)b.kx, (const float*)b.ky, (C*)b.lev,
                       (C*)b.fgw});
         // AB2 coefficients: a batch only runs members that have their history
-        const float a_cur = (float)(1.5 * x.dt), a_prev = (float)(-0.5 * x.dt);
-        up.push_back({h, b.nchunk, x.L0, x.L1, x.stride, (float)x.Pr, (float)x.dt, a_cur, a_prev, 1, b.cgrp, b.cbeg,
-                      b.gmem, (const float*)b.gmat, (const float*)b.k2, (C*)b.X[0], (C*)b.X[1], (C*)b.X[2],
-                      (const C*)b.Nn[0], (const C*)b.Nn[1], (const C*)b.Nn[2], (C*)b.Rp[0], (C*)b.Rp[1],
-                      (C*)b.Rp[2]});
-        fi.push_back({h, b.rows, (C*)b.X[0], (C*)b.X[1], (C*)b.X[2], (float)x.Pr, (float)x.dt, a_cur, a_prev, 1,
-                      (C*)b.XF, (C*)b.XG, (const C*)b.NF, (const C*)b.NG, (C*)b.RpF, (C*)b.RpG, b.health});
+        up.push_back(update_args<float>(h, b, x.L0, x.L1, x.stride, x.Pr, x.dt, {1.5 * x.dt, -0.5 * x.dt, 1}, b.X, b.Nn,
+                                        b.Rp, b.XF, b.XG, b.NF, b.NG, b.RpF, b.RpG));
         sb->nchunk_max = std::max(sb->nchunk_max, b.nchunk);
     }
     try {
@@ -2889,8 +2427,8 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
         sb->yi = upload_table(yi);
         sb->rw = upload_table(rw);
         sb->yf = upload_table(yf);
+        sb->up0 = up[0];
         sb->up = upload_table(up);
-        sb->fi = upload_table(fi);
     } catch (const HipError&) {
         batch_destroy(sb);
         throw;
@@ -2899,7 +2437,7 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
 }
 
 // One AB2 step of every member, in the stage order of a single step (evaluation, inverse
-// y-FFT, rows, forward y-FFT with the combinations, projection, group update, finish).
+// y-FFT, rows, forward y-FFT with the combinations, projection, group update).
 void batch_step(const StepBatch* sb, hipStream_t s) {
     const DevGeom& g = sb->g;
     const int B = sb->B;
@@ -2961,15 +2499,7 @@ void batch_step(const StepBatch* sb, hipStream_t s) {
     } else {
         launch_project<float>(sb->ppj0, sb->ppj, B, s);
     }
-    {
-        const dim3 gr((sb->nchunk_max + 3) / 4, 1, B);
-        if (g.L <= 16) hipLaunchKernelGGL((k_update32_batch<float, 16>), gr, dim3(256), 0, s, sb->up, 1);
-        else hipLaunchKernelGGL((k_update32_batch<float, 32>), gr, dim3(256), 0, s, sb->up, 1);
-    }
-    {
-        const int n = 3 * g.NYc * g.L;
-        hipLaunchKernelGGL(k_finish_batch<float>, dim3((n + 255) / 256 + 1, 1, B), dim3(256), 0, s, sb->fi, 1);
-    }
+    launch_update<float>(sb->up0, UPD_STEP, sb->up, sb->nchunk_max, B, s);
 }
 
 }  // namespace rbc

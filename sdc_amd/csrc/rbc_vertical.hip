@@ -863,7 +863,9 @@ void launch_project(const ProjectArgs<T>& a, const ProjectArgs<T>* batch, int B,
             return;
         }
     }
-#define RBC_PRP(KSV)                                                                                           if (batch) hipLaunchKernelGGL((k_project_parity_batch<T, KSV>), grid, dim3(64 * KSV), 0, s, batch);        else hipLaunchKernelGGL((k_project_parity<T, KSV>), grid, dim3(64 * KSV), 0, s, a)
+#define RBC_PRP(KSV)                                                                                       \
+    if (batch) hipLaunchKernelGGL((k_project_parity_batch<T, KSV>), grid, dim3(64 * KSV), 0, s, batch);    \
+    else hipLaunchKernelGGL((k_project_parity<T, KSV>), grid, dim3(64 * KSV), 0, s, a)
     // one wave per 16 modes while those fill the chip, else the levels split (us, KS = 1 / 2 / 4): 1024 x 128 x 40
     // FP32 74.4 / 76.2 / 79.0, 256^2 x 24 FP64 32.2 / 29.9 / 34.1, 64^2 x 8 FP64 9.5 / 8.6 / 8.6
     const int work = (a.g.P + 15) / 16 * (int)grid.y;
