@@ -572,23 +572,19 @@ int op_call(rbc_ctx* c, int which, const double* th, const double* f, const doub
 
 // device buffers in the reference layout <-> the context's compact fields, on its stream
 void dev_in(rbc_ctx* c, const void* const f3[3], const void* F, const void* G, void* const X[3], void* XF,
-                   void* XG) {
-    if (c->rsz == 8) Launch<double>::from_ref(c->dg, f3, X, c->stream);
-    else Launch<float>::from_ref(c->dg, f3, X, c->stream);
+                   void* XG, int* health = nullptr) {
+    const VecPair vec{F, G, XF, XG, health};
+    if (c->rsz == 8) Launch<double>::from_ref(c->dg, f3, X, vec, c->stream);
+    else Launch<float>::from_ref(c->dg, f3, X, vec, c->stream);
     HIPCHK(hipGetLastError());
-    const size_t vb = (size_t)c->dg.L * c->csz();
-    if (F) HIPCHK(hipMemcpyAsync(XF, F, vb, hipMemcpyDeviceToDevice, c->stream));
-    if (G) HIPCHK(hipMemcpyAsync(XG, G, vb, hipMemcpyDeviceToDevice, c->stream));
 }
 
 void dev_out(rbc_ctx* c, void* const X[3], const void* XF, const void* XG, void* const f3[3], void* F,
                     void* G) {
-    if (c->rsz == 8) Launch<double>::to_ref(c->dg, X, f3, c->stream);
-    else Launch<float>::to_ref(c->dg, X, f3, c->stream);
+    const VecPair vec{XF, XG, F, G, nullptr};
+    if (c->rsz == 8) Launch<double>::to_ref(c->dg, X, f3, vec, c->stream);
+    else Launch<float>::to_ref(c->dg, X, f3, vec, c->stream);
     HIPCHK(hipGetLastError());
-    const size_t vb = (size_t)c->dg.L * c->csz();
-    if (F) HIPCHK(hipMemcpyAsync(F, XF, vb, hipMemcpyDeviceToDevice, c->stream));
-    if (G) HIPCHK(hipMemcpyAsync(G, XG, vb, hipMemcpyDeviceToDevice, c->stream));
 }
 
 int op_call_device(rbc_ctx* c, int which, const void* th, const void* f, const void* g, const void* F,
@@ -632,8 +628,8 @@ int rbc_set_state_device(rbc_ctx* c, const void* th, const void* f, const void* 
     try {
         hipSetDevice(c->p.device);
         const void* in3[3] = {th, f, g};
-        dev_in(c, in3, F, G, c->b.X, c->b.XF, c->b.XG);
-        clear_health(c);
+        dev_in(c, in3, F, G, c->b.X, c->b.XF, c->b.XG, c->b.health);
+        c->bad_step = 0;
     } catch (const HipError& e) {
         return hip_fail(c, e);
     }

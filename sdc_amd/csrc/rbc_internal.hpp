@@ -185,6 +185,14 @@ void field_to_ref64(const DevGeom& g, int rsz, const void* src, void* ref, hipSt
 void vertical_tables(int L, int nq, int PS, bool f64, const std::vector<double>& ev, const std::vector<double>& pr,
                    std::vector<double>& evP, std::vector<double>& prP);
 
+// the L-vectors that go with an exchange of the three fields (null: not copied), and the health word
+// to clear (null: none)
+struct VecPair {
+    const void *F = nullptr, *G = nullptr;
+    void *oF = nullptr, *oG = nullptr;
+    int* health = nullptr;
+};
+
 template <typename T>
 struct Launch {
     // stage 1: vertical evaluation -> six level fields (spectral)
@@ -204,9 +212,11 @@ struct Launch {
     static void nusselt(const DevGeom& g, const Buffers& b, const void* ia1, hipStream_t s);
     // device fields in the reference layout ((M/2+1) x N x L, T complex) -> compact [p][m]
     // (kept modes); null source fields are skipped
-    static void from_ref(const DevGeom& g, const void* const src[3], void* const dst[3], hipStream_t s);
+    static void from_ref(const DevGeom& g, const void* const src[3], void* const dst[3], const VecPair& vec,
+                         hipStream_t s);
     // compact [p][m] -> reference layout with zeros in the removed band; null targets skipped
-    static void to_ref(const DevGeom& g, const void* const src[3], void* const dst[3], hipStream_t s);
+    static void to_ref(const DevGeom& g, const void* const src[3], void* const dst[3], const VecPair& vec,
+                       hipStream_t s);
     // initial state of the context's X, XF, XG (kind: 0 zeros, 1 random theta, 2 init_test)
     static void init_state(const DevGeom& g, const Buffers& b, int kind, uint64_t seed, double amp, hipStream_t s);
     // the real plane of an initial pattern (util/init.cu), [row][col] of M x N, in the real type

@@ -378,12 +378,28 @@ __device__ __forceinline__ int kept_index_of(const DevGeom& g, int row) {  // -1
     return row <= a ? row : (row >= g.N - a ? g.NYc - (g.N - row) : -1);
 }
 
+// The L-vectors F and G ride along on block (0, 0, 0) (null: none), and with them the health word that
+// a new state clears: copies and a clear of their own cost 3 to 4 us each, beside 5 us for the fields
+// of a 128^2 x 16 state (operators at 512 x 128 x 11, twelve vectors a pass: 160 -> 136 us).
+template <typename T, typename TD>
+__device__ __forceinline__ void exchange_vecs(int L, const VecPair& v) {
+    if (blockIdx.x + blockIdx.y + blockIdx.z != 0) return;
+    for (int i = threadIdx.x; i < 4 * L; i += blockDim.x) {
+        const int j = i < 2 * L ? i : i - 2 * L;
+        const T* s = (const T*)(i < 2 * L ? v.F : v.G);
+        TD* d = (TD*)(i < 2 * L ? v.oF : v.oG);
+        if (s && d) d[j] = (TD)s[j];
+    }
+    if (threadIdx.x == 0 && v.health) v.health[0] = 0;
+}
+
 template <typename T, typename TD = T>
 __global__ void __launch_bounds__(256) k_ref_to_compact(DevGeom g, const cpx<T>* __restrict__ s0,
                                                         const cpx<T>* __restrict__ s1, const cpx<T>* __restrict__ s2,
                                                         cpx<TD>* __restrict__ d0, cpx<TD>* __restrict__ d1,
-                                                        cpx<TD>* __restrict__ d2) {
+                                                        cpx<TD>* __restrict__ d2, VecPair vec) {
     __shared__ cpx<T> tile[32][33];  // [m][kx]
+    exchange_vecs<T, TD>(g.L, vec);
     const int mtn = (g.L + 31) / 32, fld = blockIdx.z / mtn, m0 = (blockIdx.z - fld * mtn) * 32;
     const cpx<T>* src = fld == 0 ? s0 : (fld == 1 ? s1 : s2);
     cpx<TD>* dst = fld == 0 ? d0 : (fld == 1 ? d1 : d2);
@@ -411,8 +427,9 @@ template <typename T, typename TD = T>
 __global__ void __launch_bounds__(256) k_compact_to_ref(DevGeom g, const cpx<T>* __restrict__ s0,
                                                         const cpx<T>* __restrict__ s1, const cpx<T>* __restrict__ s2,
                                                         cpx<TD>* __restrict__ d0, cpx<TD>* __restrict__ d1,
-                                                        cpx<TD>* __restrict__ d2) {
+                                                        cpx<TD>* __restrict__ d2, VecPair vec) {
     __shared__ cpx<TD> tile[32][33];  // [kx][m]
+    exchange_vecs<T, TD>(g.L, vec);
     const int mtn = (g.L + 31) / 32, fld = blockIdx.z / mtn, m0 = (blockIdx.z - fld * mtn) * 32;
     const cpx<T>* src = fld == 0 ? s0 : (fld == 1 ? s1 : s2);
     cpx<TD>* dst = fld == 0 ? d0 : (fld == 1 ? d1 : d2);
@@ -2175,19 +2192,21 @@ void Launch<T>::nusselt(const DevGeom& g, const Buffers& b, const void* ia1, hip
 }
 
 template <typename T>
-void Launch<T>::from_ref(const DevGeom& g, const void* const src[3], void* const dst[3], hipStream_t s) {
+void Launch<T>::from_ref(const DevGeom& g, const void* const src[3], void* const dst[3], const VecPair& vec,
+                         hipStream_t s) {
     const int mtn = (g.L + 31) / 32;
     hipLaunchKernelGGL(k_ref_to_compact<T>, dim3((g.KX + 31) / 32, g.NYc, 3 * mtn), dim3(256), 0, s, g,
                        (const cpx<T>*)src[0], (const cpx<T>*)src[1], (const cpx<T>*)src[2], (cpx<T>*)dst[0],
-                       (cpx<T>*)dst[1], (cpx<T>*)dst[2]);
+                       (cpx<T>*)dst[1], (cpx<T>*)dst[2], vec);
 }
 
 template <typename T>
-void Launch<T>::to_ref(const DevGeom& g, const void* const src[3], void* const dst[3], hipStream_t s) {
+void Launch<T>::to_ref(const DevGeom& g, const void* const src[3], void* const dst[3], const VecPair& vec,
+                       hipStream_t s) {
     const int mtn = (g.L + 31) / 32;
     hipLaunchKernelGGL(k_compact_to_ref<T>, dim3((g.M / 2 + 1 + 31) / 32, g.N, 3 * mtn), dim3(256), 0, s, g,
                        (const cpx<T>*)src[0], (const cpx<T>*)src[1], (const cpx<T>*)src[2], (cpx<T>*)dst[0],
-                       (cpx<T>*)dst[1], (cpx<T>*)dst[2]);
+                       (cpx<T>*)dst[1], (cpx<T>*)dst[2], vec);
 }
 
 // one field between an FP64 reference-layout buffer and the compact field of the context's real
@@ -2197,20 +2216,20 @@ void field_from_ref64(const DevGeom& g, int rsz, const void* ref, void* dst, hip
     const dim3 grid((g.KX + 31) / 32, g.NYc, mtn);
     if (rsz == 8)
         hipLaunchKernelGGL((k_ref_to_compact<double, double>), grid, dim3(256), 0, s, g, (const cpx<double>*)ref,
-                           nullptr, nullptr, (cpx<double>*)dst, nullptr, nullptr);
+                           nullptr, nullptr, (cpx<double>*)dst, nullptr, nullptr, VecPair{});
     else
         hipLaunchKernelGGL((k_ref_to_compact<double, float>), grid, dim3(256), 0, s, g, (const cpx<double>*)ref,
-                           nullptr, nullptr, (cpx<float>*)dst, nullptr, nullptr);
+                           nullptr, nullptr, (cpx<float>*)dst, nullptr, nullptr, VecPair{});
 }
 void field_to_ref64(const DevGeom& g, int rsz, const void* src, void* ref, hipStream_t s) {
     const int mtn = (g.L + 31) / 32;
     const dim3 grid((g.M / 2 + 1 + 31) / 32, g.N, mtn);
     if (rsz == 8)
         hipLaunchKernelGGL((k_compact_to_ref<double, double>), grid, dim3(256), 0, s, g, (const cpx<double>*)src,
-                           nullptr, nullptr, (cpx<double>*)ref, nullptr, nullptr);
+                           nullptr, nullptr, (cpx<double>*)ref, nullptr, nullptr, VecPair{});
     else
         hipLaunchKernelGGL((k_compact_to_ref<float, double>), grid, dim3(256), 0, s, g, (const cpx<float>*)src,
-                           nullptr, nullptr, (cpx<double>*)ref, nullptr, nullptr);
+                           nullptr, nullptr, (cpx<double>*)ref, nullptr, nullptr, VecPair{});
 }
 
 template <typename T>
