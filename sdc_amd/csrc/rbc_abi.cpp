@@ -716,8 +716,8 @@ int rbc_set_penalization(rbc_ctx* c, double eta, int shape, const double* mask) 
         upload_reals(c, pen.ia2, ia2);
         // work arrays: the level-space buffers when they are large enough (the penalty runs after
         // the projection has consumed them), else arrays of their own
-        const size_t cs = c->csz(), spec = (size_t)10 * g.L * g.P * cs, hyb = (size_t)10 * g.L * g.N * g.KXp * cs;
-        const bool reuse = 10 * g.L <= 6 * g.nq;
+        const size_t cs = c->csz(), spec = (size_t)7 * g.L * g.PS * cs, hyb = (size_t)7 * g.L * g.N * g.KXp * cs;
+        const bool reuse = 7 * g.L <= 6 * g.nq;
         pen.spec = reuse ? c->b.lev : al(spec);
         pen.spec_out = reuse ? c->b.prod : al(spec);
         pen.hin = reuse ? c->b.hin : al(hyb);

@@ -150,10 +150,10 @@ struct Penalty {
     void* mask = nullptr;    // M * N reals, x fastest
     void* iac = nullptr;     // L * L reals, Iac(j, k) at j + k L (coeff.cu:77-116, quirk kept)
     void* ia2 = nullptr;     // L * L reals, Ia2(i, j) = <C_i S'_j> at i + j L
-    void* spec = nullptr;    // [10][L][P] complex: the mode-space fields before the transforms
-    void* hin = nullptr;     // [10][L][N][KXp] complex (row-major hybrid rows)
+    void* spec = nullptr;    // [7][L][PS] complex: the mode-space fields before the transforms
+    void* hin = nullptr;     // [7][L][N][KXp] complex (row-major hybrid rows)
     void* hout = nullptr;    // same, after the mask products
-    void* spec_out = nullptr;  // [10][L][P] complex: the transforms of the mask products
+    void* spec_out = nullptr;  // [7][L][PS] complex: the transforms of the mask products
 };
 
 // Ia2(i, j) = <C_i S'_j> by a 4 L + 64 point Gauss-Legendre rule (coeff.cu's ra2), i + j L.

@@ -512,75 +512,108 @@ __global__ void k_force_mean(cpx<T>* XF, double v) {
 // ---------------------------------------------------------------------------------------
 // Penalization (PENALIZED builds, nonlinear_operator_rayleigh_noslip.cu:1097-1343).  The mask
 // chi(x, y) does not depend on z, so every sum over the source mode j of a summand commutes with
-// the mask product and the transforms: the summands need, per output mode k, the transforms
-// H = R2C(chi u / (M N)) of ten mode-space fields u (the reference forms six per j and sums
-// after the transforms):
-//   0: i kx a_k, 1: i ky a_k                 a_k = sum_j Iac(j, k) f_j   (f summands 1, 3)
-//   2: i ky b_k + bF_k d_k0,                 b_k = sum_j Ia2(k, j) g_j, bF_k, bG_k from F, G
-//   3: -i kx b_k + bG_k d_k0                                             (f summands 2, 4)
-//   4: k^2 f_k                                                           (f summand 5)
-//   5: i kx c_k, 6: i ky c_k                 c_k = sum_j Ia2(j, k) f_j   (g 1, 3; F, G 1)
-//   7: i ky g_k + F_k d_k0, 8: -i kx g_k + G_k d_k0   (u12_k, u22_k: g 2, 4; F, G 2)
-//   9: theta_k                                                           (theta)
+// the mask product and the transforms, and so do the sums over summands: per output mode k the
+// transforms H = R2C(chi u / (M N)) of seven mode-space fields u are enough (the reference forms six
+// per j and sums after the transforms):
+//   0: i kx a_k + i ky b_k + bF_k d_k0       a_k = sum_j Iac(j, k) f_j    (f summands 1 to 4)
+//   1: i ky a_k - i kx b_k + bG_k d_k0       b_k = sum_j Ia2(k, j) g_j, bF_k, bG_k from F, G
+//   2: k^2 f_k                                                            (f summand 5)
+//   3: i kx c_k - (i ky g_k + F_k d_k0) / 2  c_k = sum_j Ia2(j, k) f_j    (g 1, 2; F)
+//   4: i ky c_k                                                           (g 3; G)
+//   5: -i kx g_k + G_k d_k0                                               (g 4; G)
+//   6: theta_k                                                            (theta)
 // (d_k0: at kx = ky = 0 only, add_dc_part).  After the mask products and the transforms:
-//   N_theta += -(1/(2 eta)) H9
-//   N_f     += -(1/eta) (i kx (H0 + H2) + i ky (H1 + H3) + k^2 H4)
-//   N_g     += -(1/eta) (-i ky H5 + i kx H6 + i ky (H7 - H8) / 2)   (summand 4 is d_y, as there)
-//   N_F     += -(1/eta) (-H5 + H7 / 2) at k = 0,  N_G += -(1/eta) (-H6 + H8 / 2) at k = 0
-// which are the reference's summands scaled by -1 (theta) and -1/Pr (:1366-1370).
+//   N_theta += -(1/(2 eta)) H6
+//   N_f     += -(1/eta) (i kx H0 + i ky H1 + k^2 H2)
+//   N_g     += -(1/eta) (-i ky H3 + i kx H4 - i ky H5 / 2)   (summand 4 is d_y, as there)
+//   N_F     += (1/eta) H3 at k = 0,  N_G += (1/eta) (H4 - H5 / 2) at k = 0
+// which are the reference's summands scaled by -1 (theta) and -1/Pr (:1366-1370).  Summed before the
+// transforms the ten distinct fields become seven, and so do the four transforms' passes over them.
+// At 256 x 128 x 20 FP32, us a step: fields 35 -> 12, inverse y 18 -> 7, mask rows 47 -> 11,
+// forward y 19 -> 8, combination 6.7 -> 8.7.
 // ---------------------------------------------------------------------------------------
+constexpr int kPenFields = 7;
+
+// Block: 64 Fourier modes (lanes) x 8 output modes k (two per wave).  f and g are staged in LDS
+// sixteen source modes at a time (read in runs of 16 values), the matrix entries are wave-uniform.
 template <typename T>
 __global__ void __launch_bounds__(256) k_pen_fields(DevGeom g, const T* __restrict__ iac, const T* __restrict__ ia2,
                                                     const cpx<T>* __restrict__ Xt, const cpx<T>* __restrict__ Xf,
                                                     const cpx<T>* __restrict__ Xg, const cpx<T>* __restrict__ XF,
                                                     const cpx<T>* __restrict__ XG, const T* __restrict__ kxa,
                                                     const T* __restrict__ kya, cpx<T>* __restrict__ out) {
+    __shared__ cpx<T> sf[16][65], sg[16][65];
     const int L = g.L, P = g.P;
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)L * P) return;
-    const int k = (int)(e / P), p = (int)(e % P);
-    const cpx<T>* f = Xf + (size_t)p * L;
-    const cpx<T>* gg = Xg + (size_t)p * L;
-    cpx<T> a = mk(T(0), T(0)), b = a, c = a, bF = a, bG = a;
-    for (int j = 0; j < L; ++j) {
-        const T cac = iac[j + (size_t)k * L], ckj = ia2[k + (size_t)j * L], cjk = ia2[j + (size_t)k * L];
-        const cpx<T> fj = f[j], gj = gg[j];
-        a = a + cscale(fj, cac);
-        b = b + cscale(gj, ckj);
-        c = c + cscale(fj, cjk);
-        if (p == 0) {
-            bF = bF + cscale(XF[j], ckj);
-            bG = bG + cscale(XG[j], ckj);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p0 = blockIdx.x * 64, p = min(p0 + lane, P - 1), k0 = blockIdx.y * 8 + 2 * wave;
+    cpx<T> a[2], b[2], c[2], bF[2], bG[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a[i] = b[i] = c[i] = bF[i] = bG[i] = mk(T(0), T(0));
+    for (int j0 = 0; j0 < L; j0 += 16) {
+        __syncthreads();
+        for (int e = threadIdx.x; e < 64 * 16; e += 256) {
+            const int pp = e >> 4, jj = e & 15;
+            const size_t at = (size_t)min(p0 + pp, P - 1) * L + min(j0 + jj, L - 1);
+            const cpx<T> f = Xf[at], gg = Xg[at];
+            const bool in = j0 + jj < L;
+            sf[jj][pp] = mk(in ? f.x : T(0), in ? f.y : T(0));
+            sg[jj][pp] = mk(in ? gg.x : T(0), in ? gg.y : T(0));
+        }
+        __syncthreads();
+        const int jn = min(16, (L - j0 + 3) & ~3);  // zeros beyond L
+#pragma unroll 4
+        for (int jj = 0; jj < jn; ++jj) {
+            const int j = min(j0 + jj, L - 1);
+            const cpx<T> fj = sf[jj][lane], gj = sg[jj][lane];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int k = min(k0 + i, L - 1);
+                a[i] = a[i] + cscale(fj, iac[j + (size_t)k * L]);
+                b[i] = b[i] + cscale(gj, ia2[k + (size_t)j * L]);
+                c[i] = c[i] + cscale(fj, ia2[j + (size_t)k * L]);
+            }
         }
     }
-    const T kx = kxa[p], ky = kya[p];
-    const cpx<T> fk = f[k], gk = gg[k];
-    cpx<T> v[10];
-    v[0] = imul(a, kx);
-    v[1] = imul(a, ky);
-    v[2] = imul(b, ky);
-    v[3] = imul(b, -kx);
-    v[4] = cscale(fk, kx * kx + ky * ky);
-    v[5] = imul(c, kx);
-    v[6] = imul(c, ky);
-    v[7] = imul(gk, ky);
-    v[8] = imul(gk, -kx);
-    v[9] = Xt[(size_t)p * L + k];
-    if (p == 0) {
-        v[2] = v[2] + bF;
-        v[3] = v[3] + bG;
-        v[7] = v[7] + XF[k];
-        v[8] = v[8] + XG[k];
-    }
-    const size_t fs = (size_t)L * P;
+    if (p0 == 0)  // only lane 0 (p = 0) uses these
+        for (int j = 0; j < L; ++j)
 #pragma unroll
-    for (int q = 0; q < 10; ++q) out[q * fs + e] = v[q];
+            for (int i = 0; i < 2; ++i) {
+                const T ckj = ia2[min(k0 + i, L - 1) + (size_t)j * L];
+                bF[i] = bF[i] + cscale(XF[j], ckj);
+                bG[i] = bG[i] + cscale(XG[j], ckj);
+            }
+    if (p0 + lane >= P) return;
+    const T kx = kxa[p], ky = kya[p];
+    const size_t fs = (size_t)L * g.PS;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int k = k0 + i;
+        if (k >= L) break;
+        const cpx<T> fk = Xf[(size_t)p * L + k], gk = Xg[(size_t)p * L + k];
+        cpx<T> v[kPenFields];
+        v[0] = imul(a[i], kx) + imul(b[i], ky);
+        v[1] = imul(a[i], ky) + imul(b[i], -kx);
+        v[2] = cscale(fk, kx * kx + ky * ky);
+        v[3] = imul(c[i], kx) + imul(gk, T(-0.5) * ky);
+        v[4] = imul(c[i], ky);
+        v[5] = imul(gk, -kx);
+        v[6] = Xt[(size_t)p * L + k];
+        if (p == 0) {
+            v[0] = v[0] + bF[i];
+            v[1] = v[1] + bG[i];
+            v[3] = v[3] + cscale(XF[k], T(-0.5));
+            v[5] = v[5] + XG[k];
+        }
+        const size_t e = (size_t)k * g.PS + p;
+#pragma unroll
+        for (int q = 0; q < kPenFields; ++q) out[q * fs + e] = v[q];
+    }
 }
 
-// one (y row, mode k, field group) per block: the group's one or two hybrid rows as one complex
-// M-point transform (X1 + i X2, the kx = 0 imaginary parts dropped as a C2R does), the product
-// with chi(x, y) / (M N), the forward transform and the unpacking to kx < KX.  Groups pair
-// fields of like size: (0, 1), (2, 3), (5, 6), (7, 8), (4), (9).
+// one (row pair y, y + 1, mode k, field) per block, grid sizes outside k_rows_mask_w: the two hybrid
+// rows as one complex M-point transform (X1 + i X2, the kx = 0 imaginary parts dropped as a C2R does),
+// the product with chi(x, y) / (M N), the forward transform and the unpacking to kx < KX.  The pair is
+// two rows of one field, so both are of like size.
 template <typename T>
 __global__ void __launch_bounds__(256) k_rows_mask(DevGeom g, const T* __restrict__ mask,
                                                    const cpx<T>* __restrict__ hin, const cpx<T>* __restrict__ twM,
@@ -588,17 +621,13 @@ __global__ void __launch_bounds__(256) k_rows_mask(DevGeom g, const T* __restric
     extern __shared__ unsigned char smem_raw[];
     cpx<T>* a = reinterpret_cast<cpx<T>*>(smem_raw);
     cpx<T>* bb = a + g.M;
-    const int M = g.M, N = g.N, KX = g.KX, KXp = g.KXp, L = g.L;
-    const int y = blockIdx.x, k = blockIdx.y, grp = blockIdx.z;
-    const int f1 = grp < 4 ? (grp == 0 ? 0 : grp == 1 ? 2 : grp == 2 ? 5 : 7) : (grp == 4 ? 4 : 9);
-    const int f2 = grp < 4 ? f1 + 1 : -1;
-    const size_t fstride = (size_t)L * N * KXp;
-    const size_t roff = ((size_t)k * N + y) * KXp;
+    const int M = g.M, N = g.N, KX = g.KX, KXp = g.KXp;
+    const int y = 2 * blockIdx.x;
+    const size_t off = (((size_t)blockIdx.z * g.L + blockIdx.y) * N + y) * KXp;
     for (int e = threadIdx.x; e < M; e += blockDim.x) a[e] = mk(T(0), T(0));
     __syncthreads();
     for (int kk = threadIdx.x; kk < KX; kk += blockDim.x) {
-        cpx<T> x1 = hin[(size_t)f1 * fstride + roff + kk];
-        cpx<T> x2 = f2 >= 0 ? hin[(size_t)f2 * fstride + roff + kk] : mk(T(0), T(0));
+        cpx<T> x1 = hin[off + kk], x2 = hin[off + KXp + kk];
         if (kk == 0) {
             x1.y = T(0);
             x2.y = T(0);
@@ -609,39 +638,59 @@ __global__ void __launch_bounds__(256) k_rows_mask(DevGeom g, const T* __restric
     __syncthreads();
     cpx<T>* r = lds_fft(a, bb, g.logM, 1, twM, true);
     const T s = T(1) / (T(M) * T(N));
-    for (int x = threadIdx.x; x < M; x += blockDim.x) r[x] = cscale(r[x], s * mask[(size_t)y * M + x]);
+    for (int x = threadIdx.x; x < M; x += blockDim.x)
+        r[x] = mk(r[x].x * (s * mask[(size_t)y * M + x]), r[x].y * (s * mask[(size_t)(y + 1) * M + x]));
     __syncthreads();
     cpx<T>* R = lds_fft(r, r == a ? bb : a, g.logM, 1, twM, false);
     for (int kk = threadIdx.x; kk < KX; kk += blockDim.x) {
         const cpx<T> zk = R[kk], zm = R[(M - kk) & (M - 1)];
-        hout[(size_t)f1 * fstride + roff + kk] = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
-        if (f2 >= 0) hout[(size_t)f2 * fstride + roff + kk] = mk(T(0.5) * (zk.y + zm.y), T(-0.5) * (zk.x - zm.x));
+        hout[off + kk] = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
+        hout[off + KXp + kk] = mk(T(0.5) * (zk.y + zm.y), T(-0.5) * (zk.x - zm.x));
     }
 }
 
+// Block: 64 Fourier modes x 8 vertical modes; the transforms are read with the Fourier modes along
+// the lanes and the sums added to N in runs of 8 vertical modes (through LDS).
 template <typename T>
 __global__ void __launch_bounds__(256) k_pen_combine(DevGeom g, T ie, const cpx<T>* __restrict__ H,
                                                      const T* __restrict__ kxa, const T* __restrict__ kya,
                                                      cpx<T>* __restrict__ Nt, cpx<T>* __restrict__ Nf,
                                                      cpx<T>* __restrict__ Ng, cpx<T>* __restrict__ NF,
                                                      cpx<T>* __restrict__ NG) {
+    __shared__ cpx<T> tile[3][64][9];
     const int L = g.L, P = g.P;
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)L * P) return;
-    const int p = (int)(e / L), k = (int)(e % L);
-    const size_t fs = (size_t)L * P, at = (size_t)k * P + p;
-    cpx<T> h[10];
-#pragma unroll
-    for (int q = 0; q < 10; ++q) h[q] = H[q * fs + at];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p0 = blockIdx.x * 64, p = min(p0 + lane, P - 1), k0 = blockIdx.y * 8;
+    const size_t fs = (size_t)L * g.PS;
     const T kx = kxa[p], ky = kya[p];
-    const cpx<T> ft = imul(h[0] + h[2], kx) + imul(h[1] + h[3], ky) + cscale(h[4], kx * kx + ky * ky);
-    const cpx<T> gt = imul(h[5], -ky) + imul(h[6], kx) + imul(h[7] - h[8], T(0.5) * ky);
-    Nt[e] = Nt[e] + cscale(h[9], T(-0.5) * ie);
-    Nf[e] = Nf[e] + cscale(ft, -ie);
-    Ng[e] = Ng[e] + cscale(gt, -ie);
-    if (p == 0) {
-        NF[k] = NF[k] + cscale(cscale(h[7], T(0.5)) - h[5], -ie);
-        NG[k] = NG[k] + cscale(cscale(h[8], T(0.5)) - h[6], -ie);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int k = k0 + 2 * wave + i;
+        if (k >= L) break;
+        cpx<T> h[kPenFields];
+#pragma unroll
+        for (int q = 0; q < kPenFields; ++q) h[q] = H[q * fs + (size_t)k * g.PS + p];
+        const cpx<T> ft = imul(h[0], kx) + imul(h[1], ky) + cscale(h[2], kx * kx + ky * ky);
+        const cpx<T> gt = imul(h[3], -ky) + imul(h[4], kx) + imul(h[5], T(-0.5) * ky);
+        tile[0][lane][2 * wave + i] = cscale(h[6], T(-0.5) * ie);
+        tile[1][lane][2 * wave + i] = cscale(ft, -ie);
+        tile[2][lane][2 * wave + i] = cscale(gt, -ie);
+        if (p0 + lane == 0) {
+            NF[k] = NF[k] + cscale(h[3], ie);
+            NG[k] = NG[k] + cscale(h[4] + cscale(h[5], T(-0.5)), ie);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+        cpx<T>* Nn = f == 0 ? Nt : (f == 1 ? Nf : Ng);
+        for (int e = threadIdx.x; e < 64 * 8; e += 256) {
+            const int pp = p0 + (e >> 3), k = k0 + (e & 7);
+            if (pp < P && k < L) {
+                const size_t at = (size_t)pp * L + k;
+                Nn[at] = Nn[at] + tile[f][e >> 3][e & 7];
+            }
+        }
     }
 }
 
@@ -1193,6 +1242,66 @@ __global__ void __launch_bounds__(64 * WPB) k_rows_w(DevGeom g, const cpx<T>* __
                                                 const cpx<T>* __restrict__ twM, cpx<T>* __restrict__ hout) {
     k_rows_w_body<T, LOGM, WPB>(g, hin, twM, hout);
 }
+// The penalization's rows: the hybrid rows y and y + 1 of one field and mode as X1 + i X2 (as
+// k_rows_mask), times chi / (M N), and back, in the registers of a group of M / E lanes; the rows of all
+// fields and modes in one flat range of pairs (pairs past its end are computed on the last one and not
+// stored).  Bound by memory at large grids, 2 x 7 L N KX values and the mask.
+template <typename T, int LOGM, int WPB>
+__global__ void __launch_bounds__(64 * WPB) k_rows_mask_w(DevGeom g, int npair, const T* __restrict__ mask,
+                                                          const cpx<T>* __restrict__ hin,
+                                                          const cpx<T>* __restrict__ twM, cpx<T>* __restrict__ hout) {
+    using R = RowShape<T, LOGM, WPB>;
+    constexpr int M = R::M, E = R::E, W = R::W, G = R::G, RPB = R::RPB, KX = kept_cols(M);
+    __shared__ cpx<T> tw[M];
+    __shared__ cpx<T> scr[RPB][R::SP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
+    const int KXp = g.KXp;
+    const int pr0 = blockIdx.x * RPB + wave * G + grp, pr = min(pr0, npair - 1);
+    const int y = (2 * pr) & (g.N - 1);
+    const cpx<T>* x1 = hin + (size_t)(2 * pr) * KXp;
+    const cpx<T>* x2 = x1 + KXp;
+    cpx<T> v[1][E];
+    T m1[E], m2[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int k = j + W * r;
+        const int src = k < KX ? k : (k > M - KX ? M - k : -1);
+        cpx<T> a = mk(T(0), T(0)), b = a;
+        if (src >= 0) {
+            a = x1[src];
+            b = x2[src];
+            if (src == 0) a.y = b.y = T(0);
+        }
+        v[0][r] = k < KX ? mk(a.x - b.y, a.y + b.x) : mk(a.x + b.y, -a.y + b.x);
+        m1[r] = mask[(size_t)y * M + k];
+        m2[r] = mask[(size_t)(y + 1) * M + k];
+    }
+    for (int e = threadIdx.x; e < M; e += blockDim.x) tw[e] = twM[e];
+    __syncthreads();
+    cpx<T>* sb = scr[wave * G + grp];
+    fft_group<LOGM, true, 1>(v, sb, tw, j);
+    const T s = T(1) / (T(M) * T(g.N));
+#pragma unroll
+    for (int r = 0; r < E; ++r) v[0][r] = mk(v[0][r].x * (s * m1[r]), v[0][r].y * (s * m2[r]));
+    wave_sync();
+    fft_group<LOGM, false, 1>(v, sb, tw, j);
+    wave_sync();
+#pragma unroll
+    for (int r = 0; r < E; ++r) sb[pad8(j + W * r)] = v[0][r];
+    wave_sync();
+    cpx<T>* o1 = hout + (size_t)(2 * pr) * KXp;
+    cpx<T>* o2 = o1 + KXp;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int k = j + W * r;
+        if (k < KX && pr0 < npair) {
+            const cpx<T> zk = v[0][r], zm = sb[pad8((M - k) & (M - 1))];
+            o1[k] = mk(T(0.5) * (zk.x + zm.x), T(0.5) * (zk.y - zm.y));
+            o2[k] = mk(T(0.5) * (zk.y + zm.y), T(-0.5) * (zk.x - zm.x));
+        }
+    }
+}
+
 // one member's arguments of k_rows_w_batch, which runs the k_rows_w body for member
 // blockIdx.z / zdim of a batch (the rest of blockIdx.z is the body's own z index)
 struct k_rows_w_args {
@@ -2244,29 +2353,57 @@ void Launch<T>::force_mean(const Buffers& b, double v, hipStream_t s) {
     hipLaunchKernelGGL(k_force_mean<T>, dim3(1), dim3(64), 0, s, (cpx<T>*)b.XF, v);
 }
 
+template <typename T, int LOGM>
+static void launch_rows_mask(const DevGeom& g, const Penalty& pen, const void* twM, hipStream_t s) {
+    constexpr int WPB = RowShape<T, LOGM, 4>::lds <= 65536 ? 4 : 2;
+    static_assert(RowShape<T, LOGM, WPB>::lds <= 65536, "row pair tile");
+    constexpr int RPB = RowShape<T, LOGM, WPB>::RPB;
+    const int npair = kPenFields * g.L * (g.N / 2);
+    hipLaunchKernelGGL((k_rows_mask_w<T, LOGM, WPB>), dim3((npair + RPB - 1) / RPB), dim3(64 * WPB), 0, s, g, npair,
+                       (const T*)pen.mask, (const cpx<T>*)pen.hin, (const cpx<T>*)twM, (cpx<T>*)pen.hout);
+}
+
 template <typename T>
 void Launch<T>::penalty(const DevGeom& g, const Buffers& b, const Penalty& pen, double Pr, void* const X[3],
                         const void* XF, const void* XG, void* const Nout[3], void* NF, void* NG, hipStream_t s) {
     (void)Pr;
-    const size_t n = (size_t)g.L * g.P;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_pen_fields<T>, dim3(nb), dim3(256), 0, s, g, (const T*)pen.iac, (const T*)pen.ia2,
+    const dim3 gm((g.P + 63) / 64, (g.L + 7) / 8);
+    hipLaunchKernelGGL(k_pen_fields<T>, gm, dim3(256), 0, s, g, (const T*)pen.iac, (const T*)pen.ia2,
                        (const cpx<T>*)X[0], (const cpx<T>*)X[1], (const cpx<T>*)X[2], (const cpx<T>*)XF,
                        (const cpx<T>*)XG, (const T*)b.kx, (const T*)b.ky, (cpx<T>*)pen.spec);
-    // the generic y-transforms with the L modes in place of the levels, ten fields
+    // y-transforms with the L modes in place of the levels, seven fields: in registers at 16 to 1024
+    // points (FP64: 512), the LDS kernels beyond
     DevGeom gp = g;
     gp.nq = g.L;
-    gp.PS = g.P;
     const int TX = fft_tile(g.N, sizeof(cpx<T>));
     const size_t sm = (size_t)2 * TX * g.N * sizeof(cpx<T>);
-    const dim3 gy((g.KX + TX - 1) / TX, g.L, 10);
-    hipLaunchKernelGGL(k_fft_y_inv<T>, gy, dim3(256), sm, s, gp, TX, (const cpx<T>*)pen.spec, b.rows,
-                       (const cpx<T>*)b.twN, (cpx<T>*)pen.hin);
-    hipLaunchKernelGGL(k_rows_mask<T>, dim3(g.N, g.L, 6), dim3(256), (size_t)2 * g.M * sizeof(cpx<T>), s, gp,
-                       (const T*)pen.mask, (const cpx<T>*)pen.hin, (const cpx<T>*)b.twM, (cpx<T>*)pen.hout);
-    hipLaunchKernelGGL(k_fft_y_fwd<T>, gy, dim3(256), sm, s, gp, TX, (const cpx<T>*)pen.hout, b.rows,
-                       (const cpx<T>*)b.twN, (cpx<T>*)pen.spec_out);
-    hipLaunchKernelGGL(k_pen_combine<T>, dim3(nb), dim3(256), 0, s, g, (T)(1.0 / pen.eta),
+    const dim3 gy((g.KX + TX - 1) / TX, g.L, kPenFields);
+    if (!launch_y_inv_group<T>(gp, kPenFields, (const cpx<T>*)pen.spec, (const cpx<T>*)b.twN, (cpx<T>*)pen.hin, s))
+        hipLaunchKernelGGL(k_fft_y_inv<T>, gy, dim3(256), sm, s, gp, TX, (const cpx<T>*)pen.spec, b.rows,
+                           (const cpx<T>*)b.twN, (cpx<T>*)pen.hin);
+    const bool kept = g.KX == kept_cols(g.M);
+    switch (kept ? g.logM : 0) {
+        case 4: launch_rows_mask<T, 4>(g, pen, b.twM, s); break;
+        case 5: launch_rows_mask<T, 5>(g, pen, b.twM, s); break;
+        case 6: launch_rows_mask<T, 6>(g, pen, b.twM, s); break;
+        case 7: launch_rows_mask<T, 7>(g, pen, b.twM, s); break;
+        case 8: launch_rows_mask<T, 8>(g, pen, b.twM, s); break;
+        case 9: launch_rows_mask<T, 9>(g, pen, b.twM, s); break;
+        case 10:
+            if constexpr (sizeof(T) == 4) {
+                launch_rows_mask<T, 10>(g, pen, b.twM, s);
+                break;
+            }
+            [[fallthrough]];
+        default:
+            hipLaunchKernelGGL(k_rows_mask<T>, dim3(g.N / 2, g.L, kPenFields), dim3(256),
+                               (size_t)2 * g.M * sizeof(cpx<T>), s, gp, (const T*)pen.mask, (const cpx<T>*)pen.hin,
+                               (const cpx<T>*)b.twM, (cpx<T>*)pen.hout);
+    }
+    if (!launch_y_fwd_group<T>(gp, kPenFields, (const cpx<T>*)pen.hout, (const cpx<T>*)b.twN, (cpx<T>*)pen.spec_out, s))
+        hipLaunchKernelGGL(k_fft_y_fwd<T>, gy, dim3(256), sm, s, gp, TX, (const cpx<T>*)pen.hout, b.rows,
+                           (const cpx<T>*)b.twN, (cpx<T>*)pen.spec_out);
+    hipLaunchKernelGGL(k_pen_combine<T>, gm, dim3(256), 0, s, g, (T)(1.0 / pen.eta),
                        (const cpx<T>*)pen.spec_out, (const T*)b.kx, (const T*)b.ky, (cpx<T>*)Nout[0],
                        (cpx<T>*)Nout[1], (cpx<T>*)Nout[2], (cpx<T>*)NF, (cpx<T>*)NG);
 }
