@@ -291,6 +291,14 @@ __device__ __forceinline__ void fft_group(cpx<T> (&v)[NF][E], cpx<T>* sb, const 
     }
 }
 
+// Shape of the register row transforms (M points): E elements per lane, groups of W lanes, G groups
+// per wave, RPB per block.
+template <typename T, int LOGM, int WPB>
+struct RowShape {
+    static constexpr int M = 1 << LOGM, E = group_elems(LOGM), W = M / E, G = 64 / W, RPB = WPB * G, SP = M + M / 8;
+    static constexpr size_t lds = ((size_t)M + (size_t)RPB * SP) * sizeof(cpx<T>);
+};
+
 // ---------------------------------------------------------------------------------------
 // Stockham FFT on nb sequences of length n = 2^logn held in LDS (a), with b as the ping-pong
 // buffer: radix-4 passes while two or more radix-2 stages remain, then one radix-2 pass if

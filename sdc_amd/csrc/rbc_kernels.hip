@@ -1131,11 +1131,6 @@ __global__ void __launch_bounds__(192) k_rows512t(DevGeom g, int nblk, int per, 
 // values.  256^2 x 24 FP64: 101 us (3.4 TB/s; the
 // LDS radix-4 form it replaces there: 243 us); 1024 x 128 x 40 FP32: 173 us (579).
 template <typename T, int LOGM, int WPB>
-struct RowShape {
-    static constexpr int M = 1 << LOGM, E = group_elems(LOGM), W = M / E, G = 64 / W, RPB = WPB * G, SP = M + M / 8;
-    static constexpr size_t lds = ((size_t)M + (size_t)RPB * SP) * sizeof(cpx<T>);
-};
-template <typename T, int LOGM, int WPB>
 __device__ __forceinline__ void k_rows_w_body(DevGeom g, const cpx<T>* __restrict__ hin,
                                               const cpx<T>* __restrict__ twM, cpx<T>* __restrict__ hout) {
     using R = RowShape<T, LOGM, WPB>;

@@ -112,49 +112,80 @@ __global__ void __launch_bounds__(256) k_point_basis(int np, int L, const float*
 }
 
 // ---------------------------------------------------------------------------------------
-// Spectral velocity at nz heights: spec[c][l][p] for c = u, v, w (complex), thread per mode.
-// zb[l][3][L] = C'_m, C_m, S_m at height l.
+// Spectral velocity at nz heights: spec[c][l][p] for c = u, v, w (complex), thread per mode and
+// kLev heights.  zb[l][3][L] = C'_m, C_m, S_m at height l (wave-uniform, scalar loads).
+// A thread per mode and height read the mode's 2 L coefficients, L values apart between lanes, again
+// for each of the 128 heights (128^2 x 16 state: 63 us); with four heights they are read a quarter as
+// often: 17 us, for 11 MB written.
 // ---------------------------------------------------------------------------------------
+constexpr int kLev = 4;
 template <typename T, typename O>
 __global__ void __launch_bounds__(256) k_vel_levels(DevGeom g, int nz, const double* __restrict__ zb,
                                                     const cpx<T>* __restrict__ Xf, const cpx<T>* __restrict__ Xg,
                                                     const cpx<T>* __restrict__ XF, const cpx<T>* __restrict__ XG,
                                                     const T* __restrict__ kxa, const T* __restrict__ kya,
                                                     cpx<O>* __restrict__ spec) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x, l = blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x, l0 = blockIdx.y * kLev;
     if (p >= g.P) return;
     const int L = g.L;
-    const double* tb = zb + (size_t)l * 3 * L;
-    cpx<double> A = mk<double>(0, 0), B = A, Cc = A;
+    const double* tb[kLev];
+    cpx<double> A[kLev], B[kLev], Cc[kLev];
+#pragma unroll
+    for (int i = 0; i < kLev; ++i) {
+        tb[i] = zb + (size_t)min(l0 + i, nz - 1) * 3 * L;
+        A[i] = B[i] = Cc[i] = mk<double>(0, 0);
+    }
+#pragma unroll 4
     for (int m = 0; m < L; ++m) {
         const cpx<T> f = Xf[(size_t)p * L + m], gg = Xg[(size_t)p * L + m];
         const cpx<double> fd = mk<double>(f.x, f.y), gd = mk<double>(gg.x, gg.y);
-        A = A + cscale(fd, tb[m]);
-        Cc = Cc + cscale(fd, tb[L + m]);
-        B = B + cscale(gd, tb[2 * L + m]);
-    }
-    const double kx = kxa[p], ky = kya[p];
-    cpx<double> u = imul(A, kx) + imul(B, ky);
-    cpx<double> v = imul(A, ky) - imul(B, kx);
-    const cpx<double> w = cscale(Cc, kx * kx + ky * ky);
-    if (p == 0) {  // add_dc_part (calculate_velocity_operator.cu:479-494)
-        for (int m = 0; m < L; ++m) {
-            u = u + cscale(mk<double>(XF[m].x, XF[m].y), tb[2 * L + m]);
-            v = v + cscale(mk<double>(XG[m].x, XG[m].y), tb[2 * L + m]);
+#pragma unroll
+        for (int i = 0; i < kLev; ++i) {
+            A[i] = A[i] + cscale(fd, tb[i][m]);
+            Cc[i] = Cc[i] + cscale(fd, tb[i][L + m]);
+            B[i] = B[i] + cscale(gd, tb[i][2 * L + m]);
         }
     }
+    const double kx = kxa[p], ky = kya[p];
     const size_t plane = (size_t)nz * g.P;
-    cpx<O>* o = spec + (size_t)l * g.P + p;
-    o[0] = mk<O>((O)u.x, (O)u.y);
-    o[plane] = mk<O>((O)v.x, (O)v.y);
-    o[2 * plane] = mk<O>((O)w.x, (O)w.y);
+#pragma unroll
+    for (int i = 0; i < kLev; ++i) {
+        if (l0 + i >= nz) break;
+        cpx<double> u = imul(A[i], kx) + imul(B[i], ky);
+        cpx<double> v = imul(A[i], ky) - imul(B[i], kx);
+        const cpx<double> w = cscale(Cc[i], kx * kx + ky * ky);
+        if (p == 0) {  // add_dc_part (calculate_velocity_operator.cu:479-494)
+            for (int m = 0; m < L; ++m) {
+                u = u + cscale(mk<double>(XF[m].x, XF[m].y), tb[i][2 * L + m]);
+                v = v + cscale(mk<double>(XG[m].x, XG[m].y), tb[i][2 * L + m]);
+            }
+        }
+        cpx<O>* o = spec + (size_t)(l0 + i) * g.P + p;
+        o[0] = mk<O>((O)u.x, (O)u.y);
+        o[plane] = mk<O>((O)v.x, (O)v.y);
+        o[2 * plane] = mk<O>((O)w.x, (O)w.y);
+    }
 }
 
 // ---------------------------------------------------------------------------------------
-// x C2R of the hybrid rows [c][l][y][kx] of the three components into the real grid
-// [c][l][y][x] (the reference's u_i[x + y M + l M N] layout).  Block per (y, l): u + i v and
-// w go through two complex inverse FFTs of length M.
+// x C2R of the hybrid rows [c][l][y][kx] of the three components into the real grid, at point
+// (l, y, x): PLANAR, [c][l][y][x] (the reference's u_i[x + y M + l M N] layout), or one float4
+// (u, v, w, 0) per point, so that the eight corners of an interpolation are eight loads.
 // ---------------------------------------------------------------------------------------
+template <bool PLANAR>
+__device__ __forceinline__ void put_velocity(float* __restrict__ grid, size_t cs, size_t at, float u, float v, float w) {
+    if constexpr (PLANAR) {
+        grid[at] = u;
+        grid[cs + at] = v;
+        grid[2 * cs + at] = w;
+    } else {
+        reinterpret_cast<float4*>(grid)[at] = make_float4(u, v, w, 0.f);
+    }
+}
+
+// Block per (y, l), row lengths outside k_vel_rows_w: u + i v and w go through two complex inverse
+// FFTs of length M.
+template <bool PLANAR>
 __global__ void __launch_bounds__(256) k_vel_rows(DevGeom g, const cpx<float>* __restrict__ hyb,
                                                   const cpx<float>* __restrict__ twM, float* __restrict__ grid) {
     extern __shared__ unsigned char smem_raw[];
@@ -180,12 +211,57 @@ __global__ void __launch_bounds__(256) k_vel_rows(DevGeom g, const cpx<float>* _
     }
     __syncthreads();
     const cpx<float>* r = lds_fft(a, b, g.logM, 2, twM, true);
-    const size_t cs = (size_t)nz * N * M;
-    float* o = grid + ((size_t)l * N + y) * M;
-    for (int x = threadIdx.x; x < M; x += blockDim.x) {
-        o[x] = r[x].x;
-        o[cs + x] = r[x].y;
-        o[2 * cs + x] = r[M + x].x;
+    const size_t cs = (size_t)nz * N * M, at = ((size_t)l * N + y) * M;
+    for (int x = threadIdx.x; x < M; x += blockDim.x) put_velocity<PLANAR>(grid, cs, at + x, r[x].x, r[x].y, r[M + x].x);
+}
+
+// Row pair (y, y + 1) of one height on a group of M / E lanes, in registers: u + i v of each row and
+// w of the two rows, three transforms for six real rows; the pairs of all heights in one flat range
+// (pairs past its end are computed on the last one and not stored).  Bound by memory: 3 nz N KX
+// values in, the grid out.  128^2 x 128: 29 -> 13 us.
+template <int LOGM, int WPB, bool PLANAR>
+__global__ void __launch_bounds__(64 * WPB) k_vel_rows_w(DevGeom g, int npair, const cpx<float>* __restrict__ hyb,
+                                                         const cpx<float>* __restrict__ twM, float* __restrict__ grid) {
+    using R = RowShape<float, LOGM, WPB>;
+    constexpr int M = R::M, E = R::E, W = R::W, G = R::G, RPB = R::RPB, KX = kept_cols(M);
+    __shared__ cpx<float> tw[M];
+    __shared__ cpx<float> scr[RPB][R::SP];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, grp = lane / W, j = lane - grp * W;
+    const int KXp = g.KXp;
+    const int pr0 = blockIdx.x * RPB + wave * G + grp, pr = min(pr0, npair - 1);
+    const size_t fstride = (size_t)g.nq * g.N * KXp;
+    const cpx<float>* x1 = hyb + (size_t)(2 * pr) * KXp;
+    cpx<float> v[3][E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int k = j + W * r;
+        const int src = k < KX ? k : (k > M - KX ? M - k : -1);
+        cpx<float> a[3][2];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                a[c][h] = mk<float>(0, 0);
+                if (src >= 0) a[c][h] = x1[c * fstride + h * KXp + src];
+                if (src == 0) a[c][h].y = 0.f;  // a C2R ignores the imaginary part at kx = 0
+            }
+        auto join = [&](const cpx<float>& p, const cpx<float>& q) {  // P + i Q
+            return k < KX ? mk(p.x - q.y, p.y + q.x) : mk(p.x + q.y, -p.y + q.x);
+        };
+        v[0][r] = join(a[0][0], a[1][0]);
+        v[1][r] = join(a[0][1], a[1][1]);
+        v[2][r] = join(a[2][0], a[2][1]);
+    }
+    for (int e = threadIdx.x; e < M; e += blockDim.x) tw[e] = twM[e];
+    __syncthreads();
+    fft_group<LOGM, true, 3>(v, scr[wave * G + grp], tw, j);
+    if (pr0 >= npair) return;
+    const size_t cs = (size_t)g.nq * g.N * M;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const size_t at = (size_t)(2 * pr) * M + j + W * r;
+        put_velocity<PLANAR>(grid, cs, at, v[0][r].x, v[0][r].y, v[2][r].x);
+        put_velocity<PLANAR>(grid, cs, at + M, v[1][r].x, v[1][r].y, v[2][r].y);
     }
 }
 
@@ -195,8 +271,7 @@ __global__ void __launch_bounds__(256) k_vel_rows(DevGeom g, const cpx<float>* _
 // (:692-717) and reflection at the lids (:722-764).  Mixed float/double expressions are
 // kept in the reference's types.
 // ---------------------------------------------------------------------------------------
-__device__ inline void vel_trilinear(const float* __restrict__ ux, const float* __restrict__ uy,
-                                     const float* __restrict__ uz, int xs, int ys, float clx, float cly, float x,
+__device__ inline void vel_trilinear(const float4* __restrict__ uvw, int xs, int ys, float clx, float cly, float x,
                                      float y, float z, float& ru, float& rv, float& rw) {
     const int xy = xs * ys;
     float xg = x * xs / clx;
@@ -215,9 +290,10 @@ __device__ inline void vel_trilinear(const float* __restrict__ ux, const float* 
     float wR = xg - float(ix0), wL = 1 - wR;
     auto lerpx = [&](int iy, int iz, float& a, float& b, float& c) {
         const int i0 = ix0 + iy * xs + iz * xy, i1 = ix1 + iy * xs + iz * xy;
-        a = wL * ux[i0] + wR * ux[i1];
-        b = wL * uy[i0] + wR * uy[i1];
-        c = wL * uz[i0] + wR * uz[i1];
+        const float4 p = uvw[i0], q = uvw[i1];
+        a = wL * p.x + wR * q.x;
+        b = wL * p.y + wR * q.y;
+        c = wL * p.z + wR * q.z;
     };
     float x00, y00, z00, x10, y10, z10, x01, y01, z01, x11, y11, z11;
     lerpx(iy0, iz0, x00, y00, z00);
@@ -250,31 +326,32 @@ __device__ inline void finish_particle(float& x, float& y, float& z, int i, int 
     }
 }
 
-__global__ void __launch_bounds__(256) k_tracer_rk4(int np, const float* __restrict__ grid, int M, int N, float Lx,
+// Bound by the gathers of four dependent stages: eight corners of three components each, from a grid of
+// (u, v, w, 0) points (24 MB at 128^2 x 128 heights, 33 MB here): 24 loads a stage from separate
+// components 72 us for 100,000 particles, eight 16-byte loads 24 us.
+__global__ void __launch_bounds__(256) k_tracer_rk4(int np, const float4* __restrict__ grid, int M, int N, float Lx,
                                                     float Ly, const float* __restrict__ x0, const float* __restrict__ y0,
                                                     const float* __restrict__ z0, float dt, float* __restrict__ x1,
                                                     float* __restrict__ y1, float* __restrict__ z1, float sigma,
                                                     uint64_t seed, uint64_t ctr0) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
-    const size_t cs = (size_t)kZNum * N * M;
-    const float *ux = grid, *uy = grid + cs, *uz = grid + 2 * cs;
     float x = x0[i], y = y0[i], z = z0[i];
     float vx, vy, vz;
-    vel_trilinear(ux, uy, uz, M, N, Lx, Ly, x, y, z, vx, vy, vz);
+    vel_trilinear(grid, M, N, Lx, Ly, x, y, z, vx, vy, vz);
     const float dx1 = dt * vx, dy1 = dt * vy, dz1 = dt * vz;
     float xt = x + 0.5 * dx1, yt = y + 0.5 * dy1, zt = z + 0.5 * dz1;
-    vel_trilinear(ux, uy, uz, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
+    vel_trilinear(grid, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
     const float dx2 = dt * vx, dy2 = dt * vy, dz2 = dt * vz;
     xt = x + 0.5 * dx2;
     yt = y + 0.5 * dy2;
     zt = z + 0.5 * dz2;
-    vel_trilinear(ux, uy, uz, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
+    vel_trilinear(grid, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
     const float dx3 = dt * vx, dy3 = dt * vy, dz3 = dt * vz;
     xt = x + dx3;
     yt = y + dy3;
     zt = z + dz3;
-    vel_trilinear(ux, uy, uz, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
+    vel_trilinear(grid, M, N, Lx, Ly, xt, yt, zt, vx, vy, vz);
     const float dx4 = dt * vx, dy4 = dt * vy, dz4 = dt * vz;
     x += (dx1 + 2 * (dx2 + dx3) + dx4) / 6.;
     y += (dy1 + 2 * (dy2 + dy3) + dy4) / 6.;
@@ -1034,7 +1111,7 @@ void padded_mode_table(const rbc_ctx* c, std::vector<float>& t, std::vector<int>
 template <typename T>
 void launch_vel_levels(rbc_ctx* c, const DevGeom& gt, int nz, const double* zb, void* spec) {
     const Buffers& b = c->b;
-    dim3 grid((c->dg.P + 255) / 256, nz);
+    dim3 grid((c->dg.P + 255) / 256, (nz + kLev - 1) / kLev);
     hipLaunchKernelGGL((k_vel_levels<T, float>), grid, dim3(256), 0, c->stream, gt, nz, zb, (const cpx<T>*)b.X[1],
                        (const cpx<T>*)b.X[2], (const cpx<T>*)b.XF, (const cpx<T>*)b.XG, (const T*)b.kx,
                        (const T*)b.ky, (cpx<float>*)spec);
@@ -1047,11 +1124,12 @@ struct GridWork {
     cpx<float>* hyb = nullptr;  // [3][nz][N][KXp]
     cpx<float>* twM = nullptr;
     cpx<float>* twN = nullptr;
-    float* grid = nullptr;      // [3][nz][N][M]
+    float* grid = nullptr;      // [3][nz][N][M], or [nz][N][M][4] (planar = false)
+    bool planar = true;
     int nz = 0;
 };
 
-void alloc_grid_work(rbc_ctx* c, int nz, GridWork& w, std::vector<void*>& owned) {
+void alloc_grid_work(rbc_ctx* c, int nz, bool planar, GridWork& w, std::vector<void*>& owned) {
     const DevGeom& g = c->dg;
     auto al = [&](size_t bytes) {
         void* p = nullptr;
@@ -1060,10 +1138,11 @@ void alloc_grid_work(rbc_ctx* c, int nz, GridWork& w, std::vector<void*>& owned)
         return p;
     };
     w.nz = nz;
+    w.planar = planar;
     w.zb = (double*)al((size_t)nz * 3 * g.L * sizeof(double));
     w.spec = (cpx<float>*)al((size_t)3 * nz * g.P * sizeof(cpx<float>));
     w.hyb = (cpx<float>*)al((size_t)3 * nz * g.N * g.KXp * sizeof(cpx<float>));
-    w.grid = (float*)al((size_t)3 * nz * g.N * g.M * sizeof(float));
+    w.grid = (float*)al((size_t)(planar ? 3 : 4) * nz * g.N * g.M * sizeof(float));
     w.twM = (cpx<float>*)al((size_t)g.M * sizeof(cpx<float>));
     w.twN = (cpx<float>*)al((size_t)g.N * sizeof(cpx<float>));
     const std::vector<float> tm = twiddles_f(g.M), tn = twiddles_f(g.N);
@@ -1074,6 +1153,31 @@ void alloc_grid_work(rbc_ctx* c, int nz, GridWork& w, std::vector<void*>& owned)
 void set_heights(rbc_ctx* c, GridWork& w, const std::vector<double>& z) {
     const std::vector<double> t = basis_table(c->dg.L, z);
     HIPCHK(hipMemcpy(w.zb, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+}
+
+template <int LOGM, bool PLANAR>
+void launch_vel_rows_w(rbc_ctx* c, const DevGeom& gt, const GridWork& w) {
+    constexpr int WPB = 4, RPB = RowShape<float, LOGM, WPB>::RPB;
+    static_assert(RowShape<float, LOGM, WPB>::lds <= 65536, "row pair tile");
+    const int npair = w.nz * (gt.N / 2);
+    hipLaunchKernelGGL((k_vel_rows_w<LOGM, WPB, PLANAR>), dim3((npair + RPB - 1) / RPB), dim3(64 * WPB), 0, c->stream, gt,
+                       npair, (const cpx<float>*)w.hyb, (const cpx<float>*)w.twM, w.grid);
+}
+// in registers at 16 to 1024 points, through LDS else
+template <bool PLANAR>
+void launch_vel_rows(rbc_ctx* c, const DevGeom& gt, const GridWork& w) {
+    switch (gt.KX == kept_cols(gt.M) ? gt.logM : 0) {
+        case 4: return launch_vel_rows_w<4, PLANAR>(c, gt, w);
+        case 5: return launch_vel_rows_w<5, PLANAR>(c, gt, w);
+        case 6: return launch_vel_rows_w<6, PLANAR>(c, gt, w);
+        case 7: return launch_vel_rows_w<7, PLANAR>(c, gt, w);
+        case 8: return launch_vel_rows_w<8, PLANAR>(c, gt, w);
+        case 9: return launch_vel_rows_w<9, PLANAR>(c, gt, w);
+        case 10: return launch_vel_rows_w<10, PLANAR>(c, gt, w);
+        default:
+            hipLaunchKernelGGL(k_vel_rows<PLANAR>, dim3(gt.N, w.nz), dim3(256), (size_t)4 * gt.M * sizeof(cpx<float>),
+                               c->stream, gt, (const cpx<float>*)w.hyb, (const cpx<float>*)w.twM, w.grid);
+    }
 }
 
 // velocity grid at the heights of w (spectral -> y-FFT -> x C2R), on the context's stream
@@ -1090,8 +1194,8 @@ void velocity_grid(rbc_ctx* c, const GridWork& w) {
         hipLaunchKernelGGL(k_fft_y_inv<float>, gy, dim3(256), (size_t)2 * TX * gt.N * sizeof(cpx<float>), c->stream,
                            gt, TX, (const cpx<float>*)w.spec, c->b.rows, (const cpx<float>*)w.twN, w.hyb);
     }
-    hipLaunchKernelGGL(k_vel_rows, dim3(gt.N, w.nz), dim3(256), (size_t)4 * gt.M * sizeof(cpx<float>), c->stream, gt,
-                       (const cpx<float>*)w.hyb, (const cpx<float>*)w.twM, w.grid);
+    if (w.planar) launch_vel_rows<true>(c, gt, w);
+    else launch_vel_rows<false>(c, gt, w);
     HIPCHK(hipGetLastError());
 }
 
@@ -1404,7 +1508,7 @@ int rbc_tracer_create(rbc_ctx* c, int num_particles, int buffer_size, int mode, 
         t->z = (float*)al(pos);
         t->red = (double*)al(4 * sizeof(double));
         if (mode == RBC_TRACER_RK4_TRILINEAR) {
-            alloc_grid_work(c, kZNum, t->gw, t->owned);
+            alloc_grid_work(c, kZNum, false, t->gw, t->owned);
             // linspace(-PARTICLE_Z_MAX, PARTICLE_Z_MAX) in the device real type (particle_tracer.cu:494-501)
             const float zmin = (float)(-kZMax), zmax = (float)kZMax;
             std::vector<double> zl(kZNum);
@@ -1490,7 +1594,7 @@ int rbc_tracer_step(rbc_tracer* t, double dt) {
         hipSetDevice(c->p.device);
         if (t->mode == RBC_TRACER_RK4_TRILINEAR) {
             velocity_grid(c, t->gw);
-            hipLaunchKernelGGL(k_tracer_rk4, pg, dim3(256), 0, c->stream, np, (const float*)t->gw.grid, c->dg.M,
+            hipLaunchKernelGGL(k_tracer_rk4, pg, dim3(256), 0, c->stream, np, (const float4*)t->gw.grid, c->dg.M,
                                c->dg.N, (float)c->p.Lx, (float)c->p.Ly, (const float*)t->x + in,
                                (const float*)t->y + in, (const float*)t->z + in, (float)dt, t->x + outo, t->y + outo,
                                t->z + outo, sigma, t->seed, ctr0);
@@ -1596,7 +1700,7 @@ int rbc_velocity_grid(rbc_ctx* c, int nz, const double* z, float* ux, float* uy,
             vw->gw_owned.clear();
             vw->gw = GridWork();
             vw->gw_cap = 0;
-            alloc_grid_work(c, nz, vw->gw, vw->gw_owned);
+            alloc_grid_work(c, nz, true, vw->gw, vw->gw_owned);
             vw->gw_cap = nz;
         }
         GridWork& w = vw->gw;
@@ -1626,7 +1730,7 @@ int rbc_characteristic_velocity(rbc_ctx* c, int nz, double* U) {
             vw->gw_owned.clear();
             vw->gw = GridWork();
             vw->gw_cap = 0;
-            alloc_grid_work(c, nz, vw->gw, vw->gw_owned);
+            alloc_grid_work(c, nz, true, vw->gw, vw->gw_owned);
             vw->gw_cap = nz;
         }
         GridWork& w = vw->gw;
