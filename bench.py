@@ -430,7 +430,7 @@ def _max_rel(a, b, keep):
 
 
 def tracer_flops(P, L, npart):
-    """Matrix-core FP32 operations of one spectral velocity evaluation (k_vel_points_mma) at npart
+    """FP32 operations of one spectral velocity evaluation (k_vel_points_mma) at npart
     particles over P kept modes: per (particle, mode) six length-L vertical sums (A = sum f C',
     Cc = sum f C, B = sum g S, real and imaginary parts), 12 L operations."""
     return npart * P * 12 * L
@@ -501,9 +501,9 @@ def run_tracers(a):
                        "frac": round(tf / FP32_PEAK_TFLOPS, 4),
                        "kernel": "k_vel_points_mma (two per spectral RK2 step)",
                        "algorithmic_flops_per_step": fl, "kept_modes": P,
-                       "note": "FP32 matrix-core flops of the vertical sums over the whole tracer step time (both "
-                               "evaluations, the slice sums and the position updates); the phases and the velocity "
-                               "combination run on the VALU, which does not overlap the matrix cores here"}
+                       "note": "FP32 flops of the vertical sums (as six products of BF16 parts) over the whole tracer step time (both "
+                               "evaluations, the slice sums and the position updates) against the FP32 matrix peak; the "
+                               "phases and the velocity combination on the VALU bound it"}
     S.close()
     print(json.dumps(out))
 

@@ -457,16 +457,15 @@ __global__ void __launch_bounds__(256) k_vel_points(DevGeom g, int np, const flo
     }
 }
 
-// The same sums on the FP32 matrix cores (FP32 state, L <= 32).  Block = 8 waves x 16
-// particles.  For a tile of 16 modes the six vertical sums of every (mode, particle) pair,
-// A = sum f_m C'_m, Cc = sum f_m C_m and B = sum g_m S_m with their real and imaginary parts,
-// are products D[mode][particle] = sum_m coef[mode][m] basis[m][particle] with k = m:
-// v_mfma_f32_16x16x4_f32 (K = 4), A operand = staged coefficients (row = mode = lane % 16,
-// k = lane / 16), B operand = basis values at the lane's particle (column = particle = lane % 16,
-// k = lane / 16).  The phase and the velocity combination then run on the VALU in the MFMA output
-// layout: lane l holds column l % 16 (its particle) and the mode rows 4 (l / 16) + r, r < 4, so the
-// four 16-lane groups hold complementary rows of the same particles and are added at the end.
-// The weight w_k (1 at kx = 0, else 2) is folded into the staged coefficients.  The modes come
+// The same sums on the matrix cores (FP32 state, L <= 32).  Block = 8 waves x 16 particles.  For a
+// sub-tile of 16 modes the six vertical sums of every (mode, particle) pair, A = sum f_m C'_m,
+// Cc = sum f_m C_m and B = sum g_m S_m with their real and imaginary parts, are products
+// D[mode][particle] = sum_m coef[mode][m] basis[m][particle] with k = m (A operand: coefficients, row =
+// mode; B operand: basis values at the particle's height, column = particle).  The phase and the velocity
+// combination then run on the VALU in the MFMA output layout: lane l holds column l % 16 (its
+// particle) and the mode rows 4 (l / 16) + r, r < 4, so the four 16-lane groups hold complementary
+// rows of the same particles and are added at the end.  The weight w_k (1 at kx = 0, else 2) is
+// folded into the staged coefficients.  The modes come
 // from the padded list (padded_mode_table), where the 4 rows of a lane group share kx and have
 // consecutive ky: one sincospi per group gives exp(2 pi i k.x) of its first row, and the others
 // follow by a complex product with exp(2 pi i r y / Ly), r = 1, 2, 3, taken once per particle.
@@ -503,172 +502,45 @@ __device__ __forceinline__ void vel_combine(const float2* sg, const float4* sm, 
         w += k2 * (cs * acc[2][r] - sn * acc[3][r]);
     }
 }
-template <int LMAX>
-__global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_mma(
-    DevGeom g, int np, const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
-    const cpx<float>* __restrict__ Xf, const cpx<float>* __restrict__ Xg, const cpx<float>* __restrict__ XF,
-    const cpx<float>* __restrict__ XG, const double* __restrict__ lam, const float4* __restrict__ modes,
-    const int* __restrict__ pmap, int npad, int tiles_per_slice, float* __restrict__ part, const float4* __restrict__ zb) {
-    static_assert(LMAX % 4 == 0 && LMAX <= 32, "k-steps of 4 modes");
-    constexpr int KS = LMAX / 4;
-    constexpr int PER = (kTile * LMAX + kVelMmaThreads - 1) / kVelMmaThreads;  // staged values per thread
-    __shared__ float4 sc[kTile][LMAX + 1];  // w_k (f.re, f.im, g.re, g.im); odd row length spreads the banks
-    __shared__ float4 sm[kTile];            // (kx, ky, k^2, 0)
-    __shared__ float2 sg[kTile / 4];        // (kx index, ky index) of the first mode of each group of 4
-    const int L = g.L, P = g.P, NYc = g.NYc;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, q = lane >> 4;
-    const int i = blockIdx.x * (kVelMmaThreads / 4) + wave * 16 + j;
-    const int slice = blockIdx.y;
-    const bool live = i < np;
-    const float x = live ? px[i] : 0.f, y = live ? py[i] : 0.f, z = live ? pz[i] : 0.f;
-    // basis values of the lane's k index m = 4 s + q at the particle's height
-    float bcp[KS], bcc[KS], bss[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const int m = 4 * s + q;
-        bcp[s] = bcc[s] = bss[s] = 0.f;
-        if (m < L) {
-            if (zb) {  // computed once per evaluation by k_point_basis
-                if (live) {
-                    const float4 t = zb[(size_t)i * L + m];
-                    bcp[s] = t.x;
-                    bcc[s] = t.y;
-                    bss[s] = t.z;
-                }
-            } else {
-                double C = 0, Cp = 0, S = 0;
-                basis_at(m, lam[m], (double)z, C, Cp, S);
-                bcp[s] = (float)Cp;
-                bcc[s] = (float)C;
-                bss[s] = (float)S;
-            }
-        }
-    }
-    const float xr = x / (float)g.Lx - floorf(x / (float)g.Lx);
-    const float yr = y / (float)g.Ly - floorf(y / (float)g.Ly);
-    // exp(2 pi i r yr), r = 1, 2, 3
-    float ds[4], dc[4];
-    sincospif(2.0f * yr, &ds[1], &dc[1]);
-    dc[2] = dc[1] * dc[1] - ds[1] * ds[1];
-    ds[2] = 2.f * ds[1] * dc[1];
-    dc[3] = dc[2] * dc[1] - ds[2] * ds[1];
-    ds[3] = ds[2] * dc[1] + dc[2] * ds[1];
-    float u = 0.f, v = 0.f, w = 0.f;
-    if (slice == 0) {  // mean flow (k = 0), each lane group its residue of m modulo 4
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const int m = 4 * s + q;
-            if (m < L) {
-                u += bss[s] * XF[m].x;
-                v += bss[s] * XG[m].x;
-            }
-        }
-    }
-    const int ntile = (npad + kTile - 1) / kTile;
-    const int t0 = slice * tiles_per_slice, t1 = min(ntile, t0 + tiles_per_slice);
-    // the coefficients of tile t into registers: value e = threadIdx.x + u * threads of the tile
-    float4 pre[PER], pmd = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto fetch = [&](int t) {
-        const int pbase = t * kTile, nm = min(kTile, npad - pbase);
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int e = threadIdx.x + u * kVelMmaThreads, jj = e / LMAX, m = e - jj * LMAX;
-            float4 val = make_float4(0.f, 0.f, 0.f, 0.f);
-            const int p = (e < kTile * LMAX && jj < nm) ? pmap[pbase + jj] : -1;
-            if (p >= 0 && p < P && m < L) {
-                const cpx<float> f = Xf[(size_t)p * L + m], gg = Xg[(size_t)p * L + m];
-                const float wk = p < NYc ? 1.f : 2.f;  // compact p < NYc <=> kx = 0
-                val = make_float4(wk * f.x, wk * f.y, wk * gg.x, wk * gg.y);
-            }
-            pre[u] = val;
-        }
-        if (threadIdx.x < kTile)
-            pmd = (int)threadIdx.x < nm ? modes[pbase + threadIdx.x] : make_float4(0.f, 0.f, 0.f, 0.f);
-    };
-    if (t0 < t1) fetch(t0);
-    for (int t = t0; t < t1; ++t) {
-        const int nm = min(kTile, npad - t * kTile);
-        lds_barrier();  // the previous tile is consumed
-#pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int e = threadIdx.x + u * kVelMmaThreads;
-            if (e < kTile * LMAX) sc[e / LMAX][e % LMAX] = pre[u];
-        }
-        if (threadIdx.x < kTile) {
-            sm[threadIdx.x] = make_float4(pmd.z, pmd.w, pmd.z * pmd.z + pmd.w * pmd.w, 0.f);
-            if ((threadIdx.x & 3) == 0) sg[threadIdx.x >> 2] = make_float2(pmd.x, pmd.y);
-        }
-        lds_barrier();
-        if (t + 1 < t1) fetch(t + 1);  // in flight while tile t is computed
-        const int nsub = (nm + 15) / 16;
-        // the six products of a 16-mode sub-tile on the matrix cores
-        auto products = [&](int sub, vpf32x4 (&acc)[6]) {
-#pragma unroll
-            for (int k = 0; k < 6; ++k) acc[k] = vpf32x4{0.f, 0.f, 0.f, 0.f};
-            const float4* row = sc[sub * 16 + j];
-#pragma unroll
-            for (int s = 0; s < KS; ++s) {
-                const float4 c4 = row[4 * s + q];
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.x, bcp[s], acc[0], 0, 0, 0);  // A.re
-                acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.y, bcp[s], acc[1], 0, 0, 0);  // A.im
-                acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.x, bcc[s], acc[2], 0, 0, 0);  // Cc.re
-                acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.y, bcc[s], acc[3], 0, 0, 0);  // Cc.im
-                acc[4] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.z, bss[s], acc[4], 0, 0, 0);  // B.re
-                acc[5] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4.w, bss[s], acc[5], 0, 0, 0);  // B.im
-            }
-        };
-        auto combine = [&](int sub, const vpf32x4 (&acc)[6]) {
-            vel_combine(sg, sm, sub * 16 + 4 * q, xr, yr, dc, ds, acc, u, v, w);
-        };
-        // software pipeline: the products of sub-tile sub + 1 are issued before the combination of
-        // sub-tile sub, so that the matrix cores and the VALU work at the same time
-        vpf32x4 acc0[6], acc1[6];
-        products(0, acc0);
-#pragma unroll
-        for (int sub = 0; sub < kTile / 16; sub += 2) {
-            if (sub + 1 < nsub) products(sub + 1, acc1);
-            if (sub < nsub) combine(sub, acc0);
-            if (sub + 2 < nsub) products(sub + 2, acc0);
-            if (sub + 1 < nsub) combine(sub + 1, acc1);
-        }
-    }
-    u += __shfl_xor(u, 16);
-    v += __shfl_xor(v, 16);
-    w += __shfl_xor(w, 16);
-    u += __shfl_xor(u, 32);
-    v += __shfl_xor(v, 32);
-    w += __shfl_xor(w, 32);
-    if (live && q == 0) {
-        float* o = part + (size_t)slice * 3 * np;
-        o[i] = u;
-        o[np + i] = v;
-        o[2 * (size_t)np + i] = w;
-    }
-}
-
-// BF16X3 form of k_vel_points_mma (contexts of precision RBC_BF16X3): the same six vertical sums
-// with every FP32 operand split into BF16 hi + lo halves and a.b ~ ah.bh + ah.bl + al.bh
-// accumulated in FP32 (v_mfma_f32_16x16x32_bf16, K = 32 in one instruction).  Lane (j, q) takes the
-// KPL = LMAX / 4 modes m = KPL q + e, e < KPL, at k = 8 q + e and zeros at the other k of its
-// slice, so that the basis values per lane stay balanced for every L.  The coefficients are split
-// once, when a tile is staged ([component][hi, lo][mode][m] BF16 in LDS); the basis values once per
-// particle.  Phases, combination, slices and prefetch as in k_vel_points_mma.
 typedef __bf16 vpbf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int vpu32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned short bf16_bits(float x) { return __builtin_bit_cast(unsigned short, (__bf16)x); }
 __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as_float((unsigned)h << 16); }
-template <int LMAX>
-__global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
+// The FP32 operands enter the products as sums of NS BF16 parts, each the rounded rest of the parts
+// before, over FP32 accumulators (v_mfma_f32_16x16x32_bf16).  NS = 3 (RBC_F32): a = a1 + a2 + a3 holds the 24
+// bits, and the six products a_i b_j with i + j <= 4 leave out terms below 2^-24 of a b; the small ones
+// are summed apart from a1 b1 (+ a2 b1), which keeps the error of the sums at or below that of the FP32
+// instructions (rms 1.0e-7 to 6.0e-7 against 1.2e-7 to 7.1e-7 where the phases are exact; in one
+// accumulator up to 2.1e-6).  NS = 2
+// (RBC_BF16X3, as the step's vertical transforms): a1 b1 + a1 b2 + a2 b1.  Lane (j, q) takes the KPL =
+// LMAX / 4 modes m = KPL q + e; up to L = 16 two products share an instruction, (a1 | a2) . (b | b') in
+// the lane's eight k, up to L = 8 (three parts) four.  The coefficients are split when a tile is staged, the basis values once per
+// particle.
+// With FP32 matrix instructions the six sums were 61 % of the kernel at L = 16 and the VALU the other
+// 40 %, without overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU now (107
+// instructions a sub-tile for the phases and the combination, of them about 30 for sincospi).  Two blocks
+// per CU (128 registers, one set of accumulators), so that one computes while the other stages: 1475
+// without at L = 16).  us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, L = 16 / 24 / 32:
+// FP32 1638 / 2677 / 3377 -> 1259 / 2047 / 2175, BF16X3 1439 / 1601 / 1686 -> 971 / 1181 / 1305; 64^2 x 8
+// 376 -> 351 and 436 -> 315.  At random positions the error
+// against FP64 (1e-6, from the rounded phases) is the same.
+template <int LMAX, int NS>
+__global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     DevGeom g, int np, const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
     const cpx<float>* __restrict__ Xf, const cpx<float>* __restrict__ Xg, const cpx<float>* __restrict__ XF,
     const cpx<float>* __restrict__ XG, const double* __restrict__ lam, const float4* __restrict__ modes,
     const int* __restrict__ pmap, int npad, int tiles_per_slice, float* __restrict__ part, const float4* __restrict__ zb) {
     static_assert(LMAX % 8 == 0 && LMAX <= 32, "KPL = LMAX / 4 even, at most 8");
     constexpr int KPL = LMAX / 4;
-    constexpr int RS = LMAX == 24 ? 40 : LMAX + 8;  // LDS row (BF16 values): 8-byte aligned, spreads the banks
+    constexpr bool PACK = KPL <= 4;  // two products in the eight k of a lane
+    constexpr bool QUAD = KPL == 2 && NS == 3;  // four
+    constexpr int NA = QUAD ? 1 : (PACK ? NS - 1 : NS);
+    constexpr int NB = QUAD ? 2 : NS;
     constexpr int NPAIR = kTile * LMAX / 2;         // (mode, pair of m) entries of a tile
     constexpr int PER = (NPAIR + kVelMmaThreads - 1) / kVelMmaThreads;
-    __shared__ unsigned int sa[4][2][kTile][RS / 2];  // [f.re, f.im, g.re, g.im][hi, lo][mode][m pair]
+    // [f.re, f.im, g.re, g.im][operand][mode][lane group q: 8 BF16], rows of 20 words: the 16 modes of a
+    // lane group start in different banks
+    __shared__ __align__(16) unsigned int sa[4][NA][kTile][20];
     __shared__ float4 sm[kTile];                      // (kx, ky, k^2, 0)
     __shared__ float2 sg[kTile / 4];                  // (kx index, ky index) of the first mode of each group of 4
     const int L = g.L, P = g.P, NYc = g.NYc;
@@ -677,14 +549,14 @@ __global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
     const int slice = blockIdx.y;
     const bool live = i < np;
     const float x = live ? px[i] : 0.f, y = live ? py[i] : 0.f, z = live ? pz[i] : 0.f;
-    // basis values of m = KPL q + e at the particle's height, split into BF16 hi and lo
-    vpbf16x8 bh[3], bl[3];  // C', C, S
+    // basis values of m = KPL q + e at the particle's height, split; bv[basis][operand]
+    vpbf16x8 bv[3][NB];  // C', C, S
     float ssf[KPL];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < KPL; ++e) {
         const int m = KPL * q + e;
         float val[3] = {0.f, 0.f, 0.f};
-        if (e < KPL && m < L) {
+        if (m < L) {
             if (zb) {  // computed once per evaluation by k_point_basis
                 if (live) {
                     const float4 t = zb[(size_t)i * L + m];
@@ -700,13 +572,49 @@ __global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
                 val[2] = (float)S;
             }
         }
+        ssf[e] = val[2];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            const unsigned short h = bf16_bits(val[k]);
-            bh[k][e] = __builtin_bit_cast(__bf16, h);
-            bl[k][e] = (__bf16)(val[k] - bf16_value(h));
+            __bf16 part[NS];
+            float rest = val[k];
+#pragma unroll
+            for (int n = 0; n < NS; ++n) {
+                part[n] = (__bf16)rest;
+                rest -= (float)part[n];
+            }
+            if constexpr (QUAD) {  // b1 | b1 | b2 | b1 and b3 | b2 | 0 | 0
+                bv[k][0][e] = bv[k][0][e + 2] = bv[k][0][e + 6] = part[0];
+                bv[k][0][e + 4] = bv[k][1][e + 2] = part[1];
+                bv[k][1][e] = part[2];
+                bv[k][1][e + 4] = bv[k][1][e + 6] = (__bf16)0.f;
+            } else if constexpr (PACK) {  // b1 | b1, then b2 | b2 and b3 | b1 (two parts: b2 | 0)
+                bv[k][0][e] = bv[k][0][e + 4] = part[0];
+                bv[k][1][e] = part[1];
+                bv[k][1][e + 4] = NS == 3 ? part[1] : (__bf16)0.f;
+                if constexpr (NS == 3) {
+                    bv[k][2][e] = part[2];
+                    bv[k][2][e + 4] = part[0];
+                }
+            } else {
+#pragma unroll
+                for (int n = 0; n < NS; ++n) bv[k][n][e] = part[n];
+            }
         }
-        if (e < KPL) ssf[e] = val[2];
+    }
+    // slots without a mode
+    if constexpr (!QUAD) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if ((PACK ? (e & 3) : e) >= KPL) bv[k][n][e] = (__bf16)0.f;
+    }
+    // the k slots without a mode are zero in every tile too
+    if constexpr (!QUAD && KPL != 4 && KPL != 8) {
+        for (int e = threadIdx.x; e < 4 * NA * kTile * 20; e += kVelMmaThreads) (&sa[0][0][0][0])[e] = 0u;
+        __syncthreads();
     }
     const float xr = x / (float)g.Lx - floorf(x / (float)g.Lx);
     const float yr = y / (float)g.Ly - floorf(y / (float)g.Ly);
@@ -753,12 +661,30 @@ __global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
         if (threadIdx.x < kTile)
             pmd = (int)threadIdx.x < nm ? modes[pbase + threadIdx.x] : make_float4(0.f, 0.f, 0.f, 0.f);
     };
-    // hi and lo BF16 of (a, b) packed into two 32-bit words (a in the low half)
-    auto split2 = [](float a, float b, unsigned int& hi, unsigned int& lo) {
-        const unsigned short ha = bf16_bits(a), hb = bf16_bits(b);
-        const unsigned short la = bf16_bits(a - bf16_value(ha)), lb = bf16_bits(b - bf16_value(hb));
-        hi = (unsigned int)ha | ((unsigned int)hb << 16);
-        lo = (unsigned int)la | ((unsigned int)lb << 16);
+    // the parts of (a, b), each pair in a word (a in the low half), to the operands of (mode, pair of m)
+    auto stage = [&](int c, int jj, int mp, float a, float b) {
+        unsigned int part[NS];
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+            const unsigned short ha = bf16_bits(a), hb = bf16_bits(b);
+            a -= bf16_value(ha);
+            b -= bf16_value(hb);
+            part[n] = (unsigned int)ha | ((unsigned int)hb << 16);
+        }
+        const int qq = mp / (KPL / 2), at = 4 * qq + mp - qq * (KPL / 2);
+        if constexpr (QUAD) {  // a1 | a2 | a1 | a3
+            *reinterpret_cast<uint4*>(&sa[c][0][jj][4 * mp]) = make_uint4(part[0], part[1], part[0], part[2]);
+        } else if constexpr (PACK) {  // a1 | a2 and a1 | a3
+            sa[c][0][jj][at] = part[0];
+            sa[c][0][jj][at + 2] = part[1];
+            if constexpr (NS == 3) {
+                sa[c][1][jj][at] = part[0];
+                sa[c][1][jj][at + 2] = part[2];
+            }
+        } else {
+#pragma unroll
+            for (int n = 0; n < NS; ++n) sa[c][n][jj][at] = part[n];
+        }
     };
     if (t0 < t1) fetch(t0);
     for (int t = t0; t < t1; ++t) {
@@ -769,19 +695,10 @@ __global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
             const int e = threadIdx.x + uu * kVelMmaThreads;
             if (e < NPAIR) {
                 const int jj = e / (LMAX / 2), mp = e - jj * (LMAX / 2);
-                unsigned int hi, lo;
-                split2(pf[uu].x, pf[uu].z, hi, lo);  // f.re at m, m + 1
-                sa[0][0][jj][mp] = hi;
-                sa[0][1][jj][mp] = lo;
-                split2(pf[uu].y, pf[uu].w, hi, lo);  // f.im
-                sa[1][0][jj][mp] = hi;
-                sa[1][1][jj][mp] = lo;
-                split2(pg[uu].x, pg[uu].z, hi, lo);  // g.re
-                sa[2][0][jj][mp] = hi;
-                sa[2][1][jj][mp] = lo;
-                split2(pg[uu].y, pg[uu].w, hi, lo);  // g.im
-                sa[3][0][jj][mp] = hi;
-                sa[3][1][jj][mp] = lo;
+                stage(0, jj, mp, pf[uu].x, pf[uu].z);  // f.re at m, m + 1
+                stage(1, jj, mp, pf[uu].y, pf[uu].w);  // f.im
+                stage(2, jj, mp, pg[uu].x, pg[uu].z);  // g.re
+                stage(3, jj, mp, pg[uu].y, pg[uu].w);  // g.im
             }
         }
         if (threadIdx.x < kTile) {
@@ -793,39 +710,38 @@ __global__ void __launch_bounds__(kVelMmaThreads) k_vel_points_bf3(
         const int nsub = (nm + 15) / 16;
         auto products = [&](int sub, vpf32x4 (&acc)[6]) {
             const int row = sub * 16 + j;
-            vpbf16x8 ah[4], al[4];
+            vpbf16x8 av[4][NA];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                vpu32x4 wh = {0u, 0u, 0u, 0u}, wl = {0u, 0u, 0u, 0u};
+            for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int e2 = 0; e2 < KPL / 2; ++e2) {
-                    wh[e2] = sa[c][0][row][(KPL * q) / 2 + e2];
-                    wl[e2] = sa[c][1][row][(KPL * q) / 2 + e2];
-                }
-                ah[c] = __builtin_bit_cast(vpbf16x8, wh);
-                al[c] = __builtin_bit_cast(vpbf16x8, wl);
-            }
+                for (int n = 0; n < NA; ++n)
+                    av[c][n] = __builtin_bit_cast(vpbf16x8, *reinterpret_cast<const vpu32x4*>(&sa[c][n][row][4 * q]));
             static constexpr int comp[6] = {0, 1, 0, 1, 2, 3}, kind[6] = {0, 0, 1, 1, 2, 2};
+            // one list of (A operand, B operand) per form, the smallest products first
+            static constexpr int pa[5][6] = {{0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 2, 1, 1, 0, 0}, {0, 0}};
+            static constexpr int pb[5][6] = {{1, 0}, {2, 1, 0}, {1, 0, 0}, {2, 0, 1, 0, 1, 0}, {1, 0}};
+            constexpr int F = QUAD ? 4 : (PACK ? 0 : 2) + NS - 2, NP = QUAD ? 2 : (PACK ? NS : (NS == 2 ? 3 : 6));
 #pragma unroll
             for (int k = 0; k < 6; ++k) {
+                auto mul = [&](int n, const vpf32x4& c) __attribute__((always_inline)) {
+                    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[comp[k]][pa[F][n]], bv[kind[k]][pb[F][n]], c, 0, 0, 0);
+                };
                 vpf32x4 a4 = {0.f, 0.f, 0.f, 0.f};
-                a4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[comp[k]], bh[kind[k]], a4, 0, 0, 0);
-                a4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[comp[k]], bl[kind[k]], a4, 0, 0, 0);
-                a4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[comp[k]], bh[kind[k]], a4, 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n + 1 < NP; ++n) a4 = mul(n, a4);
+                // three parts: the largest product in a sum of its own, added with one rounding
+                if constexpr (NS == 3) a4 += mul(NP - 1, vpf32x4{0.f, 0.f, 0.f, 0.f});
+                else a4 = mul(NP - 1, a4);
                 acc[k] = a4;
             }
         };
         auto combine = [&](int sub, const vpf32x4 (&acc)[6]) {
             vel_combine(sg, sm, sub * 16 + 4 * q, xr, yr, dc, ds, acc, u, v, w);
         };
-        vpf32x4 acc0[6], acc1[6];
-        products(0, acc0);
-#pragma unroll
-        for (int sub = 0; sub < kTile / 16; sub += 2) {
-            if (sub + 1 < nsub) products(sub + 1, acc1);
-            if (sub < nsub) combine(sub, acc0);
-            if (sub + 2 < nsub) products(sub + 2, acc0);
-            if (sub + 1 < nsub) combine(sub + 1, acc1);
+        for (int sub = 0; sub < nsub; ++sub) {
+            vpf32x4 acc[6];
+            products(sub, acc);
+            combine(sub, acc);
         }
     }
     u += __shfl_xor(u, 16);
@@ -1357,16 +1273,14 @@ void launch_points_t(rbc_ctx* c, int np, const float* x, const float* y, const f
                                z, (const double*)pw.lam, pw.zb);
         }
         dim3 grid((np + kVelMmaThreads / 4 - 1) / (kVelMmaThreads / 4), pw.nslice);
-        if (c->p.precision == RBC_BF16X3)  // BF16 hi/lo split products, as the step's vertical transforms
-            hipLaunchKernelGGL((k_vel_points_bf3<LM>), grid, dim3(kVelMmaThreads), 0, c->stream, c->dg, np, x, y, z,
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(kVelMmaThreads), 0, c->stream, c->dg, np, x, y, z,
                                (const cpx<float>*)b.X[1], (const cpx<float>*)b.X[2], (const cpx<float>*)b.XF,
                                (const cpx<float>*)b.XG, (const double*)pw.lam, pw.pmodes, pw.pmap, pw.npad,
                                pw.tiles_per_slice, pw.part, zb);
-        else
-            hipLaunchKernelGGL((k_vel_points_mma<LM>), grid, dim3(kVelMmaThreads), 0, c->stream, c->dg, np, x, y, z,
-                               (const cpx<float>*)b.X[1], (const cpx<float>*)b.X[2], (const cpx<float>*)b.XF,
-                               (const cpx<float>*)b.XG, (const double*)pw.lam, pw.pmodes, pw.pmap, pw.npad,
-                               pw.tiles_per_slice, pw.part, zb);
+        };
+        if (c->p.precision == RBC_BF16X3) go(k_vel_points_mma<LM, 2>);
+        else go(k_vel_points_mma<LM, 3>);
     } else {
         dim3 grid((np + 255) / 256, pw.nslice);
         hipLaunchKernelGGL((k_vel_points<T, LM>), grid, dim3(256), 0, c->stream, c->dg, np, x, y, z,
