@@ -79,11 +79,11 @@ def fft_product_stage(st, stages, cs):
     return out
 
 
-# kernels of each stage on the 512 x 512 FP32 path (BF16X3 runs the <1> variants of the two
-# matrix-core kernels, with the same memory traffic)
-STAGE_KERNELS = {"eval": ["k_eval_mma<0, false>"], "fft_y_inv": ["k_fft_y_inv512"], "rows_products": ["k_rows512t"],
+# kernels of each stage on the 512 x 512 FP32 path (BF16X3 runs k_eval_mma and k_project_mma for the
+# vertical transforms, with the same algorithmic traffic)
+STAGE_KERNELS = {"eval": ["k_eval_plain<8>"], "fft_y_inv": ["k_fft_y_inv512"], "rows_products": ["k_rows512t"],
                  "fft_y_fwd": ["k_fft_y_fwd512c2<8>"],
-                 "project": ["k_project_mma<0, 4, 1>"], "update": ["k_update<float, 32, 32, 0>"], "finish": []}
+                 "project": ["k_project_plain<1>"], "update": ["k_update<float, 32, 32, 0>"], "finish": []}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "hbm_traffic_512x512x32_f32.md")
 
 
