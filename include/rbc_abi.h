@@ -41,7 +41,7 @@ extern "C" {
  *   RBC_BF16X3 : as RBC_F32, but the vertical transforms run as BF16 hi/lo split MFMA
  *                products accumulated in FP32 (L <= 32, and one level combination of
  *                2 nq P floats below 2^31 bytes; rbc_create refuses larger grids with
- *                RBC_ERR_ARG, where RBC_F32 falls back to VALU vertical transforms)
+ *                RBC_ERR_ARG, where RBC_F32 takes a form without that limit)
  * Per-wavenumber factors are always built in FP64 on the host. */
 typedef enum { RBC_F64 = 0, RBC_F32 = 1, RBC_BF16X3 = 2 } rbc_precision;
 
@@ -221,7 +221,8 @@ int rbc_nusselt(rbc_ctx* c, double* nu3);
 
 /* Per-stage timing with HIP events on the context's stream: runs nsteps steps and writes
  * the mean milliseconds per call of each stage into ms[RBC_NSTAGES] (stage names from
- * rbc_stage_name). */
+ * rbc_stage_name; the last, "finish", is part of the update and reads as the time between two
+ * events). */
 #define RBC_NSTAGES 7
 int rbc_profile_steps(rbc_ctx* c, int nsteps, double* ms);
 const char* rbc_stage_name(int i);
