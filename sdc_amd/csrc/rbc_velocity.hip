@@ -467,12 +467,35 @@ __global__ void __launch_bounds__(256) k_vel_points(DevGeom g, int np, const flo
 // rows of the same particles and are added at the end.  The weight w_k (1 at kx = 0, else 2) is
 // folded into the staged coefficients.  The modes come
 // from the padded list (padded_mode_table), where the 4 rows of a lane group share kx and have
-// consecutive ky: one sincospi per group gives exp(2 pi i k.x) of its first row, and the others
+// consecutive ky: one sincos_turn per group gives exp(2 pi i k.x) of its first row, and the others
 // follow by a complex product with exp(2 pi i r y / Ly), r = 1, 2, 3, taken once per particle.
 // The coefficients of the next 64-mode tile are loaded into registers while the current tile is
 // computed, across LDS-only barriers.
 typedef float vpf32x4 __attribute__((ext_vector_type(4)));
 constexpr int kVelMmaThreads = 512;  // 8 waves
+
+// sin and cos of 2 pi ph: the nearest quarter turn off (exact: both are multiples of ph's last bit), then
+// the Taylor sums of the rest, |2 pi r| <= pi / 4 (terms left out below 2e-9), and the quadrant's swap and signs.
+// Largest error 8.4e-8 over |ph| < 90.  A tracer step at 128^2 x 16 (spectral RK2):
+// 1280 -> 1230 us FP32, 985 -> 940 BF16X3 against sincospif.
+__device__ __forceinline__ void sincos_turn(float ph, float& sn, float& cs) {
+    const float n = rintf(4.0f * ph), r = fmaf(-0.25f, n, ph), t = r * r;
+    float s = 42.058692932128906f, c = -26.42625617980957f;
+    s = fmaf(s, t, -76.70585632324219f);
+    s = fmaf(s, t, 81.6052474975586f);
+    s = fmaf(s, t, -41.34170150756836f);
+    s = fmaf(s, t, 6.2831854820251465f);
+    c = fmaf(c, t, 60.2446403503418f);
+    c = fmaf(c, t, -85.45681762695312f);
+    c = fmaf(c, t, 64.93939208984375f);
+    c = fmaf(c, t, -19.739208221435547f);
+    s *= r;
+    c = fmaf(c, t, 1.0f);
+    const int q = (int)n;
+    const float a = q & 1 ? c : s, b = q & 1 ? s : c;
+    sn = __int_as_float(__float_as_int(a) ^ ((q & 2) << 30));
+    cs = __int_as_float(__float_as_int(b) ^ (((q + 1) & 2) << 30));
+}
 
 // phases and velocity combination of one 16-mode sub-tile in the MFMA output layout of
 // v_mfma_f32_16x16x*: lane l holds its particle's (column l % 16) mode rows b0 + r, r < 4, with
@@ -483,9 +506,7 @@ __device__ __forceinline__ void vel_combine(const float2* sg, const float4* sm, 
     float s0, c0;
     {
         const float2 m0 = sg[b0 >> 2];
-        float ph = m0.x * xr + m0.y * yr;
-        ph -= rintf(ph);
-        sincospif(2.0f * ph, &s0, &c0);
+        sincos_turn(m0.x * xr + m0.y * yr, s0, c0);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -518,11 +539,11 @@ __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as
 // particle.
 // With FP32 matrix instructions the six sums were 61 % of the kernel at L = 16 and the VALU the other
 // 40 %, without overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU now (107
-// instructions a sub-tile for the phases and the combination, of them about 30 for sincospi).  Two blocks
+// instructions a sub-tile for the phases and the combination with sincospif, about 90 with sincos_turn).  Two blocks
 // per CU (128 registers, one set of accumulators), so that one computes while the other stages: 1475
 // without at L = 16).  us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, L = 16 / 24 / 32:
-// FP32 1638 / 2677 / 3377 -> 1259 / 2047 / 2175, BF16X3 1439 / 1601 / 1686 -> 971 / 1181 / 1305; 64^2 x 8
-// 376 -> 351 and 436 -> 315.  At random positions the error
+// FP32 1638 / 2677 / 3377 -> 1230 / 1950 / 2165, BF16X3 1439 / 1601 / 1686 -> 940 / 1162 / 1293; 64^2 x 8
+// 376 -> 345 and 436 -> 307.  At random positions the error
 // against FP64 (1e-6, from the rounded phases) is the same.
 template <int LMAX, int NS>
 __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
