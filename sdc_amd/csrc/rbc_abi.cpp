@@ -392,12 +392,20 @@ int rbc_create(const rbc_params* p, rbc_ctx** out) {
         HIPCHK(hipMemcpy(b.rows, g.rows.data(), g.rows.size() * sizeof(int), hipMemcpyHostToDevice));
         b.gmem = (int*)c->dalloc(c->fac.members.size() * sizeof(int));
         HIPCHK(hipMemcpy(b.gmem, c->fac.members.data(), c->fac.members.size() * sizeof(int), hipMemcpyHostToDevice));
-        {  // chunks of members, one chunk per wave of the group update: a wave runs its members
-           // one after another, so small grids (few modes, a few thousand waves at most) take one
-           // member per wave; larger grids take 4, which matches the usual group size (the
-           // (+-kx, +-ky) images of a mode) and shares the group's matrix loads (measured at
-           // 512^2 x 32: 98 us with 4, 103 us with 2, 116 us with 8 members per chunk)
-            const int kChunk = g.P() >= 8192 ? kUpdateChunk : 1;
+        {  // chunks of members, one chunk per wave of the group update: a wave shares the group's matrices
+           // among its members and runs them one after another, so grids with few modes, where the
+           // waves are few, take one member per wave unless the matrices are the larger part.  Update
+           // stage, us with 1 / 2 / 4 members: 512^2 x 32 FP32 102 / 80 / 75, 256^2 x 24 FP64 49 / 41 / 35
+           // (8192 modes and more: 4); 128^2 (3740 modes) x 40 FP32 25.8 / 19.9 / 15.9, x 48 FP64 54 / 41 / 33
+           // (L > 32: 4), x 24 FP32 12.3 / 10.6 / 12.1, x 16 FP64 11.3 / 10.0 / 10.7 (records above 4 KiB: 2),
+           // x 16 FP32 8.2 / 8.4 / 9.8; 128 x 64 (1892 modes) x 24 FP64 10.1 / 10.7 / 10.8, 32^2 x 8 FP64 6.7 /
+           // 8.1 / 10.0 (1)
+            const size_t rec = (size_t)c->fac.stride * c->rsz;
+            const int kChunk = g.P() >= 8192 ? kUpdateChunk
+                               : g.P() < 2048 ? 1
+                               : p->L > 32    ? kUpdateChunk
+                               : rec > 4096   ? 2
+                                              : 1;
             std::vector<int> cg, cb;
             const auto& gs = c->fac.group_start;
             for (int gi = 0; gi + 1 < (int)gs.size(); ++gi)

@@ -67,7 +67,7 @@ __device__ __forceinline__ T g_factor(T k2, T mpi, T dtPr) {
 // and of three members are in flight at once; everything after them is registers and LDS broadcasts.
 // us a step, against one block of 64 lanes per group with the matrices read per member from memory
 // (W = 64) and a kernel whose FP64 members lived in scratch memory (W = 32): 1024 x 128 x 40 FP32
-// 217 -> 120, 128^2 x 48 FP64 396 -> 57, 256^2 x 24 FP64 45 -> 36, 128^2 x 16 FP32 9.8 -> 8.2; 512^2
+// 217 -> 120, 128^2 x 48 FP64 396 -> 33, 256^2 x 24 FP64 45 -> 36, 128^2 x 16 FP32 9.8 -> 8.2; 512^2
 // x 32 FP32 72 + 6 (the end of the step apart) -> 75.  Allocations held to one more wave per SIMD
 // (launch bounds) cost 1 to 2 us at each of these sizes.
 //
