@@ -474,22 +474,24 @@ __global__ void __launch_bounds__(256) k_vel_points(DevGeom g, int np, const flo
 typedef float vpf32x4 __attribute__((ext_vector_type(4)));
 constexpr int kVelMmaThreads = 512;  // 8 waves
 
-// sin and cos of 2 pi ph: the nearest quarter turn off (exact: both are multiples of ph's last bit), then
-// the Taylor sums of the rest, |2 pi r| <= pi / 4 (terms left out below 2e-9), and the quadrant's swap and signs.
-// Largest error 8.4e-8 over |ph| < 90.  A tracer step at 128^2 x 16 (spectral RK2):
+// sin and cos of 2 pi ph: the nearest quarter turn off, and the quadrant's swap and signs.  The rest r,
+// |2 pi r| <= pi / 4, is exact for every ph below 2^22 (ph and n / 4 are multiples of ph's last bit), so the
+// error is that of the two polynomials at any grid's phases: at most 5.2e-8, 1.50e-8 rms (sincospif: 5.1e-8
+// and 1.50e-8).  sin = r (2 pi + t s(t)), t = r^2, with 2 pi as a sum of two floats, so that only the last fma rounds
+// at the size of the result; cos = 1 + t c(t).  The coefficients have the smallest largest error over |r| <= 1/8 (below
+// 1e-9), each rounded before the next ones are fitted.  A tracer step at 128^2 x 16 (spectral RK2):
 // 1280 -> 1230 us FP32, 985 -> 940 BF16X3 against sincospif.
 __device__ __forceinline__ void sincos_turn(float ph, float& sn, float& cs) {
     const float n = rintf(4.0f * ph), r = fmaf(-0.25f, n, ph), t = r * r;
-    float s = 42.058692932128906f, c = -26.42625617980957f;
-    s = fmaf(s, t, -76.70585632324219f);
-    s = fmaf(s, t, 81.6052474975586f);
+    float s = 40.53968811035156f, c = 58.561214447021484f;
+    s = fmaf(s, t, -76.66972351074219f);
+    s = fmaf(s, t, 81.60494995117188f);
     s = fmaf(s, t, -41.34170150756836f);
-    s = fmaf(s, t, 6.2831854820251465f);
-    c = fmaf(c, t, 60.2446403503418f);
-    c = fmaf(c, t, -85.45681762695312f);
-    c = fmaf(c, t, 64.93939208984375f);
+    s = fmaf(s, t, -1.7484555e-7f);  // 2 pi - 6.2831855f
+    s = fmaf(r, 6.2831855f, r * s);
+    c = fmaf(c, t, -85.4231185913086f);
+    c = fmaf(c, t, 64.93914031982422f);
     c = fmaf(c, t, -19.739208221435547f);
-    s *= r;
     c = fmaf(c, t, 1.0f);
     const int q = (int)n;
     const float a = q & 1 ? c : s, b = q & 1 ? s : c;
