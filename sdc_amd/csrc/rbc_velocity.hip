@@ -529,24 +529,24 @@ typedef __bf16 vpbf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int vpu32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned short bf16_bits(float x) { return __builtin_bit_cast(unsigned short, (__bf16)x); }
 __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as_float((unsigned)h << 16); }
-// The FP32 operands enter the products as sums of NS BF16 parts, each the rounded rest of the parts
-// before, over FP32 accumulators (v_mfma_f32_16x16x32_bf16).  NS = 3 (RBC_F32): a = a1 + a2 + a3 holds the 24
-// bits, and the six products a_i b_j with i + j <= 4 leave out terms below 2^-24 of a b; the small ones
-// are summed apart from a1 b1 (+ a2 b1), which keeps the error of the sums at or below that of the FP32
-// instructions (rms 1.0e-7 to 6.0e-7 against 1.2e-7 to 7.1e-7 where the phases are exact; in one
-// accumulator up to 2.1e-6).  NS = 2
-// (RBC_BF16X3, as the step's vertical transforms): a1 b1 + a1 b2 + a2 b1.  Lane (j, q) takes the KPL =
-// LMAX / 4 modes m = KPL q + e; up to L = 16 two products share an instruction, (a1 | a2) . (b | b') in
-// the lane's eight k, up to L = 8 (three parts) four.  The coefficients are split when a tile is staged, the basis values once per
-// particle.
-// With FP32 matrix instructions the six sums were 61 % of the kernel at L = 16 and the VALU the other
-// 40 %, without overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU now (107
-// instructions a sub-tile for the phases and the combination with sincospif, about 90 with sincos_turn).  Two blocks
-// per CU (128 registers, one set of accumulators), so that one computes while the other stages: 1475
-// without at L = 16).  us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, L = 16 / 24 / 32:
-// FP32 1638 / 2677 / 3377 -> 1230 / 1950 / 2165, BF16X3 1439 / 1601 / 1686 -> 940 / 1162 / 1293; 64^2 x 8
-// 376 -> 345 and 436 -> 307.  At random positions the error
-// against FP64 (1e-6, from the rounded phases) is the same.
+// NS = 1 (RBC_F32, L <= 8): v_mfma_f32_16x16x4_f32, a chain of FMAs in the order of m.  Else the FP32 operands enter as
+// sums of NS BF16 parts, each the rounded rest of the parts before, over FP32 accumulators
+// (v_mfma_f32_16x16x32_bf16).  NS = 3 (RBC_F32): a = a1 + a2 + a3 holds the 24 bits, and the six products a_i b_j with
+// i + j <= 4 are summed (a2 b3 and a3 b2, left out, reach 2^-24 of a b together), a1 b1 apart from the small ones and
+// added to them with one rounding: its 16-bit terms add nearly without rounding, and less so with a small product beside
+// it in the instruction.  NS = 2 (RBC_BF16X3, as the step's vertical transforms): a1 b1 + a1 b2 + a2 b1.
+// Lane (j, q) takes the KPL = LMAX / 4 modes m = KPL q + e (NS = 1: 4 e + q); up to L = 16 two products share an
+// instruction, (a | a') . (b | b') in the lane's eight k.  The coefficients are split when a tile is staged, the basis
+// values once per particle.
+// Error of a vertical sum, rms over 20,000 heights against the FMA chain's, the largest of the six sums of two random
+// states: L <= 8 the same (three parts there 1.2 to 2.1, and 1.05 at L = 5 with a1 b1 apart, for 921 us at L = 8), 9 <= L <= 16
+// 0.56 to 0.96 (with a2 b1 beside a1 b1, an instruction less, 1140 us at L = 16: up to 1.27), L > 16 0.55 to 0.73.
+// us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, all FP32 instructions -> now, same box: L = 4 / 8 / 10 / 16 /
+// 24 / 32 972 / 995 / 1569 / 1602 / 2658 / 3375 -> 920 / 941 / 1156 / 1250 / 1894 / 2125; BF16X3, L = 8 / 16 1185 / 1412 -> 712 / 856.
+// With FP32 instructions the six sums are 61 % of the kernel at L = 16 and the VALU the other 40 %, without
+// overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU (about 90 instructions a sub-tile for the
+// phases and the combination) and the 24 or 36 products (NS = 1: 6 or 12 of twice the cycles) about alike.  Two blocks per CU
+// (128 registers, one set of accumulators), so that one computes while the other stages: with one 1475 against 1207 us at L = 16.
 template <int LMAX, int NS>
 __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     DevGeom g, int np, const float* __restrict__ px, const float* __restrict__ py, const float* __restrict__ pz,
@@ -555,15 +555,14 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     const int* __restrict__ pmap, int npad, int tiles_per_slice, float* __restrict__ part, const float4* __restrict__ zb) {
     static_assert(LMAX % 8 == 0 && LMAX <= 32, "KPL = LMAX / 4 even, at most 8");
     constexpr int KPL = LMAX / 4;
-    constexpr bool PACK = KPL <= 4;  // two products in the eight k of a lane
-    constexpr bool QUAD = KPL == 2 && NS == 3;  // four
-    constexpr int NA = QUAD ? 1 : (PACK ? NS - 1 : NS);
-    constexpr int NB = QUAD ? 2 : NS;
+    constexpr bool PACK = NS > 1 && KPL <= 4;  // two products in the eight k of a lane
+    constexpr int NA = PACK ? NS - 1 : NS, NB = NS;
     constexpr int NPAIR = kTile * LMAX / 2;         // (mode, pair of m) entries of a tile
     constexpr int PER = (NPAIR + kVelMmaThreads - 1) / kVelMmaThreads;
     // [f.re, f.im, g.re, g.im][operand][mode][lane group q: 8 BF16], rows of 20 words: the 16 modes of a
-    // lane group start in different banks
-    __shared__ __align__(16) unsigned int sa[4][NA][kTile][20];
+    // lane group start in different banks.  NS = 1: [mode][m] (f.re, f.im, g.re, g.im), odd row length
+    __shared__ __align__(16) unsigned int sa[4][NA][NS == 1 ? 1 : kTile][20];
+    __shared__ float4 sc[NS == 1 ? kTile : 1][LMAX + 1];
     __shared__ float4 sm[kTile];                      // (kx, ky, k^2, 0)
     __shared__ float2 sg[kTile / 4];                  // (kx index, ky index) of the first mode of each group of 4
     const int L = g.L, P = g.P, NYc = g.NYc;
@@ -572,12 +571,13 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     const int slice = blockIdx.y;
     const bool live = i < np;
     const float x = live ? px[i] : 0.f, y = live ? py[i] : 0.f, z = live ? pz[i] : 0.f;
-    // basis values of m = KPL q + e at the particle's height, split; bv[basis][operand]
+    auto mode = [&](int e) { return NS == 1 ? 4 * e + q : KPL * q + e; };
+    // basis values of the lane's modes at the particle's height, split; bv[basis][operand]
     vpbf16x8 bv[3][NB];  // C', C, S
-    float ssf[KPL];
+    float bf[3][KPL];
 #pragma unroll
     for (int e = 0; e < KPL; ++e) {
-        const int m = KPL * q + e;
+        const int m = mode(e);
         float val[3] = {0.f, 0.f, 0.f};
         if (m < L) {
             if (zb) {  // computed once per evaluation by k_point_basis
@@ -595,9 +595,9 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
                 val[2] = (float)S;
             }
         }
-        ssf[e] = val[2];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
+            bf[k][e] = val[k];
             __bf16 part[NS];
             float rest = val[k];
 #pragma unroll
@@ -605,18 +605,15 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
                 part[n] = (__bf16)rest;
                 rest -= (float)part[n];
             }
-            if constexpr (QUAD) {  // b1 | b1 | b2 | b1 and b3 | b2 | 0 | 0
-                bv[k][0][e] = bv[k][0][e + 2] = bv[k][0][e + 6] = part[0];
-                bv[k][0][e + 4] = bv[k][1][e + 2] = part[1];
-                bv[k][1][e] = part[2];
-                bv[k][1][e + 4] = bv[k][1][e + 6] = (__bf16)0.f;
-            } else if constexpr (PACK) {  // b1 | b1, then b2 | b2 and b3 | b1 (two parts: b2 | 0)
-                bv[k][0][e] = bv[k][0][e + 4] = part[0];
+            if constexpr (PACK) {  // three parts b1 | 0, b2 | b1 and b3 | b2, two parts b1 | b1 and b2 | 0
+                const __bf16 o = (__bf16)0.f;
+                bv[k][0][e] = part[0];
+                bv[k][0][e + 4] = NS == 3 ? o : part[0];
                 bv[k][1][e] = part[1];
-                bv[k][1][e + 4] = NS == 3 ? part[1] : (__bf16)0.f;
+                bv[k][1][e + 4] = NS == 3 ? part[0] : o;
                 if constexpr (NS == 3) {
                     bv[k][2][e] = part[2];
-                    bv[k][2][e + 4] = part[0];
+                    bv[k][2][e + 4] = part[1];
                 }
             } else {
 #pragma unroll
@@ -624,8 +621,7 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
             }
         }
     }
-    // slots without a mode
-    if constexpr (!QUAD) {
+    if constexpr (NS > 1 && KPL != 4 && KPL != 8) {  // the k slots without a mode are zero in every tile
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
@@ -633,9 +629,6 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     if ((PACK ? (e & 3) : e) >= KPL) bv[k][n][e] = (__bf16)0.f;
-    }
-    // the k slots without a mode are zero in every tile too
-    if constexpr (!QUAD && KPL != 4 && KPL != 8) {
         for (int e = threadIdx.x; e < 4 * NA * kTile * 20; e += kVelMmaThreads) (&sa[0][0][0][0])[e] = 0u;
         __syncthreads();
     }
@@ -651,10 +644,10 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     if (slice == 0) {  // mean flow (k = 0), each lane group its KPL modes
 #pragma unroll
         for (int e = 0; e < KPL; ++e) {
-            const int m = KPL * q + e;
+            const int m = mode(e);
             if (m < L) {
-                u += ssf[e] * XF[m].x;
-                v += ssf[e] * XG[m].x;
+                u += bf[2][e] * XF[m].x;
+                v += bf[2][e] * XG[m].x;
             }
         }
     }
@@ -695,14 +688,12 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
             part[n] = (unsigned int)ha | ((unsigned int)hb << 16);
         }
         const int qq = mp / (KPL / 2), at = 4 * qq + mp - qq * (KPL / 2);
-        if constexpr (QUAD) {  // a1 | a2 | a1 | a3
-            *reinterpret_cast<uint4*>(&sa[c][0][jj][4 * mp]) = make_uint4(part[0], part[1], part[0], part[2]);
-        } else if constexpr (PACK) {  // a1 | a2 and a1 | a3
+        if constexpr (PACK) {  // a1 | a2, and of three parts a3 | a2
             sa[c][0][jj][at] = part[0];
             sa[c][0][jj][at + 2] = part[1];
             if constexpr (NS == 3) {
-                sa[c][1][jj][at] = part[0];
-                sa[c][1][jj][at + 2] = part[2];
+                sa[c][1][jj][at] = part[2];
+                sa[c][1][jj][at + 2] = part[1];
             }
         } else {
 #pragma unroll
@@ -718,10 +709,16 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
             const int e = threadIdx.x + uu * kVelMmaThreads;
             if (e < NPAIR) {
                 const int jj = e / (LMAX / 2), mp = e - jj * (LMAX / 2);
-                stage(0, jj, mp, pf[uu].x, pf[uu].z);  // f.re at m, m + 1
-                stage(1, jj, mp, pf[uu].y, pf[uu].w);  // f.im
-                stage(2, jj, mp, pg[uu].x, pg[uu].z);  // g.re
-                stage(3, jj, mp, pg[uu].y, pg[uu].w);  // g.im
+                const float4 f = pf[uu], gg = pg[uu];
+                if constexpr (NS == 1) {
+                    sc[jj][2 * mp] = make_float4(f.x, f.y, gg.x, gg.y);
+                    sc[jj][2 * mp + 1] = make_float4(f.z, f.w, gg.z, gg.w);
+                } else {
+                    stage(0, jj, mp, f.x, f.z);  // f.re at m, m + 1
+                    stage(1, jj, mp, f.y, f.w);  // f.im
+                    stage(2, jj, mp, gg.x, gg.z);  // g.re
+                    stage(3, jj, mp, gg.y, gg.w);  // g.im
+                }
             }
         }
         if (threadIdx.x < kTile) {
@@ -733,29 +730,43 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
         const int nsub = (nm + 15) / 16;
         auto products = [&](int sub, vpf32x4 (&acc)[6]) {
             const int row = sub * 16 + j;
-            vpbf16x8 av[4][NA];
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int n = 0; n < NA; ++n)
-                    av[c][n] = __builtin_bit_cast(vpbf16x8, *reinterpret_cast<const vpu32x4*>(&sa[c][n][row][4 * q]));
             static constexpr int comp[6] = {0, 1, 0, 1, 2, 3}, kind[6] = {0, 0, 1, 1, 2, 2};
-            // one list of (A operand, B operand) per form, the smallest products first
-            static constexpr int pa[5][6] = {{0, 0}, {1, 0, 0}, {0, 1, 0}, {0, 2, 1, 1, 0, 0}, {0, 0}};
-            static constexpr int pb[5][6] = {{1, 0}, {2, 1, 0}, {1, 0, 0}, {2, 0, 1, 0, 1, 0}, {1, 0}};
-            constexpr int F = QUAD ? 4 : (PACK ? 0 : 2) + NS - 2, NP = QUAD ? 2 : (PACK ? NS : (NS == 2 ? 3 : 6));
+            if constexpr (NS == 1) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                auto mul = [&](int n, const vpf32x4& c) __attribute__((always_inline)) {
-                    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[comp[k]][pa[F][n]], bv[kind[k]][pb[F][n]], c, 0, 0, 0);
-                };
-                vpf32x4 a4 = {0.f, 0.f, 0.f, 0.f};
+                for (int k = 0; k < 6; ++k) acc[k] = vpf32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int n = 0; n + 1 < NP; ++n) a4 = mul(n, a4);
-                // three parts: the largest product in a sum of its own, added with one rounding
-                if constexpr (NS == 3) a4 += mul(NP - 1, vpf32x4{0.f, 0.f, 0.f, 0.f});
-                else a4 = mul(NP - 1, a4);
-                acc[k] = a4;
+                for (int e = 0; e < KPL; ++e) {
+                    const float4 c4 = sc[row][4 * e + q];
+                    const float a[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+                    for (int k = 0; k < 6; ++k)
+                        acc[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[comp[k]], bf[kind[k]][e], acc[k], 0, 0, 0);
+                }
+            } else {
+                vpbf16x8 av[4][NA];
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int n = 0; n < NA; ++n)
+                        av[c][n] = __builtin_bit_cast(vpbf16x8, *reinterpret_cast<const vpu32x4*>(&sa[c][n][row][4 * q]));
+                // one list of (A operand, B operand) per form, the smallest products first
+                static constexpr int pa[4][6] = {{0, 0}, {1, 0, 0, 0}, {0, 1, 0}, {0, 2, 1, 1, 0, 0}};
+                static constexpr int pb[4][6] = {{1, 0}, {0, 2, 1, 0}, {1, 0, 0}, {2, 0, 1, 0, 1, 0}};
+                static constexpr int count[4] = {2, 4, 3, 6};
+                constexpr int F = (PACK ? 0 : 2) + NS - 2, NP = count[F];
+#pragma unroll
+                for (int k = 0; k < 6; ++k) {
+                    auto mul = [&](int n, const vpf32x4& c) __attribute__((always_inline)) {
+                        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[comp[k]][pa[F][n]], bv[kind[k]][pb[F][n]], c, 0, 0, 0);
+                    };
+                    vpf32x4 a4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int n = 0; n + 1 < NP; ++n) a4 = mul(n, a4);
+                    // three parts: the largest product in a sum of its own, added with one rounding
+                    if constexpr (NS == 3) a4 += mul(NP - 1, vpf32x4{0.f, 0.f, 0.f, 0.f});
+                    else a4 = mul(NP - 1, a4);
+                    acc[k] = a4;
+                }
             }
         };
         auto combine = [&](int sub, const vpf32x4 (&acc)[6]) {
@@ -1303,7 +1314,7 @@ void launch_points_t(rbc_ctx* c, int np, const float* x, const float* y, const f
                                pw.tiles_per_slice, pw.part, zb);
         };
         if (c->p.precision == RBC_BF16X3) go(k_vel_points_mma<LM, 2>);
-        else go(k_vel_points_mma<LM, 3>);
+        else go(k_vel_points_mma<LM, LM == 8 ? 1 : 3>);
     } else {
         dim3 grid((np + 255) / 256, pw.nslice);
         hipLaunchKernelGGL((k_vel_points<T, LM>), grid, dim3(256), 0, c->stream, c->dg, np, x, y, z,
