@@ -542,7 +542,7 @@ __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as
 // states: L <= 8 the same (three parts there 1.2 to 2.1, and 1.05 at L = 5 with a1 b1 apart, for 921 us at L = 8), 9 <= L <= 16
 // 0.56 to 0.96 (with a2 b1 beside a1 b1, an instruction less, 1140 us at L = 16: up to 1.27), L > 16 0.55 to 0.73.
 // us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, all FP32 instructions -> now, same box: L = 4 / 8 / 10 / 16 /
-// 24 / 32 972 / 995 / 1569 / 1602 / 2658 / 3375 -> 920 / 941 / 1156 / 1250 / 1894 / 2125; BF16X3, L = 8 / 16 1185 / 1412 -> 712 / 856.
+// 24 / 32 972 / 995 / 1569 / 1602 / 2658 / 3375 -> 921 / 941 / 1166 / 1249 / 1837 / 2030; BF16X3, L = 8 / 16 1185 / 1412 -> 705 / 846.
 // With FP32 instructions the six sums are 61 % of the kernel at L = 16 and the VALU the other 40 %, without
 // overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU (about 90 instructions a sub-tile for the
 // phases and the combination) and the 24 or 36 products (NS = 1: 6 or 12 of twice the cycles) about alike.  Two blocks per CU
@@ -565,6 +565,7 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
     __shared__ float4 sc[NS == 1 ? kTile : 1][LMAX + 1];
     __shared__ float4 sm[kTile];                      // (kx, ky, k^2, 0)
     __shared__ float2 sg[kTile / 4];                  // (kx index, ky index) of the first mode of each group of 4
+    __shared__ int sbig[2];                           // NS = 3: a coefficient of the tile (two in turn) is 2^-80 or more
     const int L = g.L, P = g.P, NYc = g.NYc;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, q = lane >> 4;
     const int i = blockIdx.x * (kVelMmaThreads / 4) + wave * 16 + j;
@@ -700,10 +701,36 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
             for (int n = 0; n < NS; ++n) sa[c][n][jj][at] = part[n];
         }
     };
+    if constexpr (NS == 3) {
+        if (threadIdx.x < 2) sbig[threadIdx.x] = 0;
+        lds_barrier();
+    }
     if (t0 < t1) fetch(t0);
     for (int t = t0; t < t1; ++t) {
         const int nm = min(kTile, npad - t * kTile);
+        // The last of three parts of a number below 2^-109 falls under the BF16 range: a tile whose coefficients
+        // are all below 2^-80 is staged times 2^64, and its kx, ky and k^2 times 2^-64 (the check: 1230 -> 1249 us
+        // a step at L = 16, 1885 -> 1837 at L = 24).  An infinite coefficient gives NaN: its rest is inf - inf.
+        if constexpr (NS == 3) {
+            float big = 0.f;
+#pragma unroll
+            for (int uu = 0; uu < PER; ++uu)
+                for (const float4& c4 : {pf[uu], pg[uu]})
+                    big = fmaxf(big, fmaxf(fmaxf(fabsf(c4.x), fabsf(c4.y)), fmaxf(fabsf(c4.z), fabsf(c4.w))));
+            if (__any(big >= 0x1p-80f) && lane == 0) sbig[t & 1] = 1;
+        }
         lds_barrier();  // the previous tile is consumed
+        float down = 1.f;
+        if constexpr (NS == 3) {
+            if (threadIdx.x == 0) sbig[(t + 1) & 1] = 0;
+            if (!__builtin_amdgcn_readfirstlane(sbig[t & 1])) {
+                down = 0x1p-64f;
+#pragma unroll
+                for (int uu = 0; uu < PER; ++uu)
+                    for (float4* c4 : {&pf[uu], &pg[uu]})
+                        *c4 = make_float4(c4->x * 0x1p64f, c4->y * 0x1p64f, c4->z * 0x1p64f, c4->w * 0x1p64f);
+            }
+        }
 #pragma unroll
         for (int uu = 0; uu < PER; ++uu) {
             const int e = threadIdx.x + uu * kVelMmaThreads;
@@ -722,7 +749,7 @@ __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(
             }
         }
         if (threadIdx.x < kTile) {
-            sm[threadIdx.x] = make_float4(pmd.z, pmd.w, pmd.z * pmd.z + pmd.w * pmd.w, 0.f);
+            sm[threadIdx.x] = make_float4(pmd.z * down, pmd.w * down, (pmd.z * pmd.z + pmd.w * pmd.w) * down, 0.f);
             if ((threadIdx.x & 3) == 0) sg[threadIdx.x >> 2] = make_float2(pmd.x, pmd.y);
         }
         lds_barrier();

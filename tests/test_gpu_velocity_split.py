@@ -62,3 +62,32 @@ def test_vertical_sums_bf16x3(L):
     print(f"case: vertical sums bf16x3 L={L}", flush=True)
     for got, c, b in _sums(L, "bf16x3", L):
         assert np.all(np.abs(got - c @ b) <= 2.0 ** -15 * (np.abs(c) @ np.abs(b)))
+
+
+@pytest.mark.parametrize("k", [60, 84, 100, 112])
+@pytest.mark.parametrize("L", [6, 11, 20, 31])
+def test_velocity_of_a_state_times_a_power_of_two(L, k):
+    """2^-k times a state of coefficients of size 1/2 to 2 has 2^-k times its velocity.  Products and sums scale
+    exactly as long as they stay above 2^-126; a term of a sum that falls below is held to 2^-150, and at k = 112
+    the 2 * 16 * 21 modes' terms, each below 2^-111 in a sum above 2^-109 in the root mean square, to 672 * 2^-150 < 2^-31 of it; the
+    last steps round at 2^-24 again, three times: 2^-22 of the root mean square."""
+    print(f"case: state times 2^-{k} L={L}", flush=True)
+    from sdc_amd import Stepper
+    from sdc_amd.initial import kept_mask
+    m, n = 32, 64
+    r = np.random.default_rng(L)
+    keep = kept_mask(m, n)
+
+    def field(shape):
+        return r.uniform(0.5, 2, shape) * np.exp(2j * np.pi * r.random(shape))
+
+    st = [field((L, n, m // 2 + 1)).astype(np.complex64).astype(complex) * keep for _ in range(3)]
+    st += [r.uniform(0.5, 2, L).astype(np.float32).astype(complex) for _ in range(2)]
+    x, y, z = ((r.random(1000) * s - o).astype(F) for s, o in ((4.0, 0.0), (3.0, 0.0), (0.9, 0.45)))
+    with Stepper(m, n, L, 4.0, 3.0, 1e4, 0.7, 1e-4, precision="f32") as G:
+        G.set_state(*st)
+        one = [a.astype(float) for a in G.velocity_at(x, y, z)]
+        G.set_state(*[a * 2.0 ** -k for a in st])
+        small = [a.astype(float) * 2.0 ** k for a in G.velocity_at(x, y, z)]
+    for a, b in zip(small, one):
+        assert np.abs(a - b).max() <= 2.0 ** -22 * np.sqrt(np.mean(b * b)), np.abs(a - b).max()
