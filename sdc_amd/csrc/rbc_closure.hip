@@ -574,6 +574,17 @@ constexpr int kTP = 36;  // tile row stride: 32 points and a pad that spreads ro
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// an LDS tile that is also read 16 bytes at a time: aligned by its type, wherever LDS places it
+template <int N>
+struct alignas(sizeof(f32x4)) Tile {
+    float v[N];
+    __device__ __forceinline__ float& operator[](int i) { return v[i]; }
+    __device__ __forceinline__ f32x4 four(int i) const {  // i a multiple of 4
+        return *reinterpret_cast<const f32x4*>(v + i);
+    }
+};
+static_assert(alignof(Tile<32>) == 16 && sizeof(Tile<32>) == 128 && kTP % 4 == 0, "16-byte rows");
+
 __device__ __forceinline__ f32x4 mfma16(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -589,11 +600,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
                                                    const float* __restrict__ X, const float* __restrict__ Y,
                                                    float* __restrict__ gpart, double* __restrict__ lpart) {
 #pragma clang fp contract(off)
-    __shared__ float H1[NH * kTP], H2[NH * kTP], D2[NH * kTP], S1[NH * kTP];  // S1 = W2^T D2
+    __shared__ Tile<NH * kTP> H1, H2, D2, S1;  // S1 = W2^T D2
     __shared__ uint32_t wl[(NW + 1) / 2];  // the BF16 weights, for the operand gathers below
     // by point: a group's inputs, two groups in turn; targets; twice the errors; dy for the units < 32
     // and for the others
-    __shared__ float xs[2][NIN * kTP], ts[2][NOUT][32], e2[NOUT][32], dys[2][NOUT][32];
+    __shared__ Tile<NIN * kTP> xs[2];
+    __shared__ Tile<32> e2[NOUT], dys[2][NOUT];
+    __shared__ float ts[2][NOUT][32];
     __shared__ double lsum[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, kq = lane >> 4;  // column of a tile; k of a step, and row group 4 kq + r
@@ -654,13 +667,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
             inv = nm.in_inv[i];
             if (i < NOUT) scale = nm.out_scale[i < NOUT ? i : 0];
         }
-    auto rows = [&](float* tile, const f32x4 (&d)[2]) {  // accumulators -> [unit][point]
+    auto rows = [&](Tile<NH * kTP>& tile, const f32x4 (&d)[2]) {  // accumulators -> [unit][point]
 #pragma unroll
         for (int n = 0; n < 2; ++n)
 #pragma unroll
             for (int r = 0; r < 4; ++r) tile[(row0 + 4 * kq + r) * kTP + 16 * n + c] = d[n][r];
     };
-    auto product = [&](const float (&a)[16], const float* tile, f32x4 (&d)[2]) {  // d += A tile
+    auto product = [&](const float (&a)[16], Tile<NH * kTP>& tile, f32x4 (&d)[2]) {  // d += A tile
 #pragma unroll
         for (int s = 0; s < 16; ++s)
 #pragma unroll
@@ -750,12 +763,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         }
         rows(D2, d);
         // sums over points of the output layer, unit = lane: wave o < 3 has g3[o] and gb3[o], wave 3 gb2
-        auto four = [](const float* q) { return *(const f32x4*)q; };
         if (wave < NOUT) {
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const f32x4 u = four(H2 + lane * kTP + 4 * q), dy = four(&dys[lane >> 5][wave][4 * q]);
-                const f32x4 ee = four(&e2[wave][4 * q]);
+                const f32x4 u = H2.four(lane * kTP + 4 * q), dy = dys[lane >> 5][wave].four(4 * q);
+                const f32x4 ee = e2[wave].four(4 * q);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     g3 = __builtin_fmaf(u[e], dy[e], g3);
@@ -765,11 +777,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         } else {
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
-                const f32x4 u = four(H2 + lane * kTP + 4 * q);
+                const f32x4 u = H2.four(lane * kTP + 4 * q);
                 f32x4 v = {};
 #pragma unroll
                 for (int o = 0; o < NOUT; ++o) {
-                    const f32x4 dy = four(&dys[lane >> 5][o][4 * q]);
+                    const f32x4 dy = dys[lane >> 5][o].four(4 * q);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(w3u[o], dy[e], v[e]);
                 }
@@ -791,8 +803,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
         // sums over points of the input layer, unit = lane: wave w has inputs 2 w and 2 w + 1, wave 0 gb1
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const f32x4 u = four(H1 + lane * kTP + 4 * q), v = four(S1 + lane * kTP + 4 * q);
-            const f32x4 x0 = four(&xs[slot][2 * wave * kTP + 4 * q]), x1 = four(&xs[slot][(2 * wave + 1) * kTP + 4 * q]);
+            const f32x4 u = H1.four(lane * kTP + 4 * q), v = S1.four(lane * kTP + 4 * q);
+            const f32x4 x0 = xs[slot].four(2 * wave * kTP + 4 * q), x1 = xs[slot].four((2 * wave + 1) * kTP + 4 * q);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float f = __builtin_fmaf(-u[e], u[e], 1.f), d1 = f * v[e];
