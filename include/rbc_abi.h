@@ -346,10 +346,11 @@ int rbc_energy_spectrum_ref(rbc_ctx* c, double z, int cap, double* E3, int* nbin
  * history, an AB2 step for the others), then steps_per_launch steps of all members are
  * captured once into one
  * HIP graph and replayed (steps_per_launch = 0: eager launches).  Results equal stepping each
- * member alone.  rbc_ensemble_tune times launch shapes of the generic FFT kernels per size
- * class (M, N, L, precision) on the first member of the class (its state is restored) and
- * applies the fastest to the class; report (optional, 3 doubles per member) receives
- * {y-FFT columns per block, row-kernel threads, ms per step}.
+ * member alone.  rbc_ensemble_tune times the launch shapes of the FFT kernels that take one (FP32
+ * grids of 64..256 points, and the generic LDS kernels) per size class (M, N, L, precision) on the
+ * first member of the class (its state is restored) and applies the fastest to the class; report
+ * (optional, 3 doubles per member) receives {y-FFT columns per block, row-kernel threads, ms per
+ * step}, with 0 columns or threads where the kernels' own choice stays.
  * In the graph, the members of one size class (same M, N, L, nq, precision and tuned shapes)
  * on the FP32 / BF16X3 path of 64..256-point grids with L <= 32 advance together, one launch
  * per stage for the class (same per-member arithmetic as a run of its own); others are graph

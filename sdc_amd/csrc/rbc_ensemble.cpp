@@ -273,26 +273,21 @@ int rbc_ensemble_tune(rbc_ensemble* e, double* report) {
             Snapshot snap;
             take(c, snap);
             const size_t cs = c->csz();
-            const char* gen = getenv("RBC_GENERIC_FFT");
-            const bool forced = gen && gen[0] == '1';
-            // FP32 grids of 64..256 points run the group transforms: their knobs are the kx
-            // columns per y-FFT block (2, 4 or 8 waves) and the threads per row block (2, 4 or
-            // 8 waves); the generic LDS kernels take the column tile and 64..256 threads
-            const bool gy = c->rsz == 4 && !forced && c->dg.N >= 64 && c->dg.N <= 256;
-            const bool gr = c->rsz == 4 && !forced && c->dg.M >= 64 && c->dg.M <= 256;
+            // candidates where a kernel of this grid reads the knob, else the built-in choice (0): the
+            // group transforms take the kx columns per y-FFT block and the threads per row block of 2, 4 or 8
+            // waves, the generic LDS kernels the column tile and 64 to 256 threads
+            const KnobUse use = knob_use(c->dg, c->rsz);
             std::vector<int> txs, ths;
-            if (gy) {
+            if (use.ytx == KNOB_GROUP) {
                 for (int w : {2, 4, 8}) txs.push_back(w * 512 / c->dg.N);
-            } else {
+            } else if (use.ytx == KNOB_GENERIC) {
                 for (int tx = 1; tx <= 16; tx *= 2)
                     if ((size_t)2 * tx * c->dg.N * cs <= 65536) txs.push_back(tx);
-            }
-            if (gr) {
-                for (int w : {2, 4, 8})
-                    if (c->dg.N % (w * 512 / c->dg.M) == 0) ths.push_back(64 * w);
             } else {
-                ths = {64, 128, 256};
+                txs = {0};
             }
+            if (use.rows == KNOB_GROUP) ths = {128, 256, 512};
+            else if (use.rows == KNOB_GENERIC) ths = {64, 128, 256};
             // coordinate search: y-FFT tile first (rows at their default), then the row kernel
             int btx = txs.back(), bth = 0;
             double bms = 1e30;

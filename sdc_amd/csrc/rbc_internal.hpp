@@ -135,10 +135,10 @@ struct Buffers {
     // wC, wS, wS'); FP32 up to L = 32 [level tiles][k-steps][64][4] and 2 x [level pairs][64][4]
     void* evP = nullptr;
     void* prP = nullptr;
-    // launch shapes of the generic (non-512) FFT kernels; 0 = built-in choice.  Set by the
+    // launch shapes of the FFT kernels that take them (knob_use); 0 = built-in choice.  Set by the
     // ensemble autotuner; the arithmetic per element does not depend on them.
     int tune_ytx = 0;           // kx columns per block of the y-FFTs
-    int tune_rows_threads = 0;  // threads per block of the row kernel (64, 128 or 256)
+    int tune_rows_threads = 0;  // threads per block of the row kernel (64 to 512)
 };
 
 // Penalization of a PENALIZED build (nonlinear_operator_rayleigh_noslip.cu:1097-1343): the
@@ -236,6 +236,14 @@ struct Launch {
     static void penalty(const DevGeom& g, const Buffers& b, const Penalty& pen, double Pr, void* const X[3],
                         const void* XF, const void* XG, void* const Nout[3], void* NF, void* NG, hipStream_t s);
 };
+
+// Which kernels read tune_ytx and tune_rows_threads on a grid: none, the group transforms (FP32, 64 to 256
+// points; 2, 4 or 8 waves a block) or the generic LDS kernels.
+enum KnobReader { KNOB_NONE, KNOB_GROUP, KNOB_GENERIC };
+struct KnobUse {
+    KnobReader ytx, rows;
+};
+KnobUse knob_use(const DevGeom& g, int rsz);
 
 // Batched steps of the members of one ensemble size class (rbc_kernels.hip).  A member is
 // described by its geometry, buffers and step constants; batch_create returns nullptr (reason

@@ -2054,6 +2054,23 @@ static int wave_y_log(const DevGeom& g) {
     return g.logN;
 }
 
+// the forward y-FFT fused with the combinations.  Columns of 16 and 32 points: a wave takes 32 or 16 of
+// them, so the fused form, whose blocks go through a group's products in turn, needs enough columns (32 x 32 x 8
+// FP64, 480 columns: 12.0 us against 7.5 us for the generic transform and k_combine)
+template <typename T>
+static bool fused_y_fwd(const DevGeom& g) {
+    return wave_y_log<T>(g) && (g.N >= 64 || g.nq * g.KX >= 4096);
+}
+
+template <typename T>
+static KnobUse knob_use_t(const DevGeom& g) {
+    if (fast512_rows<T>(g)) return {KNOB_NONE, KNOB_NONE};
+    auto tuned = [](int n) { return sizeof(T) == 4 && n >= 64 && n <= 256; };
+    return {fused_y_fwd<T>(g) ? (tuned(g.N) ? KNOB_GROUP : KNOB_NONE) : KNOB_GENERIC,
+            wave_rows_log<T>(g) ? (tuned(g.M) ? KNOB_GROUP : KNOB_NONE) : KNOB_GENERIC};
+}
+KnobUse knob_use(const DevGeom& g, int rsz) { return rsz == 8 ? knob_use_t<double>(g) : knob_use_t<float>(g); }
+
 static inline int fft_tile(int N, size_t csz) {
     // two LDS buffers of TX columns; stay within 64 KiB
     int tx = (int)(65536 / (2 * (size_t)N * csz));
@@ -2223,10 +2240,7 @@ void Launch<T>::fft_y_fwd(const DevGeom& g, const Buffers& b, hipStream_t s) {
                            (const float*)b.ky, (cpx<float>*)b.lev, (cpx<float>*)b.fgw);
         return;
     }
-    // columns of 16 and 32 points: a wave takes 32 or 16 of them, so the fused form, whose blocks go
-    // through a group's products in turn, needs enough columns (32 x 32 x 8 FP64, 480 columns: 12.0
-    // us against 7.5 us for the generic transform and k_combine)
-    if (wave_y_log<T>(g) && (g.N >= 64 || g.nq * g.KX >= 4096)) {
+    if (fused_y_fwd<T>(g)) {
         switch (g.logN) {
             case 4: launch_y_fwd_wc<T, 4>(g, b, s); break;
             case 5: launch_y_fwd_wc<T, 5>(g, b, s); break;
@@ -2507,7 +2521,7 @@ StepBatch* batch_create(const std::vector<BatchMember>& m, std::string& why) {
     const int rows_wpb = b0.tune_rows_threads > 0 ? b0.tune_rows_threads / 64 : 4;
     if (yi_wpb != 2 && yi_wpb != 8) yi_wpb = 4;
     if (yf_wpb != 2 && yf_wpb != 8) yf_wpb = 4;
-    if ((rows_wpb != 2 && rows_wpb != 4 && rows_wpb != 8) || g.N % (rows_wpb * 512 / g.M) != 0) {
+    if (rows_wpb != 2 && rows_wpb != 4 && rows_wpb != 8) {
         why = "row launch shape outside the group kernels";
         return nullptr;
     }
