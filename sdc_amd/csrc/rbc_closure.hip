@@ -1016,6 +1016,11 @@ int y_tile(int N) {
     return std::max(1, std::min(16, tx));
 }
 
+// the row transforms in registers (k_synth_rows_w, k_anal_rows_w); else the LDS kernels
+bool group_rows(const DevGeom& g) {
+    return g.M >= 64 && g.M <= 256 && g.N % (2048 / g.M) == 0 && g.KX == kept_cols(g.M) && !generic_fft_forced();
+}
+
 // the F level-spectrum fields in cl->spec -> point values (os floats per point)
 void synth_points(rbc_closure* cl, int F, int os, int zcol, float* out) {
     rbc_ctx* c = cl->c;
@@ -1026,7 +1031,7 @@ void synth_points(rbc_closure* cl, int F, int os, int zcol, float* out) {
                            (size_t)2 * TX * g.N * sizeof(cpx<float>), c->stream, g, TX, (const cpx<float>*)cl->spec,
                            c->b.rows, (const cpx<float>*)cl->twN, cl->hyb);
     }
-    if (g.M >= 64 && g.M <= 256 && g.N % (2048 / g.M) == 0 && g.KX == kept_cols(g.M)) {
+    if (group_rows(g)) {
         const dim3 gr(g.N / (2048 / g.M), cl->nz);
 #define RBC_SYNTHW(LG)                                                                                    \
     hipLaunchKernelGGL(k_synth_rows_w<LG>, gr, dim3(256), 0, c->stream, g, F, os, zcol, (const float*)cl->zl, \
@@ -1079,7 +1084,7 @@ void apply_closure(rbc_ctx* c, void* user) {
     hipLaunchKernelGGL(k_mlp_infer, dim3(infer_blocks(cl->npts)), dim3(256), 0, c->stream, cl->npts,
                        (const uint16_t*)cl->wbf, cl->nm, (const float*)cl->feat, cl->pred);
     const DevGeom& g = cl->gz;
-    if (g.M >= 64 && g.M <= 256 && g.N % (2048 / g.M) == 0 && g.KX == kept_cols(g.M)) {
+    if (group_rows(g)) {
         const dim3 gr(g.N / (2048 / g.M), cl->nz);
         if (g.M == 64)
             hipLaunchKernelGGL(k_anal_rows_w<6>, gr, dim3(256), 0, c->stream, g, (const float*)cl->pred,

@@ -554,8 +554,8 @@ inline int y_group_waves(const DevGeom& g, int most) {
 
 // Launchers of the group y-FFTs for nf fields of g.nq levels each ([field][l][p] spectra,
 // [field][l][y][kx] hybrid rows); cb = kx columns per block (WPB = cb / (512 / N) waves of 2, 4
-// or 8; 0: built-in choice).  false (nothing launched) unless N is 16 .. 1024
-// (FP64: 512).
+// or 8; 0: built-in choice).  false (nothing launched) unless N is 16 .. 1024 (FP64: 512): at FP64 1024 and
+// FP32 2048 a block within 64 KiB would hold one column, and write its rows in pieces of 8 or 16 bytes.
 template <typename T, int LOGN, int WPB>
 inline void launch_y_group_t(bool inv, const DevGeom& g, int nf, const cpx<T>* in, const cpx<T>* twN,
                              cpx<T>* out, hipStream_t s) {
@@ -584,7 +584,7 @@ inline void launch_y_group_w(bool inv, int cb, const DevGeom& g, int nf, const c
 template <typename T>
 inline bool launch_y_group(bool inv, const DevGeom& g, int nf, const cpx<T>* in, const cpx<T>* twN,
                            cpx<T>* out, hipStream_t s, int cb = 0) {
-    if (g.N < 16 || g.N > (sizeof(T) == 8 ? 512 : 1024) || g.NYc != kept_rows(g.N)) return false;
+    if (generic_fft_forced() || g.N < 16 || g.N > (sizeof(T) == 8 ? 512 : 1024) || g.NYc != kept_rows(g.N)) return false;
     switch (g.logN) {
         case 4: launch_y_group_w<T, 4>(inv, cb, g, nf, in, twN, out, s); break;
         case 5: launch_y_group_w<T, 5>(inv, cb, g, nf, in, twN, out, s); break;

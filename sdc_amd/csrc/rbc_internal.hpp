@@ -237,6 +237,10 @@ struct Launch {
                         const void* XF, const void* XG, void* const Nout[3], void* NF, void* NG, hipStream_t s);
 };
 
+// RBC_GENERIC_FFT=1 in the environment: every transform runs the generic LDS Stockham kernels (the tests pin the
+// 512-point and group-transform kernels against them)
+bool generic_fft_forced();
+
 // Which kernels read tune_ytx and tune_rows_threads on a grid: none, the group transforms (FP32, 64 to 256
 // points; 2, 4 or 8 waves a block) or the generic LDS kernels.
 enum KnobReader { KNOB_NONE, KNOB_GROUP, KNOB_GENERIC };

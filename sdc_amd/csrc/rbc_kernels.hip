@@ -610,7 +610,7 @@ __global__ void __launch_bounds__(256) k_pen_fields(DevGeom g, const T* __restri
     }
 }
 
-// one (row pair y, y + 1, mode k, field) per block, grid sizes outside k_rows_mask_w: the two hybrid
+// one (row pair y, y + 1, mode k, field) per block, for rows that k_rows_mask_w does not take: the two hybrid
 // rows as one complex M-point transform (X1 + i X2, the kx = 0 imaginary parts dropped as a C2R does),
 // the product with chi(x, y) / (M N), the forward transform and the unpacking to kx < KX.  The pair is
 // two rows of one field, so both are of like size.
@@ -1907,7 +1907,7 @@ __global__ void __launch_bounds__(64 * CT) k_fft_y_fwd512c2(DevGeom g, int ntile
 // Forward y-FFT at N = 16 .. 1024 fused with the level combinations: blockIdx.z = the
 // combination group of YGroup (0: h, d, uv -> D0, D2; 1: uw, vw -> D1, D3 and the k = 0 values
 // of P_uw, P_vw; 2: u.grad(theta) -> D4).  A block of WPB waves handles CB kx columns of one
-// level, one group of W = N / 8 lanes per column (fft_group, natural layout); the group's
+// level, one group of W lanes per column (YShape; fft_group, natural layout); the group's
 // products are transformed in turn through the LDS tile and their combinations accumulate in
 // registers.  Writes D[t][l][p] into the level buffer (free once the inverse y-FFT has read it).
 template <typename T, int LOGN, int WPB, int GRP>
@@ -2014,8 +2014,6 @@ __global__ void __launch_bounds__(64 * WPB) k_fft_y_fwd_wc_batch(const k_fft_y_f
 // ---------------------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------------------
-// RBC_GENERIC_FFT=1 in the environment selects the generic LDS Stockham kernels everywhere (used
-// by the tests to pin the 512-point and group-transform kernels against them).
 // Blocks of `kernel` (blocks of `threads`, static LDS only) that one XCD of the current device
 // holds at once: resident blocks per CU x CUs / 8.
 static int resident_blocks_per_xcd(const void* kernel, int threads) {
@@ -2027,7 +2025,7 @@ static int resident_blocks_per_xcd(const void* kernel, int threads) {
     return std::max(1, per_cu * ncu / 8);
 }
 
-static bool generic_fft_forced() {
+bool generic_fft_forced() {
     const char* e = getenv("RBC_GENERIC_FFT");
     return e && e[0] == '1';
 }
@@ -2390,8 +2388,8 @@ void Launch<T>::penalty(const DevGeom& g, const Buffers& b, const Penalty& pen, 
     if (!launch_y_inv_group<T>(gp, kPenFields, (const cpx<T>*)pen.spec, (const cpx<T>*)b.twN, (cpx<T>*)pen.hin, s))
         hipLaunchKernelGGL(k_fft_y_inv<T>, gy, dim3(256), sm, s, gp, TX, (const cpx<T>*)pen.spec, b.rows,
                            (const cpx<T>*)b.twN, (cpx<T>*)pen.hin);
-    const bool kept = g.KX == kept_cols(g.M);
-    switch (kept ? g.logM : 0) {
+    const bool group = g.KX == kept_cols(g.M) && !generic_fft_forced();
+    switch (group ? g.logM : 0) {
         case 4: launch_rows_mask<T, 4>(g, pen, b.twM, s); break;
         case 5: launch_rows_mask<T, 5>(g, pen, b.twM, s); break;
         case 6: launch_rows_mask<T, 6>(g, pen, b.twM, s); break;

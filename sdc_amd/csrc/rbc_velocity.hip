@@ -183,7 +183,7 @@ __device__ __forceinline__ void put_velocity(float* __restrict__ grid, size_t cs
     }
 }
 
-// Block per (y, l), row lengths outside k_vel_rows_w: u + i v and w go through two complex inverse
+// Block per (y, l), for rows that k_vel_rows_w does not take: u + i v and w go through two complex inverse
 // FFTs of length M.
 template <bool PLANAR>
 __global__ void __launch_bounds__(256) k_vel_rows(DevGeom g, const cpx<float>* __restrict__ hyb,
@@ -1143,7 +1143,7 @@ void launch_vel_rows_w(rbc_ctx* c, const DevGeom& gt, const GridWork& w) {
 // in registers at 16 to 1024 points, through LDS else
 template <bool PLANAR>
 void launch_vel_rows(rbc_ctx* c, const DevGeom& gt, const GridWork& w) {
-    switch (gt.KX == kept_cols(gt.M) ? gt.logM : 0) {
+    switch (gt.KX == kept_cols(gt.M) && !generic_fft_forced() ? gt.logM : 0) {
         case 4: return launch_vel_rows_w<4, PLANAR>(c, gt, w);
         case 5: return launch_vel_rows_w<5, PLANAR>(c, gt, w);
         case 6: return launch_vel_rows_w<6, PLANAR>(c, gt, w);
