@@ -503,7 +503,7 @@ def run_tracers(a):
                        "algorithmic_flops_per_step": fl, "kept_modes": P,
                        "note": "FP32 flops of the vertical sums (as six products of BF16 parts) over the whole tracer step time (both "
                                "evaluations, the slice sums and the position updates) against the FP32 matrix peak; the "
-                               "phases and the velocity combination on the VALU bound it"}
+                               "VALU (phases, velocity combination, splitting) bounds it"}
     S.close()
     print(json.dumps(out))
 

@@ -544,8 +544,8 @@ __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as
 // us a spectral RK2 step (two evaluations), 100,000 particles at 128^2, all FP32 instructions -> now, same box: L = 4 / 8 / 10 / 16 /
 // 24 / 32 972 / 995 / 1569 / 1602 / 2658 / 3375 -> 921 / 941 / 1166 / 1249 / 1837 / 2030; BF16X3, L = 8 / 16 1185 / 1412 -> 705 / 846.
 // With FP32 instructions the six sums are 61 % of the kernel at L = 16 and the VALU the other 40 %, without
-// overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU (about 90 instructions a sub-tile for the
-// phases and the combination) and the 24 or 36 products (NS = 1: 6 or 12 of twice the cycles) about alike.  Two blocks per CU
+// overlap; BF16 products run at 16 times the FP32 rate.  Bound by the VALU, 0.69 of its issue slots at L = 16 (162
+// instructions a sub-tile, about 90 of them for the phases and the combination), beside the matrix cores' 0.42.  Two blocks per CU
 // (128 registers, one set of accumulators), so that one computes while the other stages: with one 1475 against 1207 us at L = 16.
 template <int LMAX, int NS>
 __global__ void __launch_bounds__(kVelMmaThreads, 4) k_vel_points_mma(

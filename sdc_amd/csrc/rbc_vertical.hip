@@ -53,11 +53,11 @@ struct alignas(2 * sizeof(T)) pair2 {
     T c[2];
 };
 
-// two consecutive complex values; PAIRED: one wide load (the address is a multiple of both)
+// two consecutive complex values; PAIRED: wide loads (the address is a multiple of 16 bytes)
 template <typename T, bool PAIRED>
 __device__ __forceinline__ void load_two(const cpx<T>* p, cpx<T>& a, cpx<T>& b, bool second) {
     if constexpr (PAIRED) {
-        struct alignas(sizeof(T) == 4 ? 16 : 16) two {
+        struct alignas(16) two {
             cpx<T> v[2];
         };
         const two t = *reinterpret_cast<const two*>(p);
@@ -816,8 +816,15 @@ ProjectArgs<T> project_args(const DevGeom& g, const Buffers& b, double Pr, void*
 template <typename T>
 void launch_eval(const EvalArgs<T>& a, const EvalArgs<T>* batch, int B, hipStream_t s) {
     const dim3 grid(8 * a.per + 1, 1, B);
-#define RBC_EVP(NSV, PV)                                                                                      if (batch) hipLaunchKernelGGL((k_eval_parity_batch<T, NSV, PV>), grid, dim3(256), 0, s, batch);           else hipLaunchKernelGGL((k_eval_parity<T, NSV, PV>), grid, dim3(256), 0, s, a)
-#define RBC_EVP2(NSV)             if (a.g.L % 2 == 0) {             RBC_EVP(NSV, true);       } else {                          RBC_EVP(NSV, false);      }
+#define RBC_EVP(NSV, PV)                                                                                  \
+    if (batch) hipLaunchKernelGGL((k_eval_parity_batch<T, NSV, PV>), grid, dim3(256), 0, s, batch);       \
+    else hipLaunchKernelGGL((k_eval_parity<T, NSV, PV>), grid, dim3(256), 0, s, a)
+#define RBC_EVP2(NSV)          \
+    if (a.g.L % 2 == 0) {      \
+        RBC_EVP(NSV, true);    \
+    } else {                   \
+        RBC_EVP(NSV, false);   \
+    }
     if constexpr (sizeof(T) == 4) {
         if (vertical_plain(a.g.L, a.g.nq, a.g.PS, false)) {
 #define RBC_EVPL(NSV)                                                                                     \
